@@ -1,0 +1,47 @@
+"""GPU checks of the FP64 product behind every dense step, through the Gauss
+map's lmap (C = alpha op(map) op(B) + beta C), against numpy: the small kernel
+(32 x 32 tiles, K dealt to eight waves) and the wide one (waves along M or N),
+tile and slice remainders in every dimension, K split over blocks, odd leading
+dimensions and every transposition."""
+import numpy as np
+import pytest
+
+from tests.gpu_helpers import dev, host
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+# One rounding per product and sum: the error of an inner product of length K
+# is below K eps times the product of the norms, 5000 * 2.2e-16 = 1.1e-12 here
+# at most, and its root-mean-square over a matrix about sqrt(K) eps, 2e-14.
+TOL = 1e-12
+
+
+@pytest.fixture(scope="module")
+def S():
+    import skema_amd
+
+    skema_amd.load()
+    return skema_amd
+
+
+@pytest.mark.parametrize("tA", ["N", "T"])
+@pytest.mark.parametrize("tB", ["N", "T"])
+@pytest.mark.parametrize("M,N,K", [(1, 1, 1), (33, 31, 7), (64, 98, 300), (17, 3000, 129), (401, 4111, 1000),
+                                   (4111, 401, 1003), (97, 8300, 640), (8300, 97, 33), (2300, 1204, 15),
+                                   (803, 803, 5000), (20, 40, 5000), (6000, 2500, 16), (270, 12000, 500)])
+def test_products_of_every_shape(S, tA, tB, M, N, K):
+    print(f"case gemm {M}x{N}x{K} {tA}{tB}", flush=True)
+    rng = np.random.default_rng(M + N + K)
+    D = rng.standard_normal((M, K) if tA == "N" else (K, M))
+    B = rng.standard_normal((K, N) if tB == "N" else (N, K))
+    C = rng.standard_normal((M, N))
+    mp = S.GaussDimRedux(*D.shape, data=D)
+    ref = (D if tA == "N" else D.T) @ (B if tB == "N" else B.T)
+    for beta in (0.0, -0.5):
+        # beta = 0 never reads C: NaN there must not come through
+        out = dev(C if beta else np.full((M, N), np.nan))
+        mp.lmap(1.5, dev(B), beta, tA, tB, C_out=out)
+        want = 1.5 * ref + (beta * C if beta else 0.0)
+        err = np.linalg.norm(host(out) - want) / np.linalg.norm(want)
+        assert err <= TOL, (beta, err)
