@@ -244,141 +244,198 @@ __global__ __launch_bounds__(256) void k_jacobi_round(double* A, int64_t lda, do
   if (tid == 0) atomicAdd(rotations, 1);
 }
 
-// Block-pair Jacobi round in registers.  The columns come in blocks of
-// kJacobiBlock = 8; a round's block pairs are disjoint and each takes one
-// 512-thread workgroup in which thread i holds row i of the pair's 16
-// columns of A and of V (orders up to 512), so a rotation is local to every
-// thread and only the inner products need a reduction.  A local round
-// rotates 8 disjoint column pairs at fixed register positions: one
-// block-wide reduction of their 24 inner products (fixed order), then each
-// thread applies the 8 rotations to its row.  Between local rounds the
-// columns move instead of the pair indices (so no register is indexed at run
-// time):
+// Block-pair Jacobi round.  The columns come in blocks of kJacobiBlock = 8; a
+// round's block pairs are disjoint and each takes one 8-wave workgroup (orders
+// up to 512: 64 rows a wave).  The pair's 16 columns are read once, their Gram
+// matrix G (16 x 16) is formed on the matrix cores, one wave runs the pair's
+// local rounds on G alone and collects the rotations in J (16 x 16, kept as
+// J - I), and the columns are multiplied by J on the matrix cores.  A local round rotates 8
+// disjoint column pairs: G <- J_r^T G J_r, lane (k, g) owning the 2 x 2 block of
+// column pair k and row pair g, so nothing but wave-ordered LDS accesses lies
+// between rounds.  G is formed anew by every launch, and a rotated entry G(q, r)
+// keeps an error of eps |q| |r|, like an inner product taken afresh.
 //   intra (the first round of each sweep, every block once): pairs
 //     (p, 7 - p) within each block, then positions 1..7 of each block
 //     rotate by one (the circle method; 7 rounds, back in place after);
-//   cross: pairs (p, 8 + p), then the second block shifts by one position
-//     (8 rounds, back in place after).
-// Padding columns (>= n) are zero and never rotate.
+//   cross: pairs (p, 8 + (p + r) % 8) in round r (8 rounds).
+// A pair with nothing above the tolerance leaves after G.  V's columns do not
+// enter the rotations, so they are multiplied by J one launch later, by further
+// blocks beside the next round's.  Padding columns (>= n) are zero and never
+// rotate.  Bound by the latency of one pair's chain, not by work (26 pairs at
+// order 401): holding the columns in registers and reducing 24 inner products
+// over 512 threads each local round took 28.5 us a launch at order 401, this 10.4, and
+// the relative error of the singular values went from 1.1e-13 to 2e-15.
 constexpr int kJacobiBlock = 8;
 
 // Rotation of columns x, y from their inner products (the k_jacobi_round
-// formula); false when they are already orthogonal to tol.
-__device__ inline bool jacobi_cs(double alpha, double beta, double gamma, double tol, double& c, double& s) {
-  if (!(fabs(gamma) > tol * sqrt(alpha * beta))) return false;
+// angle, without a branch), applied as x - s (y + tau x), y + s (x - tau y) with
+// tau = s / (1 + c): a rounded c near 1 would lengthen both columns by s^2 each
+// time.  s = 0 when they are already orthogonal to tol.
+__device__ __forceinline__ void jacobi_st(double alpha, double beta, double gamma, double tol, double& s, double& tau) {
+  const bool rot = fabs(gamma) > tol * sqrt(alpha * beta);
   const double zeta = (beta - alpha) / (2.0 * gamma);
   const double az = fabs(zeta);
-  const double t = (az > 1e150) ? 0.5 / zeta : copysign(1.0, zeta) / (az + sqrt(1.0 + zeta * zeta));
-  c = 1.0 / sqrt(1.0 + t * t);
-  s = c * t;
-  return true;
+  const double near = copysign(1.0, zeta) / (az + sqrt(1.0 + zeta * zeta));
+  const double t = az > 1e150 ? 0.5 / zeta : near;
+  const double c = 1.0 / sqrt(1.0 + t * t);
+  s = rot ? c * t : 0.0;
+  tau = c * t / (1.0 + c);
 }
 
-__global__ __launch_bounds__(512) void k_jacobi_rows(double* A, int64_t lda, double* V, int64_t ldv, int64_t n,
-                                                     const int2* bpairs, int intra, double tol, int* rotations) {
-  constexpr int NB = kJacobiBlock, NC = 2 * NB;
-  __shared__ double red[8][24];
-  __shared__ double par[24];
-  __shared__ double cs[8][2];
-  __shared__ int rotp[8];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int2 bp = bpairs[blockIdx.x];
-  const int64_t i = tid;
-  double a[NC], v[NC];
+// Column held at position p of an 8-column block in intra round r.
+__device__ inline int jacobi_intra_col(int p, int r) { return p == 0 ? 0 : 1 + (p + 6 - r) % 7; }
+
+struct JacobiArgs {
+  double *A, *V;
+  int64_t lda, ldv, n;
+  const int2* pairs;   // this round's block pairs (na)
+  const int2* vpairs;  // the previous round's, whose J waits for V (nv)
+  int na, nv, intra;
+  double tol;
+  double* J;  // J - I of each pair, and whether it rotated, of this round
+  int* rot;
+  const double* Jv;  // of the previous one
+  const int* rotv;
+  int* rotations;
+};
+
+// This wave's 64 rows x 16 columns of a block pair, M(row 16 t + l16, column
+// 4 s + lq) in x[t][s]; rows and columns past n are zero.
+__device__ __forceinline__ void jacobi_load(const double* M, int64_t ld, int64_t n, int2 bp, int64_t r0, int l16, int lq,
+                                            double (&x)[4][4]) {
 #pragma unroll
-  for (int t = 0; t < NC; ++t) {
-    const int64_t c = (int64_t)(t < NB ? bp.x : bp.y) * NB + (t % NB);
-    const bool ok = i < n && c < n;
-    a[t] = ok ? A[i + c * lda] : 0.0;
-    v[t] = ok ? V[i + c * ldv] : 0.0;
-  }
-  int count = 0;
-  // one local round on the pairs (pos_a(k), pos_b(k)), k < 8 (register
-  // positions known at compile time)
-  auto round = [&](auto pos_a, auto pos_b) {
-    double w[32];
+  for (int t = 0; t < 4; ++t)
 #pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      const double x = a[pos_a(k)], y = a[pos_b(k)];
-      w[3 * k] = x * x;
-      w[3 * k + 1] = y * y;
-      w[3 * k + 2] = x * y;
+    for (int s = 0; s < 4; ++s) {
+      const int64_t row = r0 + 16 * t + l16;
+      const int64_t col = (int64_t)(s < 2 ? bp.x : bp.y) * kJacobiBlock + 4 * (s & 1) + lq;
+      const bool ok = row < n && col < n;
+      const double v = M[(row < n ? row : n - 1) + (col < n ? col : n - 1) * ld];
+      x[t][s] = ok ? v : 0.0;
     }
+}
+// M <- x + x (J - I), the same rows and columns; jf holds J - I, and the sum is
+// rounded once.
+__device__ __forceinline__ void jacobi_apply(double* M, int64_t ld, int64_t n, int2 bp, int64_t r0, int l16, int lq,
+                                             const double (&x)[4][4], const double (&jf)[4]) {
 #pragma unroll
-    for (int k = 24; k < 32; ++k) w[k] = 0.0;
-    const double tot = wave_sum32(w);
-    if ((lane & 1) == 0 && (lane >> 1) < 24) red[wave][lane >> 1] = tot;
-    __syncthreads();
-    if (tid < 24) {
-      double t = 0.0;
-      for (int q = 0; q < 8; ++q) t += red[q][tid];
-      par[tid] = t;
-    }
-    __syncthreads();
-    if (tid < 8) {  // the 8 rotations, once each (FP64 divisions and square roots)
-      double c = 1.0, s = 0.0;
-      const bool rot = jacobi_cs(par[3 * tid], par[3 * tid + 1], par[3 * tid + 2], tol, c, s);
-      cs[tid][0] = c;
-      cs[tid][1] = rot ? s : 0.0;
-      rotp[tid] = rot ? 1 : 0;
-    }
-    __syncthreads();
+  for (int t = 0; t < 4; ++t) {
+    d4 acc = d4{0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      if (rotp[k]) {
-        const double c = cs[k][0], s = cs[k][1];
-        const int pa = pos_a(k), pb = pos_b(k);
-        const double x = a[pa], y = a[pb];
-        a[pa] = c * x - s * y;
-        a[pb] = s * x + c * y;
-        const double vx = v[pa], vy = v[pb];
-        v[pa] = c * vx - s * vy;
-        v[pb] = s * vx + c * vy;
-        ++count;
-      }
-    }
-    __syncthreads();  // par, red and cs are rewritten by the next round
-  };
-  if (intra) {
-    for (int r = 0; r < NB - 1; ++r) {
-      // pairs (p, 7 - p) in block X (k < 4) and block Y (k >= 4)
-      round([](int k) { return k < 4 ? k : NB + (k - 4); }, [](int k) { return k < 4 ? NB - 1 - k : NC - 1 - (k - 4); });
-      // circle method: positions 1 .. 7 of each block rotate by one
+    for (int s = 0; s < 4; ++s) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(jf[s], x[t][s], acc, 0, 0, 0);
+    const int64_t row = r0 + 16 * t + l16;
 #pragma unroll
-      for (int b = 0; b < 2; ++b) {
-        const int o = NB * b;
-        const double ta = a[o + NB - 1], tv = v[o + NB - 1];
-#pragma unroll
-        for (int p = NB - 1; p > 1; --p) {
-          a[o + p] = a[o + p - 1];
-          v[o + p] = v[o + p - 1];
-        }
-        a[o + 1] = ta;
-        v[o + 1] = tv;
-      }
+    for (int v = 0; v < 4; ++v) {
+      const int64_t col = (int64_t)(v < 2 ? bp.x : bp.y) * kJacobiBlock + 4 * (v & 1) + lq;
+      if (row < n && col < n) M[row + col * ld] = x[t][v] + acc[v];
     }
   }
-  for (int r = 0; r < NB; ++r) {
-    round([](int k) { return k; }, [](int k) { return NB + k; });
-    // the second block shifts by one position
-    const double ta = a[NB], tv = v[NB];
+}
+
+__global__ __launch_bounds__(512) void k_jacobi_pairs(JacobiArgs g) {
+  constexpr int P = 66;                 // pitch of a wave's columns in LDS
+  __shared__ double cols[8][16 * P];    // this wave's 64 rows, column-major
+  __shared__ double part[8][16][17];    // Gram of each wave's rows
+  __shared__ double G[16][17], J[16][17];
+  __shared__ int any;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l16 = lane & 15, lq = lane >> 4;
+  const int64_t r0 = 64 * (int64_t)wave;
+  const bool live = r0 < g.n;
+  double x[4][4], jf[4];
+  if ((int)blockIdx.x >= g.na) {  // V of a pair of the previous round
+    const int b = blockIdx.x - g.na;
+    if (!live || !g.rotv[b]) return;
+    const int2 bp = g.vpairs[b];
+    jacobi_load(g.V, g.ldv, g.n, bp, r0, l16, lq, x);
 #pragma unroll
-    for (int p = NB; p < NC - 1; ++p) {
-      a[p] = a[p + 1];
-      v[p] = v[p + 1];
+    for (int s = 0; s < 4; ++s) jf[s] = g.Jv[(int64_t)b * 256 + (4 * s + lq) * 16 + l16];
+    jacobi_apply(g.V, g.ldv, g.n, bp, r0, l16, lq, x, jf);
+    return;
+  }
+  const int2 bp = g.pairs[blockIdx.x];
+  d4 acc = d4{0.0, 0.0, 0.0, 0.0};
+  if (live) {
+    jacobi_load(g.A, g.lda, g.n, bp, r0, l16, lq, x);
+    double* c = cols[wave];
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int s = 0; s < 4; ++s) c[(4 * s + lq) * P + 16 * t + l16] = x[t][s];
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int s = 0; s < 16; ++s) {
+      const double v = c[l16 * P + 4 * s + lq];
+      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(v, v, acc, 0, 0, 0);
     }
-    a[NC - 1] = ta;
-    v[NC - 1] = tv;
   }
 #pragma unroll
-  for (int t = 0; t < NC; ++t) {
-    const int64_t c = (int64_t)(t < NB ? bp.x : bp.y) * NB + (t % NB);
-    if (i < n && c < n) {
-      A[i + c * lda] = a[t];
-      V[i + c * ldv] = v[t];
+  for (int v = 0; v < 4; ++v) part[wave][lq + 4 * v][l16] = acc[v];
+  __syncthreads();
+  if (tid < 256) {
+    const int i = tid >> 4, j = tid & 15;
+    double t = 0.0;
+#pragma unroll
+    for (int w = 0; w < 8; ++w) t += part[w][i][j];
+    G[i][j] = t;
+    J[i][j] = 0.0;
+  }
+  __syncthreads();
+  if (wave == 0) {
+    const int k = lane & 7, r = lane >> 3;  // column pair, row pair
+    auto over = [&](int p, int q) { return fabs(G[p][q]) > g.tol * sqrt(G[p][p] * G[q][q]); };
+    bool o = over(k, 8 + r);
+    if (g.intra && k != r) o = o || over(k < r ? k : r, k < r ? r : k) || over(8 + (k < r ? k : r), 8 + (k < r ? r : k));
+    const bool some = __any(o);
+    if (lane == 0) any = some;
+    if (some) {
+      // one local round on the column pairs (ca(j), cb(j)), j < 8
+      auto round = [&](auto ca, auto cb) {
+        const int pk = ca(k), qk = cb(k), pr = ca(r), qr = cb(r);
+        const double b00 = G[pr][pk], b01 = G[pr][qk], b10 = G[qr][pk], b11 = G[qr][qk];
+        const double u0 = J[r][pk], u1 = J[r][qk], w0 = J[8 + r][pk], w1 = J[8 + r][qk];
+        double sk, tk;
+        jacobi_st(G[pk][pk], G[qk][qk], G[pk][qk], g.tol, sk, tk);
+        const double sr = __shfl(sk, r), tr = __shfl(tk, r);  // lane r holds pair r
+        const bool rk = sk != 0.0, rr = sr != 0.0;
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_wave_barrier();
+        // columns, then rows; a pair that does not rotate is left as it is
+        const double e00 = rk ? b00 - sk * (b01 + tk * b00) : b00, e01 = rk ? b01 + sk * (b00 - tk * b01) : b01;
+        const double e10 = rk ? b10 - sk * (b11 + tk * b10) : b10, e11 = rk ? b11 + sk * (b10 - tk * b11) : b11;
+        G[pr][pk] = rr ? e00 - sr * (e10 + tr * e00) : e00;
+        G[pr][qk] = rr ? e01 - sr * (e11 + tr * e01) : e01;
+        G[qr][pk] = rr ? e10 + sr * (e00 - tr * e10) : e10;
+        G[qr][qk] = rr ? e11 + sr * (e01 - tr * e11) : e11;
+        // J - I: its own entries, with the identity's added where they are used
+        const double ip = pk == r ? 1.0 : 0.0, iq = qk == r ? 1.0 : 0.0;
+        const double jp = pk == 8 + r ? 1.0 : 0.0, jq = qk == 8 + r ? 1.0 : 0.0;
+        J[r][pk] = rk ? u0 - sk * ((u1 + iq) + tk * (u0 + ip)) : u0;
+        J[r][qk] = rk ? u1 + sk * ((u0 + ip) - tk * (u1 + iq)) : u1;
+        J[8 + r][pk] = rk ? w0 - sk * ((w1 + jq) + tk * (w0 + jp)) : w0;
+        J[8 + r][qk] = rk ? w1 + sk * ((w0 + jp) - tk * (w1 + jq)) : w1;
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_wave_barrier();
+      };
+      if (g.intra)
+        for (int q = 0; q < kJacobiBlock - 1; ++q)
+          round([&](int j) { return j < 4 ? jacobi_intra_col(j, q) : 8 + jacobi_intra_col(j - 4, q); },
+                [&](int j) { return j < 4 ? jacobi_intra_col(7 - j, q) : 8 + jacobi_intra_col(11 - j, q); });
+      for (int q = 0; q < kJacobiBlock; ++q)
+        round([&](int j) { return j; }, [&](int j) { return 8 + ((j + q) & 7); });
+      if (lane == 0) atomicAdd(g.rotations, 1);
     }
   }
-  if (tid == 0 && count) atomicAdd(rotations, count);
+  __syncthreads();
+  if (tid == 0) g.rot[blockIdx.x] = any;
+  if (!any) return;
+  if (tid < 256) g.J[(int64_t)blockIdx.x * 256 + tid] = J[tid >> 4][tid & 15];
+  if (live) {
+#pragma unroll
+    for (int s = 0; s < 4; ++s) jf[s] = J[4 * s + lq][l16];
+    jacobi_apply(g.A, g.lda, g.n, bp, r0, l16, lq, x, jf);
+  }
 }
 
 __global__ __launch_bounds__(256) void k_col_norms(const double* A, int64_t lda, int64_t n, double* S) {
@@ -843,8 +900,8 @@ int jacobi_svd(hipStream_t st, int64_t n, double* A, int64_t lda, double* U, int
                int64_t ldv, DevBuf* scratch) {
   if (n == 0) return 0;
   SKEMA_REQUIRE(n < (1 << 20), kErrUnsupported, "jacobi_svd: order too large");
-  // Block-pair rounds in registers for orders up to 512 (one launch per
-  // round of block pairs, ~n/16 per sweep), else scalar rounds (~n).
+  // Block-pair rounds for orders up to 512 (one launch per round of block
+  // pairs, ~n/8 per sweep), else scalar rounds (~n).
   const bool blocked = n > kJacobiBlock && n <= 512;
   const int64_t units = blocked ? cdiv(n, kJacobiBlock) : n;
   // Round-robin (circle method) schedule over the units: units' - 1 rounds
@@ -869,7 +926,11 @@ int jacobi_svd(hipStream_t st, int64_t n, double* A, int64_t lda, double* U, int
   const size_t off_pairs = 0;
   const size_t off_vw = align_up(pairs.size() * sizeof(int2), 256);
   const size_t off_cnt = off_vw + align_up((size_t)n * n * sizeof(double), 256);
-  const size_t off_sraw = off_cnt + 256;
+  // two rounds' J and flags per block pair
+  const size_t per_round = (size_t)(np / 2);
+  const size_t off_j = off_cnt + 256;
+  const size_t off_rot = off_j + (blocked ? 2 * per_round * 256 * sizeof(double) : 0);
+  const size_t off_sraw = off_rot + (blocked ? align_up(2 * per_round * sizeof(int), 256) : 0);
   const size_t off_perm = off_sraw + align_up((size_t)n * sizeof(double), 256);
   const size_t total = off_perm + align_up((size_t)n * sizeof(int), 256);
   scratch->reserve(total);
@@ -888,19 +949,32 @@ int jacobi_svd(hipStream_t st, int64_t n, double* A, int64_t lda, double* U, int
   constexpr int kMaxSweeps = 100;
   int sweeps = 0;
   bool converged = false;
+  int slot = 0, vround_start = 0, vcnt = 0;
+  // (the last sweep rotates nothing, so no J is left waiting for V)
   for (; sweeps < kMaxSweeps; ++sweeps) {
     fill_i32(st, d_cnt, 1, 0);
     for (int r = 0; r + 1 < (int)round_start.size(); ++r) {
       const int cnt = round_start[r + 1] - round_start[r];
       if (cnt == 0) continue;
-      if (blocked)
-        hipLaunchKernelGGL(k_jacobi_rows, dim3(cnt), dim3(512), 0, st, A, lda, Vw, n, n, d_pairs + round_start[r],
-                           r == 0 ? 1 : 0, tol, d_cnt);
-      else
+      if (blocked) {
+        JacobiArgs ja;
+        ja.A = A; ja.lda = lda; ja.V = Vw; ja.ldv = n; ja.n = n;
+        ja.pairs = d_pairs + round_start[r]; ja.na = cnt;
+        ja.vpairs = d_pairs + vround_start; ja.nv = vcnt;  // J of the round before, if any
+        ja.intra = r == 0 ? 1 : 0; ja.tol = tol; ja.rotations = d_cnt;
+        double* dj = reinterpret_cast<double*>(base + off_j);
+        int* drot = reinterpret_cast<int*>(base + off_rot);
+        ja.J = dj + (size_t)slot * per_round * 256; ja.rot = drot + slot * per_round;
+        ja.Jv = dj + (size_t)(1 - slot) * per_round * 256; ja.rotv = drot + (1 - slot) * per_round;
+        hipLaunchKernelGGL(k_jacobi_pairs, dim3(cnt + vcnt), dim3(512), 0, st, ja);
+        vround_start = round_start[r];
+        vcnt = cnt;
+        slot = 1 - slot;
+      } else
         hipLaunchKernelGGL(k_jacobi_round, dim3(cnt), dim3(256), 0, st, A, lda, Vw, n, n, d_pairs + round_start[r],
                            tol, d_cnt);
     }
-    check_launch(blocked ? "k_jacobi_rows" : "k_jacobi_round");
+    check_launch(blocked ? "k_jacobi_pairs" : "k_jacobi_round");
     int h_cnt = 0;
     SKEMA_HIP(hipMemcpyAsync(&h_cnt, d_cnt, sizeof(int), hipMemcpyDeviceToHost, st));
     SKEMA_HIP(hipStreamSynchronize(st));

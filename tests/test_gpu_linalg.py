@@ -1,0 +1,53 @@
+"""GPU checks of the factorisations inside low_rank_approx at the sizes where
+their kernels change path, against the oracle's LAPACK."""
+import numpy as np
+import pytest
+
+from oracle import skema_oracle as O
+from tests.gpu_helpers import dev, gpu_maps, to_gpu_params
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def S():
+    import skema_amd
+
+    skema_amd.load()
+    return skema_amd
+
+
+# The core solve multiplies rounding errors (eps ~ 1e-16) by the condition of
+# two Gaussian (2k+1) x k factors (about 6 each) and the vectors by the inverse
+# of the relative gap, about 1 / 0.035 at the sixth of a 0.7^i spectrum: 1e-12
+# with some room for the orders (sqrt(k)) is 1e-10.
+TOL = 1e-10
+
+
+@pytest.mark.parametrize("m,n,k", [(60, 50, 9), (60, 50, 16), (90, 61, 17), (300, 150, 64), (300, 150, 65),
+                                   (1500, 600, 130), (1300, 1100, 512), (1300, 1100, 515)])
+def test_low_rank_approx_orders(S, m, n, k):
+    """Core orders around the 8-column blocks and 64-row waves of the blocked
+    Jacobi rounds (9 to 512) and beyond them (515: scalar rounds)."""
+    print(f"case low_rank_approx {m}x{n} k={k}", flush=True)
+    rng = np.random.default_rng(k)
+    A = (rng.standard_normal((m, n)) / np.sqrt(m)) @ np.diag(0.7 ** np.arange(n)) @ rng.standard_normal((n, n))
+    A += 1e-4 * rng.standard_normal((m, n))
+    p = O.AlgParams(matrix_m=m, matrix_n=n, rank=6, sketch_range=k, sketch_core=2 * k + 1, window=m)
+    osk = O.SketchySVD(p)
+    osk.linear_update(A)
+    Ur, Sr, Vr = osk.low_rank_approx()
+    g = S.SketchySVD(to_gpu_params(p), maps=gpu_maps({"Upsilon": osk.Upsilon, "Omega": osk.Omega, "Phi": osk.Phi,
+                                                      "Psi": osk.Psi}))
+    g.linear_update(dev(A))
+    U, Sv, V = g.low_rank_approx()
+    assert np.abs(Sv - Sr).max() <= TOL * Sr[0]
+    Ua, Va = O.align_signs(U, V, Ur, Vr)
+    assert O.rel_err(Ua, Ur) <= TOL and O.rel_err(Va, Vr) <= TOL
+    # every factor of the core's SVD, not the leading six only
+    Q, P = g.checkpoint("Q"), g.checkpoint("P")
+    sv = g.checkpoint("S")[:, 0]
+    assert np.abs(sv - np.linalg.svd(g.checkpoint("C"), compute_uv=False)).max() <= 1e-13 * sv[0] * np.sqrt(k)
+    for M in (Q, P):
+        assert np.abs(M.T @ M - np.eye(k)).max() <= 1e-12
