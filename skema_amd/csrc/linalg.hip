@@ -1,6 +1,7 @@
-// FP64 finalize kernels: Householder QR (dgeqr2/dorg2r structure, which is
-// what the reference's dgeqrf/dorgqr calls with lwork = n execute,
-// src/Skema_BlasLapack.hpp:168-217), upper-triangular solve (dgels on an
+// FP64 finalize kernels: Householder QR column by column within its panels
+// (what the reference's dgeqrf/dorgqr calls with lwork = n execute,
+// src/Skema_BlasLapack.hpp:168-217) for the matrices that qr_panel.hip gives up
+// on, upper-triangular solve (dgels on an
 // already-triangular matrix, :219-243) and a one-sided Jacobi SVD standing in
 // for dgesvd (:71-97).
 #include <algorithm>
@@ -13,8 +14,6 @@
 
 namespace skema {
 namespace {
-
-constexpr int kQrThreads = 512;
 
 __device__ __forceinline__ double wave_sum(double v) {
 #pragma unroll
@@ -65,87 +64,6 @@ __device__ inline double wave_sum16(double (&v)[16]) {
   halve<1, 4>(v, lane & 4);
   const double t = v[0] + __shfl_xor(v[0], 2);
   return t + __shfl_xor(t, 1);
-}
-
-// dlarfg on column `col` of length len (col[0] = alpha, col[1..] = x).
-// The thread->element assignment (i = tid + k*bs) is the one every caller
-// uses for its own writes, so no cross-thread global visibility is needed.
-__device__ void make_reflector(double* col, int64_t len, double* tau, double* red, double* bcast) {
-  const int tid = threadIdx.x, bs = blockDim.x;
-  double ss = 0.0;
-  for (int64_t i = 1 + tid; i < len; i += bs) ss += col[i] * col[i];
-  const double xnorm2 = block_sum(ss, red);
-  if (tid == 0) bcast[0] = col[0];
-  __syncthreads();
-  const double alpha = bcast[0];
-  if (xnorm2 == 0.0) {
-    if (tid == 0) *tau = 0.0;
-    return;
-  }
-  const double beta = -copysign(hypot(alpha, sqrt(xnorm2)), alpha);
-  const double scal = 1.0 / (alpha - beta);
-  for (int64_t i = 1 + tid; i < len; i += bs) col[i] *= scal;
-  if (tid == 0) {
-    *tau = (beta - alpha) / beta;
-    col[0] = beta;
-  }
-}
-
-__global__ __launch_bounds__(kQrThreads) void k_qr_first(double* A, int64_t m, double* tau) {
-  __shared__ double red[kQrThreads / 64];
-  __shared__ double bcast[1];
-  make_reflector(A, m, tau, red, bcast);
-}
-
-// Step j: apply H_j to columns c = j+1+blockIdx.x (rows j..m-1); the block that
-// owns column j+1 then forms the next reflector from the values it wrote.
-__global__ __launch_bounds__(kQrThreads) void k_qr_step(double* A, int64_t lda, int64_t m, int64_t n,
-                                                        int64_t j, double* tau) {
-  __shared__ double red[kQrThreads / 64];
-  __shared__ double bcast[1];
-  const int tid = threadIdx.x, bs = blockDim.x;
-  const int64_t c = j + 1 + blockIdx.x;
-  const double* v = A + j + j * lda;  // v[0] = 1 implicitly
-  double* col = A + j + c * lda;
-  const int64_t len = m - j;
-  const double tj = tau[j];
-  if (tj != 0.0) {
-    double d = 0.0;
-    for (int64_t i = tid; i < len; i += bs) d += (i == 0 ? 1.0 : v[i]) * col[i];
-    const double w = block_sum(d, red) * tj;
-    for (int64_t i = tid; i < len; i += bs) col[i] -= (i == 0 ? 1.0 : v[i]) * w;
-  }
-  if (c == j + 1) {
-    // Reflector for column j+1 on rows j+1..m-1: element i of `col` is row j+i,
-    // so the sub-column starts at col+1.  Keep the same thread mapping: thread
-    // tid wrote rows j+tid+k*bs; make_reflector reads col+1 at offsets
-    // 1+tid+k*bs -> rows j+2+tid+k*bs, a different assignment, so fence.
-    __syncthreads();
-    __threadfence_block();
-    make_reflector(col + 1, len - 1, tau + j + 1, red, bcast);
-  }
-}
-
-// dorg2r step j: column j of Q from reflector j, and H_j applied to the
-// columns c > j already formed.
-__global__ __launch_bounds__(kQrThreads) void k_org_step(const double* A, int64_t lda, const double* tau,
-                                                         double* Q, int64_t ldq, int64_t m, int64_t j) {
-  __shared__ double red[kQrThreads / 64];
-  const int tid = threadIdx.x, bs = blockDim.x;
-  const int64_t c = j + blockIdx.x;
-  const double* v = A + j * lda;  // full column; rows > j hold v
-  const double tj = tau[j];
-  double* q = Q + c * ldq;
-  if (c == j) {
-    for (int64_t i = tid; i < m; i += bs)
-      q[i] = (i < j) ? 0.0 : (i == j ? 1.0 - tj : -tj * v[i]);
-    return;
-  }
-  if (tj == 0.0) return;
-  double d = 0.0;
-  for (int64_t i = j + tid; i < m; i += bs) d += (i == j ? 1.0 : v[i]) * q[i];
-  const double w = block_sum(d, red) * tj;
-  for (int64_t i = j + tid; i < m; i += bs) q[i] -= (i == j ? 1.0 : v[i]) * w;
 }
 
 __global__ void k_extract_r(int64_t n, const double* A, int64_t lda, double* R, int64_t ldr) {
@@ -823,15 +741,6 @@ void householder_qr(hipStream_t st, int64_t m, int64_t n, double* A, int64_t lda
   SKEMA_REQUIRE(m >= n && n >= 0, kErrShape, "householder_qr: needs rows >= cols");
   SKEMA_REQUIRE(lda >= m, kErrShape, "householder_qr: lda < rows");
   if (n == 0) return;
-  if (!work) {
-    hipLaunchKernelGGL(k_qr_first, dim3(1), dim3(kQrThreads), 0, st, A, m, tau);
-    check_launch("k_qr_first");
-    for (int64_t j = 0; j + 1 < n; ++j) {
-      hipLaunchKernelGGL(k_qr_step, dim3((unsigned)(n - j - 1)), dim3(kQrThreads), 0, st, A, lda, m, n, j, tau);
-    }
-    check_launch("k_qr_step");
-    return;
-  }
   const QrWork w = qr_work(work, m, n);
   for (int64_t j0 = 0; j0 < n; j0 += kQrPanel) {
     const int64_t jb = std::min(kQrPanel, n - j0), mp = m - j0;
@@ -849,17 +758,10 @@ void householder_qr(hipStream_t st, int64_t m, int64_t n, double* A, int64_t lda
   }
 }
 
-void householder_q(hipStream_t st, int64_t m, int64_t n, const double* A, int64_t lda, const double* tau,
-                   double* Q, int64_t ldq, DevBuf* work, GemmWorkspace* gws, bool reuse_t) {
+void householder_q(hipStream_t st, int64_t m, int64_t n, const double* A, int64_t lda, double* Q, int64_t ldq,
+                   DevBuf* work, GemmWorkspace* gws) {
   SKEMA_REQUIRE(m >= n && n >= 0 && lda >= m && ldq >= m, kErrShape, "householder_q: bad shape");
   if (n == 0) return;
-  if (!work) {
-    for (int64_t j = n - 1; j >= 0; --j) {
-      hipLaunchKernelGGL(k_org_step, dim3((unsigned)(n - j)), dim3(kQrThreads), 0, st, A, lda, tau, Q, ldq, m, j);
-    }
-    check_launch("k_org_step");
-    return;
-  }
   const QrWork w = qr_work(work, m, n);
   hipLaunchKernelGGL(k_eye_rect, dim3(grid_for_elems(m * n)), dim3(256), 0, st, m, n, Q, ldq);
   check_launch("k_eye_rect");
@@ -869,7 +771,7 @@ void householder_q(hipStream_t st, int64_t m, int64_t n, const double* A, int64_
     const int64_t jb = std::min(kQrPanel, n - j0), mp = m - j0, nq = n - j0;
     double* Q2 = Q + j0 + j0 * ldq;
     panel_v(st, A, lda, m, j0, jb, w);
-    const double* T = reuse_t ? w.Tall + (j0 / kQrPanel) * kQrPanel * kQrPanel : panel_t(st, m, j0, jb, tau, w, gws);
+    const double* T = w.Tall + (j0 / kQrPanel) * kQrPanel * kQrPanel;
     gemm_f64(st, 'T', 'N', jb, nq, mp, 1.0, w.V, mp, Q2, ldq, 0.0, w.W1, jb, gws);
     gemm_f64(st, 'N', 'N', jb, nq, jb, 1.0, T, jb, w.W1, jb, 0.0, w.W2, jb, gws);
     gemm_f64(st, 'N', 'N', mp, nq, jb, -1.0, w.V, mp, w.W2, jb, 1.0, Q2, ldq, gws);

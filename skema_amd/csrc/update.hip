@@ -302,13 +302,11 @@ void finalize_sketch(Sketch& sk) {
   sw.lap();
 
   // [P,~] = qr(X^T,0)  (:355-357)
-  transpose(st, k, n, sk.X.as<double>(), k, W, n);
-  householder_qr(st, n, k, W, n, tau, &c->qr, &c->gws);
-  householder_q(st, n, k, W, n, tau, P, n, &c->qr, &c->gws, true);
+  thin_qr(st, n, k, W, n, P, n, nullptr, 0, tau, &c->qr, &c->gws,
+          [&] { transpose(st, k, n, sk.X.as<double>(), k, W, n); });
   // [Q,~] = qr(Y,0)  (:381-383), on a copy: Y stays intact.
-  copy_matrix(st, m, k, sk.Y.as<double>(), m, W, m);
-  householder_qr(st, m, k, W, m, tau, &c->qr, &c->gws);
-  householder_q(st, m, k, W, m, tau, Q, m, &c->qr, &c->gws, true);
+  thin_qr(st, m, k, W, m, Q, m, nullptr, 0, tau, &c->qr, &c->gws,
+          [&] { copy_matrix(st, m, k, sk.Y.as<double>(), m, W, m); });
   tm["dgeqrf"] += sw.lap();
 
   // U1 = Phi*Q, U2 = Psi*P  (:409, :430)
@@ -332,14 +330,8 @@ void finalize_sketch(Sketch& sk) {
   double* Z2 = Z1 + k * s;  // k x k
   double* Z2t = Z2 + k * k; // k x k
   double* Cw = Z2t + k * k; // k x k (Jacobi works in place)
-  copy_matrix(st, s, k, PhiQ, s, F, s);
-  householder_qr(st, s, k, F, s, tau, &c->qr, &c->gws);
-  extract_r(st, k, F, s, T1, k);
-  householder_q(st, s, k, F, s, tau, U1, s, &c->qr, &c->gws, true);
-  copy_matrix(st, s, k, PsiP, s, F, s);
-  householder_qr(st, s, k, F, s, tau, &c->qr, &c->gws);
-  extract_r(st, k, F, s, T2, k);
-  householder_q(st, s, k, F, s, tau, U2, s, &c->qr, &c->gws, true);
+  thin_qr(st, s, k, F, s, U1, s, T1, k, tau, &c->qr, &c->gws, [&] { copy_matrix(st, s, k, PhiQ, s, F, s); });
+  thin_qr(st, s, k, F, s, U2, s, T2, k, tau, &c->qr, &c->gws, [&] { copy_matrix(st, s, k, PsiP, s, F, s); });
   tm["dgeqrf"] += sw.lap();
 
   // Z2 = (U1^T * Z) * U2  (:500, :515)
@@ -364,11 +356,8 @@ void finalize_sketch(Sketch& sk) {
     double* Rt = U1;
     double* Ur = U2;
     double* Vr = Z1;
-    copy_matrix(st, k, k, C, k, Cw, k);
-    householder_qr(st, k, k, Cw, k, tau, &c->qr, &c->gws);
-    extract_r(st, k, Cw, k, Z2, k);
+    thin_qr(st, k, k, Cw, k, Qc, k, Z2, k, tau, &c->qr, &c->gws, [&] { copy_matrix(st, k, k, C, k, Cw, k); });
     transpose(st, k, k, Z2, k, Rt, k);
-    householder_q(st, k, k, Cw, k, tau, Qc, k, &c->qr, &c->gws, true);
     jacobi_svd(st, k, Rt, k, Ur, k, Sv, Vr, k, &c->scratch);
     gemm_f64(st, 'N', 'N', k, k, k, 1.0, Qc, k, Vr, k, 0.0, Uc, k, &c->gws);
     copy_matrix(st, k, k, Ur, k, Vc, k);

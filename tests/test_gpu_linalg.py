@@ -51,3 +51,41 @@ def test_low_rank_approx_orders(S, m, n, k):
     assert np.abs(sv - np.linalg.svd(g.checkpoint("C"), compute_uv=False)).max() <= 1e-13 * sv[0] * np.sqrt(k)
     for M in (Q, P):
         assert np.abs(M.T @ M - np.eye(k)).max() <= 1e-12
+
+
+@pytest.mark.parametrize("m,n,k,decay,true_rank", [
+    (2000, 700, 33, 0.9, 700),   # a last panel of one column
+    (4100, 1030, 96, 0.9, 700),  # whole panels, a ragged last row tile
+    (64, 64, 64, 0.98, 64),      # square factors: the last column has no row below it
+    (900, 500, 40, 0.2, 500),    # columns dependent to 1e-16 within the first panel
+    (900, 500, 70, 0.8, 6),      # exactly of rank 6, below the range
+    (120, 100, 20, 0.9, 0),      # all zero
+])
+def test_thin_qr_panels(S, m, n, k, decay, true_rank):
+    """Panels factored by products, and the matrices they give up on (columns
+    too dependent), which are factored column by column: both have LAPACK's
+    signs, so Q, P, T1 and T2 compare as they are."""
+    print(f"case thin qr {m}x{n} k={k} decay={decay} rank={true_rank}", flush=True)
+    rng = np.random.default_rng(m + k)
+    A = (rng.standard_normal((m, n)) / np.sqrt(m)) @ np.diag(decay ** np.arange(n) * (np.arange(n) < true_rank))
+    A = A @ rng.standard_normal((n, n)) / np.sqrt(n)
+    p = O.AlgParams(matrix_m=m, matrix_n=n, rank=4, sketch_range=k, sketch_core=2 * k + 1, window=m)
+    osk = O.SketchySVD(p)
+    osk.linear_update(A)
+    Ur, Sr, Vr = osk.low_rank_approx()
+    g = S.SketchySVD(to_gpu_params(p), maps=gpu_maps({"Upsilon": osk.Upsilon, "Omega": osk.Omega, "Phi": osk.Phi,
+                                                      "Psi": osk.Psi}))
+    g.linear_update(dev(A))
+    U, Sv, V = g.low_rank_approx()
+    for name in ("Q", "P"):
+        M = g.checkpoint(name)
+        assert np.abs(M.T @ M - np.eye(k)).max() <= 1e-13 * np.sqrt(m), name
+    if true_rank >= k and decay > 0.5:
+        # forward error of a QR: eps (1e-16) times the condition of the k
+        # sketched columns, at most about 1e5 here
+        for name in ("Q", "P", "T1", "T2"):
+            assert O.rel_err(g.checkpoint(name), osk.checkpoints[name]) <= TOL, name
+    assert np.abs(Sv - Sr).max() <= TOL * max(Sr[0], 1e-300)
+    if true_rank:
+        Ua, Va = O.align_signs(U, V, Ur, Vr)
+        assert O.rel_err(Ua * Sv, Ur * Sr) <= TOL and O.rel_err(Va * Sv, Vr * Sr) <= TOL
