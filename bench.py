@@ -521,6 +521,7 @@ def bench_rbf(args, S, torch):
         res[form] = dict(form=form, ms=dt * 1e3, rows_per_s=n / dt, err=err, finalize_ms=fin_ms,
                          kernel_ms={kn: (v[1] / v[0] if v[0] else None) for kn, v in stats.items()},
                          right_avg_ms=stats["rbf_right"][1] / stats["rbf_right"][0],
+                         right_launches=stats["rbf_right"][0] / args.steps,
                          svals_head=[float(x) for x in Sv[:5].cpu()])
         print(f"[bench] rbf {form}: {dt * 1e3:.1f} ms/step, err {err:.6e}", file=sys.stderr, flush=True)
     base = res["fp64"]
@@ -530,8 +531,13 @@ def bench_rbf(args, S, torch):
             best = r
     nwin = math.ceil(n / w)
     avg_rows = n / nwin
-    # rbf_right per launch: sketch 2 w n (k+s) + Gram 2 w n d (algorithmic, one Gram)
-    flops_alg = 2.0 * avg_rows * n * (k + s) + 2.0 * avg_rows * n * d
+    # rbf_right per launch: sketch 2 w n (k+s); BF16 forms K in the same launch:
+    # + Gram 2 w n d (algorithmic, one Gram); FP64 takes K from memory, a range of
+    # points per launch
+    if best["form"] == "fp64":
+        flops_alg = 2.0 * n * n * (k + s) / best["right_launches"]
+    else:
+        flops_alg = 2.0 * avg_rows * n * (k + s) + 2.0 * avg_rows * n * d
     achieved = flops_alg / (best["right_avg_ms"] * 1e-3) / 1e12
     peak = PEAKS_TFLOPS[best["form"]]
     out = {

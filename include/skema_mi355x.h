@@ -57,7 +57,7 @@ extern "C" {
 #define SKEMA_KERNEL_GAUSSRBF 1
 
 /* Arithmetic of the sketch contractions (the finalize is always FP64).
- * Dense input takes every form; the fused RBF generator takes FP64 and BF16
+ * Dense input takes every form; the RBF generator takes FP64 and BF16
  * (BF16 Gram and sketch, FP32 exponent and accumulation); CSR input and
  * sparse-sign maps are FP64.  The state X, Y, Z is FP64 in every form. */
 #define SKEMA_PREC_FP64 0   /* plain: FP64 MFMA, the reference's arithmetic   */
@@ -184,8 +184,9 @@ int skema_map_rmap(skema_map* map, double alpha, const double* A, int64_t arows,
 /* GaussRBF<matrix_type>::compute for rows [row0,row0+rows) of the point set
  * (src/Skema_Kernel.cpp:5-81): K[i,j] = exp(-gamma*||x_{row0+i}-x_j||^2) for
  * all n points, K[i,row0+i] = 1.  points: device, n x d (ldp); K: device
- * rows x n (ldk).  This is the materialising form; the sketch update uses the
- * fused generator and never writes K. */
+ * rows x n (ldk).  This is the materialising form, for callers; the sketch update
+ * forms K itself (FP64: a range of points at a time in scratch memory of at most
+ * 1 GiB; BF16: inside its products, never written). */
 int skema_rbf_window(skema_ctx* ctx, const double* points, int64_t n, int64_t d, int64_t ldp, double gamma,
                      int64_t row0, int64_t rows, double* K, int64_t ldk);
 
@@ -315,7 +316,7 @@ int skema_residuals_csr(skema_ctx* ctx, int64_t m, int64_t n, int64_t r, const i
                         const double* val, const double* U, int64_t ldu, const double* S, const double* V,
                         int64_t ldv, double* rnorms);
 /* Same for A = the n x n Gaussian RBF matrix of the device point set
- * (n x d, ldp), generated in row windows by the fused generator (the
+ * (n x d, ldp), generated in row windows (the
  * GaussRBFWindow path of map_A_by_window, src/Skema_Residuals.hpp:60-121). */
 int skema_residuals_rbf(skema_ctx* ctx, const double* points, int64_t n, int64_t d, int64_t ldp, double gamma,
                         int64_t r, const double* U, int64_t ldu, const double* S, const double* V, int64_t ldv,

@@ -13,7 +13,7 @@
 #include "linalg.hpp"
 #include "lowp.hpp"
 #include "rbf.hpp"
-#include "rbf_fused.hpp"
+#include "rbf_tiles.hpp"
 #include "csr_pass.hpp"
 #include "residuals.hpp"
 #include "spd.hpp"
@@ -641,7 +641,7 @@ int skema_linear_update_rbf(skema_sketch* h, const double* points, int64_t ldp) 
     SKEMA_REQUIRE(sk.p.kernel == SKEMA_KERNEL_GAUSSRBF, kErrArg, "linear_update_rbf without an RBF window");
     check_mat(points, sk.p.n, sk.p.nfeat, ldp, "linear_update_rbf points");
     zero_state(sk);
-    for_each_window(sk, [&](int64_t r0, int64_t w) { update_rbf_window(sk, points, ldp, r0, w); });
+    for_each_window(sk, [&](int64_t r0, int64_t w) { update_rbf_window(sk, points, ldp, r0, w, r0 > 0); });
     sk.ctx->sync_if_needed();
   });
 }
@@ -1118,7 +1118,7 @@ int skema_spd_linear_update_rbf(skema_spd* h, const double* points, int64_t ldp)
     SKEMA_REQUIRE(sp.p.kernel == SKEMA_KERNEL_GAUSSRBF, kErrArg, "spd linear_update_rbf without an RBF window");
     check_mat(points, sp.p.n, sp.p.nfeat, ldp, "spd points");
     spd_zero(sp);
-    spd_windows(sp, [&](int64_t r0, int64_t w) { spd_update_rbf(sp, points, ldp, r0, w); });
+    spd_windows(sp, [&](int64_t r0, int64_t w) { spd_update_rbf(sp, points, ldp, r0, w, r0 > 0); });
     sp.updated = true;
     sp.ctx->sync_if_needed();
   });

@@ -448,10 +448,21 @@ __global__ __launch_bounds__(64 * KW) void k_gemm_ksplit(KArgs g) {
   }
 }
 
-// Deterministic split-K reduction: 32 consecutive elements x 8 groups of
-// slices per block (group q sums slices q, q + 8, ... in order, then the
-// groups are added in order), so many slices of a small product are read by
-// many threads.
+// Deterministic split-K reductions.  Large outputs: one element per thread, the
+// slices added in order.  Bound by reading the partials: 59 MB (6 slices of
+// 2048 x 604) took 52 us in the other form.
+__global__ __launch_bounds__(256) void k_splitk_sum(const double* part, int splits, int64_t M, int64_t total, GemmOut o) {
+  const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (e >= total) return;
+  double s = 0.0;
+#pragma unroll 4
+  for (int z = 0; z < splits; ++z) s += part[(int64_t)z * total + e];
+  const int64_t j = total < (int64_t)1 << 32 ? (int64_t)((uint32_t)e / (uint32_t)M) : e / M;
+  store_out(o, e - j * M, j, s);
+}
+// Small outputs: 32 consecutive elements x 8 groups of slices per block (group q
+// sums slices q, q + 8, ... in order, then the groups are added in order), so
+// many slices of a small product are read by many threads.
 __global__ __launch_bounds__(256) void k_splitk_reduce(const double* part, int splits, int64_t M, int64_t total,
                                                        GemmOut o) {
   __shared__ double red[8][33];
@@ -597,8 +608,13 @@ void gemm_f64(hipStream_t stream, char transA, char transB, int64_t M, int64_t N
   }
   if (p.splits > 1) {
     const int64_t total = M * N;
-    const int blocks = (int)std::min<int64_t>(cdiv(total, 32), 8192);
-    hipLaunchKernelGGL(k_splitk_reduce, dim3(blocks), dim3(256), 0, stream, a.partial, p.splits, M, total, out);
+    // from 65536 elements one thread each fills the chip
+    if (total >= 65536)
+      hipLaunchKernelGGL(k_splitk_sum, dim3((unsigned)cdiv(total, 256)), dim3(256), 0, stream, a.partial, p.splits, M,
+                         total, out);
+    else
+      hipLaunchKernelGGL(k_splitk_reduce, dim3((unsigned)cdiv(total, 32)), dim3(256), 0, stream, a.partial, p.splits, M,
+                         total, out);
     check_launch("k_splitk_reduce");
   }
 }

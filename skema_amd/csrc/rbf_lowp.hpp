@@ -6,7 +6,7 @@
 namespace skema {
 
 bool rbf_bf16_supported(const Sketch& sk);
-void update_rbf_window_bf16(Sketch& sk, const double* points, int64_t ldp, int64_t row0, int64_t rows);
+void update_rbf_window_bf16(Sketch& sk, const double* points, int64_t ldp, int64_t row0, int64_t rows, bool again);
 
 // Features of the rounded point set: d padded to 32, 64 or 128.
 inline int rbf_bf16_padded_features(int64_t d) { return d <= 32 ? 32 : (d <= 64 ? 64 : 128); }

@@ -6,9 +6,8 @@
 // A V and A^T U are formed on the device from the input as it is held: a
 // dense column-major A through the FP64 GEMM, a CSR A through the row
 // products and a column-compressed copy, and the Gaussian RBF matrix of a
-// point set through the fused generator window by window (K is symmetric,
-// so A^T U = K U comes out of the same pass as K V, and K is never
-// written).  The norms are one block per column with a fixed-order
+// point set window by window (K is symmetric, so A^T U = K U comes out of the
+// same pass as K V).  The norms are one block per column with a fixed-order
 // reduction, so repeated calls give identical bits.
 #include <algorithm>
 #include <vector>
@@ -16,7 +15,7 @@
 #include "gemm.hpp"
 #include "linalg.hpp"
 #include "rbf.hpp"
-#include "rbf_fused.hpp"
+#include "rbf_tiles.hpp"
 #include "residuals.hpp"
 #include "sparse.hpp"
 #include "util.hpp"
@@ -64,7 +63,7 @@ void norms_to_host(hipStream_t st, int64_t r, int64_t m1, const double* P, int64
 }
 
 // K V (and K U when U is given) over row windows of the RBF matrix of the
-// point set: one fused pass with the operator [V^T; U^T].
+// point set: one product per window with the operator [V^T; U^T].
 void rbf_products(Ctx* c, const double* X, int64_t n, int64_t d, int64_t ldp, double gamma, int64_t r,
                   const double* V, int64_t ldv, const double* U, int64_t ldu, int64_t window, double* KV,
                   double* KU) {
@@ -76,12 +75,12 @@ void rbf_products(Ctx* c, const double* X, int64_t n, int64_t d, int64_t ldp, do
   if (U) transpose(st, n, r, U, ldu, OP.as<double>() + r, h);
   for (int64_t r0 = 0; r0 < n; r0 += window) {
     const int64_t rows = std::min(window, n - r0);
-    RbfArgs a;
-    a.X = X; a.ldp = ldp; a.d = d; a.nrm = nrm.as<double>(); a.gamma = gamma; a.row0 = r0;
-    a.M = rows; a.N = h; a.K = n; a.OP = OP.as<double>(); a.ldop = h;
-    a.out.C1 = KV + r0; a.out.ldc1 = n; a.out.alpha1 = 1.0; a.out.beta1 = 0.0; a.out.nsplit = r;
-    a.out.C2 = U ? KU + r0 : KV + r0; a.out.ldc2 = n; a.out.alpha2 = 1.0; a.out.beta2 = 0.0;
-    rbf_fused_right_f64(st, a, &c->gws.buf);
+    RbfRows w;
+    w.X = X; w.n = n; w.ldp = ldp; w.d = d; w.nrm = nrm.as<double>(); w.gamma = gamma; w.row0 = r0; w.rows = rows;
+    GemmOut o;
+    o.C1 = KV + r0; o.ldc1 = n; o.alpha1 = 1.0; o.beta1 = 0.0; o.nsplit = r;
+    o.C2 = U ? KU + r0 : KV + r0; o.ldc2 = n; o.alpha2 = 1.0; o.beta2 = 0.0;
+    rbf_products_f64(c, w, nullptr, 0, 0, GemmOut{}, OP.as<double>(), h, h, o, false);
   }
 }
 

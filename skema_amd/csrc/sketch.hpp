@@ -35,6 +35,7 @@ struct Ctx {
   GemmWorkspace gws;
   DevBuf scratch;  // general grow-only scratch
   DevBuf qr;       // blocked QR workspace (panel reflectors, T, products)
+  DevBuf kwin;     // rows of an RBF matrix, a range of points at a time (at most 1 GiB)
   KernelStats stats;
   void sync_if_needed() {
     if (!async_calls) SKEMA_HIP(hipStreamSynchronize(stream));
@@ -150,7 +151,9 @@ double now_seconds();
 void update_dense_window(Sketch& sk, const double* H, int64_t ldh, int64_t row0, int64_t rows);
 void update_csr_window(Sketch& sk, const int64_t* rowptr, const int32_t* col, const double* val, int64_t row0,
                        int64_t rows);
-void update_rbf_window(Sketch& sk, const double* points, int64_t ldp, int64_t row0, int64_t rows);
+// again: a later window of one linear_update (what an earlier one derived from
+// the points, in the sketch's scratch, still holds).
+void update_rbf_window(Sketch& sk, const double* points, int64_t ldp, int64_t row0, int64_t rows, bool again = false);
 void prepare_sketch_maps(Sketch& sk);
 void finalize_sketch(Sketch& sk);
 

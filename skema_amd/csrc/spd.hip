@@ -5,7 +5,7 @@
 // counter, :795-858, so it sketches window 0 only -- not reproduced).
 // Products: dense A_w on the FP64 GEMM (or A_w Omega with a sparse Omega
 // through the dense x CSR^T kernel), CSR A_w through the row products, and
-// the Gaussian RBF window through the fused generator (K never written).
+// the Gaussian RBF window's rows formed in tiles and multiplied by the GEMM.
 //
 // Fixed-rank approximation (Tropp, Yurtsever, Udell, Cevher 2017, Alg. 3, as
 // the reference orders it, :934-1151):
@@ -22,7 +22,7 @@
 #include "gemm.hpp"
 #include "linalg.hpp"
 #include "rbf.hpp"
-#include "rbf_fused.hpp"
+#include "rbf_tiles.hpp"
 #include "sparse.hpp"
 #include "spd.hpp"
 #include "util.hpp"
@@ -159,19 +159,17 @@ void spd_update_csr(Spd& sp, const int64_t* rowptr, const int32_t* col, const do
   else csr_right_dense(c->stream, rowptr, col, val, rows, sp.omT.as<double>(), sp.k, sp.k, o);
 }
 
-void spd_update_rbf(Spd& sp, const double* points, int64_t ldp, int64_t row0, int64_t rows) {
+void spd_update_rbf(Spd& sp, const double* points, int64_t ldp, int64_t row0, int64_t rows, bool again) {
   Ctx* c = sp.ctx;
   hipStream_t st = c->stream;
   Timed t(c, "spd_update");
   const int64_t n = sp.p.n;
   sp.win.reserve((size_t)n * sizeof(double));
   double* nrm = sp.win.as<double>();
-  row_norms2(st, points, n, sp.p.nfeat, ldp, nrm);
-  RbfArgs a;
-  a.X = points; a.ldp = ldp; a.d = sp.p.nfeat; a.nrm = nrm; a.gamma = sp.p.gamma; a.row0 = row0;
-  a.M = rows; a.N = sp.k; a.K = n; a.OP = sp.omT.as<double>(); a.ldop = sp.k;
-  a.out = y_out(sp, row0);
-  rbf_fused_right_f64(st, a, &c->gws.buf);
+  if (!again) row_norms2(st, points, n, sp.p.nfeat, ldp, nrm);
+  RbfRows w;
+  w.X = points; w.n = n; w.ldp = ldp; w.d = sp.p.nfeat; w.nrm = nrm; w.gamma = sp.p.gamma; w.row0 = row0; w.rows = rows;
+  rbf_products_f64(c, w, nullptr, 0, 0, GemmOut{}, sp.omT.as<double>(), sp.k, sp.k, y_out(sp, row0), false);
 }
 
 void spd_low_rank_approx(Spd& sp, int shift_removal, double* U, int64_t ldu, double* S) {

@@ -23,7 +23,8 @@ void spd_prepare(Spd& sp);
 void spd_update_dense(Spd& sp, const double* H, int64_t ldh, int64_t row0, int64_t rows);
 void spd_update_csr(Spd& sp, const int64_t* rowptr, const int32_t* col, const double* val, int64_t row0,
                     int64_t rows);
-void spd_update_rbf(Spd& sp, const double* points, int64_t ldp, int64_t row0, int64_t rows);
+// again: a later window of one linear_update (the points' norms are at hand).
+void spd_update_rbf(Spd& sp, const double* points, int64_t ldp, int64_t row0, int64_t rows, bool again = false);
 // U (n x r, ldu, device) and S (r, device); shift_removal: 0 removes the
 // shift eps ||Y||_2 (Tropp et al. 2017, Alg. 3), 1 subtracts ||Y||_2 as the
 // reference does (src/Skema_SketchySVD.cpp:1141-1145).

@@ -15,7 +15,7 @@
 #include "linalg.hpp"
 #include "lowp.hpp"
 #include "rbf.hpp"
-#include "rbf_fused.hpp"
+#include "rbf_tiles.hpp"
 #include "rbf_lowp.hpp"
 #include "sketch.hpp"
 #include "sparse.hpp"
@@ -237,15 +237,15 @@ void update_csr_window(Sketch& sk, const int64_t* rowptr, const int32_t* col, co
   }
 }
 
-void update_rbf_window(Sketch& sk, const double* points, int64_t ldp, int64_t row0, int64_t rows) {
+void update_rbf_window(Sketch& sk, const double* points, int64_t ldp, int64_t row0, int64_t rows, bool again) {
   Ctx* c = sk.ctx;
   const int64_t n = sk.p.n;
-  if (!sk.sparse_maps && rbf_fused_supported(sk)) {
-    update_rbf_window_fused(sk, points, ldp, row0, rows);
+  if (rbf_tiles_supported(sk)) {
+    update_rbf_window_tiles(sk, points, ldp, row0, rows, again);
     return;
   }
   if (rbf_bf16_supported(sk)) {
-    update_rbf_window_bf16(sk, points, ldp, row0, rows);
+    update_rbf_window_bf16(sk, points, ldp, row0, rows, again);
     return;
   }
   sk.win.reserve((size_t)rows * n * sizeof(double));

@@ -45,3 +45,29 @@ def test_products_of_every_shape(S, tA, tB, M, N, K):
         want = 1.5 * ref + (beta * C if beta else 0.0)
         err = np.linalg.norm(host(out) - want) / np.linalg.norm(want)
         assert err <= TOL, (beta, err)
+
+
+@pytest.mark.parametrize("n,d,window", [(300, 1, 300), (1000, 17, 129), (16500, 5, 16500)])
+def test_rbf_rows_in_ranges(S, n, d, window):
+    """K's rows formed in tiles with row and point remainders and feature
+    counts off the slices of 16; at 16500 x 16500 in three ranges of points
+    (1 GiB), whose products add up.  Against windows of 128 rows, and the small
+    ones against K formed by torch."""
+    print(f"case rbf rows n={n} d={d} w={window}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(n)
+    X = torch.randn((d, n), dtype=torch.float64, device="cuda", generator=g).t()
+
+    def state(w):
+        p = S.AlgParams(matrix_m=n, matrix_n=n, rank=5, sketch_range=21, sketch_core=43, window=w,
+                        kernel_func="gaussrbf", kernel_gamma=0.5 / d, nfeat=d)
+        sk = S.SketchySVD(p, maps=S.make_maps(p, dist="normal"))
+        sk.linear_update(X)
+        return sk
+
+    whole, parts = state(window), state(128)
+    for a, b in zip(whole.state(), parts.state()):
+        assert np.linalg.norm(a - b) <= TOL * np.linalg.norm(b)
+    if n <= 1000:
+        K = np.exp(-0.5 / d * torch.cdist(X.cpu(), X.cpu()).numpy() ** 2)
+        om = whole.maps["Omega"].download()
+        assert np.linalg.norm(whole.state()[1] - K @ om.T) <= TOL * np.linalg.norm(K @ om.T)
