@@ -155,10 +155,7 @@ void check_window(const Sketch& sk, int64_t row0, int64_t rows) {
 
 // Reads rowptr[0] and rowptr[rows] of a device CSR window and checks that
 // col/val cover them.
-// ends_out (optional): rowptr[0] and rowptr[rows], read here anyway, so the
-// caller's own validation needs no second round trip.
-void check_csr_window(const int64_t* rowptr, const int32_t* col, const double* val, int64_t rows, hipStream_t st,
-                      int64_t* ends_out = nullptr) {
+void check_csr_window(const int64_t* rowptr, const int32_t* col, const double* val, int64_t rows, hipStream_t st) {
   check_dev(rowptr, (size_t)(rows + 1) * sizeof(int64_t), "rowptr");
   int64_t ends[2];
   SKEMA_HIP(hipMemcpyAsync(&ends[0], rowptr, sizeof(int64_t), hipMemcpyDeviceToHost, st));
@@ -169,10 +166,38 @@ void check_csr_window(const int64_t* rowptr, const int32_t* col, const double* v
     check_dev(col, (size_t)ends[1] * sizeof(int32_t), "col");
     check_dev(val, (size_t)ends[1] * sizeof(double), "val");
   }
-  if (ends_out) {
-    ends_out[0] = ends[0];
-    ends_out[1] = ends[1];
+}
+
+// Whole elements of `size` bytes from p to the end of its device allocation
+// (none when p is not in one).
+int64_t device_room(const void* p, size_t size) {
+  hipDeviceptr_t base = nullptr;
+  size_t bytes = 0;
+  if (!p) return 0;
+  if (hipMemGetAddressRange(&base, &bytes, const_cast<void*>(p)) != hipSuccess) {
+    (void)hipGetLastError();
+    return 0;
   }
+  return (int64_t)((bytes - (size_t)(static_cast<const char*>(p) - static_cast<const char*>(base))) / size);
+}
+
+// The same and the window's entries (row pointers in order, column indices in
+// [0, cols)) with one launch and one wait; returns the nonzeros.  Nothing is
+// indexed with rowptr or col before they have passed.
+int64_t check_csr_entries(Ctx* c, const int64_t* rowptr, const int32_t* col, const double* val, int64_t rows,
+                          int64_t cols) {
+  check_dev(rowptr, (size_t)(rows + 1) * sizeof(int64_t), "rowptr");
+  const int64_t room = std::min(device_room(col, sizeof(int32_t)), device_room(val, sizeof(double)));
+  const CsrInfo f = inspect_csr(c, rowptr, col, rows, cols, room);
+  SKEMA_REQUIRE(f.first >= 0 && f.last >= f.first, kErrArg, "CSR: bad rowptr");
+  if (f.last > 0) {
+    check_dev(col, (size_t)f.last * sizeof(int32_t), "col");
+    check_dev(val, (size_t)f.last * sizeof(double), "val");
+  }
+  SKEMA_REQUIRE(f.last - f.first < ((int64_t)1 << 31), kErrArg, "CSR window: bad rowptr range");
+  SKEMA_REQUIRE(!(f.flags & 1), kErrArg, "CSR window: rowptr is not non-decreasing");
+  SKEMA_REQUIRE(!(f.flags & 2), kErrArg, "CSR window: column index outside [0, n)");
+  return f.last - f.first;
 }
 
 template <class Fn>
@@ -574,8 +599,8 @@ int skema_update_csr(skema_sketch* h, const int64_t* rowptr, const int32_t* col,
     set_device(sk.ctx);
     SKEMA_REQUIRE(sk.p.kernel == SKEMA_KERNEL_NONE, kErrArg, "update_csr on an RBF sketch");
     check_window(sk, row0, rows);
-    check_csr_window(rowptr, col, val, rows, sk.ctx->stream);
-    update_csr_window(sk, rowptr, col, val, row0, rows);
+    const int64_t nnz = check_csr_entries(sk.ctx, rowptr, col, val, rows, sk.p.n);
+    update_csr_window(sk, rowptr, col, val, row0, rows, nnz);
     sk.finalized = false;
     sk.ctx->sync_if_needed();
   });
@@ -623,12 +648,11 @@ int skema_linear_update_csr(skema_sketch* h, const int64_t* rowptr, const int32_
     Sketch& sk = h->s;
     set_device(sk.ctx);
     SKEMA_REQUIRE(sk.p.kernel == SKEMA_KERNEL_NONE, kErrArg, "linear_update_csr on an RBF sketch");
-    int64_t ends[2];
-    check_csr_window(rowptr, col, val, sk.p.m, sk.ctx->stream, ends);
+    const int64_t nnz = check_csr_entries(sk.ctx, rowptr, col, val, sk.p.m, sk.p.n);
     // the window loop from a zero state in one pass over the whole CSR; the
     // pass writes every entry of X, Y and Z, so the state is not cleared first
     sk.finalized = false;
-    update_csr_all(sk, rowptr, col, val, ends);
+    update_csr_all(sk, rowptr, col, val, nnz);
     sk.ctx->sync_if_needed();
   });
 }
@@ -916,8 +940,8 @@ int skema_residuals_csr(skema_ctx* ctx, int64_t m, int64_t n, int64_t r, const i
     Ctx* c = &ctx->c;
     set_device(c);
     check_factors(m, n, r, U, ldu, S, V, ldv, rnorms);
-    check_csr_window(rowptr, col, val, m, c->stream);
-    residuals_csr(c, m, n, r, rowptr, col, val, U, ldu, S, V, ldv, rnorms);
+    const int64_t nnz = check_csr_entries(c, rowptr, col, val, m, n);
+    residuals_csr(c, m, n, r, nnz, rowptr, col, val, U, ldu, S, V, ldv, rnorms);
   });
 }
 

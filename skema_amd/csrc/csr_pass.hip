@@ -19,8 +19,9 @@
 //   Both accumulate in LDS in int64 fixed point (fixedpoint.hpp),
 //   so every sum is the same whatever order the atomics land in: X, Y, Z
 //   are bitwise reproducible.
-// Dense maps: one wave per column (left) or row (right), lanes own map rows,
-//   nonzeros in ascending row order over a sorted CSC (deterministic).
+// Dense maps: the window kernels over the whole matrix (sparse.hip: one wave per
+//   column, left, or row, right, lanes own map rows, nonzeros in ascending row
+//   order over a sorted CSC: deterministic).
 //   core  Z = W Psi^T: dense x CSR^T gather (sparse Psi) or the FP64 GEMM.
 #include <vector>
 
@@ -571,69 +572,6 @@ __global__ __launch_bounds__(256) void k_right_fx(const int64_t* rowptr, const i
   }
 }
 
-// out(p, j) = sum over column j's nonzeros (i, a) of a cw[i / window] M(p, i),
-// M dense (P x m logical, column-major, ld ldm); one wave per column, lanes
-// own rows p (PR per lane).
-template <int PR>
-__global__ __launch_bounds__(256) void k_left_all_dense(const int64_t* cptr, const int32_t* crow, const double* cval,
-                                                        int64_t ncols, const double* M, int64_t ldm, int64_t P,
-                                                        const double* cw, int64_t window, double* out, int64_t ldo) {
-  const int lane = threadIdx.x & 63;
-  const int64_t j = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (j >= ncols) return;
-  double acc[PR];
-#pragma unroll
-  for (int r = 0; r < PR; ++r) acc[r] = 0.0;
-  for (int64_t e = cptr[j]; e < cptr[j + 1]; ++e) {
-    const int64_t i = crow[e];
-    const double a = cval[e] * cw[(uint32_t)i / (uint32_t)window];
-    const double* mcol = M + i * ldm;
-#pragma unroll
-    for (int r = 0; r < PR; ++r) {
-      const int64_t p = lane + 64 * r;
-      if (p < P) acc[r] += a * mcol[p];
-    }
-  }
-#pragma unroll
-  for (int r = 0; r < PR; ++r) {
-    const int64_t p = lane + 64 * r;
-    if (p < P) out[p + j * ldo] = acc[r];
-  }
-}
-
-// Y(i, p) = nu Y + eta * sum over row i's nonzeros (j, a) of a M(p, j), M dense
-// (P x n logical, ld ldm); one wave per row, lanes own p.
-template <int PR>
-__global__ __launch_bounds__(256) void k_right_all_dense(const int64_t* rowptr, const int32_t* col, const double* val,
-                                                         int64_t rows, const double* M, int64_t ldm, int64_t P,
-                                                         double eta, double nu, double* Y, int64_t ldy) {
-  const int lane = threadIdx.x & 63;
-  const int64_t i = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (i >= rows) return;
-  double acc[PR];
-#pragma unroll
-  for (int r = 0; r < PR; ++r) acc[r] = 0.0;
-  for (int64_t e = rowptr[i]; e < rowptr[i + 1]; ++e) {
-    const double a = val[e];
-    const double* mcol = M + (int64_t)col[e] * ldm;
-#pragma unroll
-    for (int r = 0; r < PR; ++r) {
-      const int64_t p = lane + 64 * r;
-      if (p < P) acc[r] += a * mcol[p];
-    }
-  }
-#pragma unroll
-  for (int r = 0; r < PR; ++r) {
-    const int64_t p = lane + 64 * r;
-    if (p < P) {
-      double* y = Y + i + p * ldy;
-      *y = (nu != 0.0) ? nu * *y + eta * acc[r] : eta * acc[r];
-    }
-  }
-}
-
-unsigned nblocks(int64_t work, int64_t per) { return (unsigned)std::max<int64_t>(1, cdiv(work, per)); }
-
 SpMapCols map_cols(const Map& M) {
   SpMapCols c;
   if (M.ell_zeta > 0) {
@@ -758,30 +696,9 @@ bool csc_by_buckets(hipStream_t st, const int64_t* rowptr, const int32_t* col, c
   return true;
 }
 
-void left_dense(hipStream_t st, const CscWindow& H, const double* M, int64_t ldm, int64_t P, const double* cw,
-                int64_t window, double* out, int64_t ldo) {
-  for (int64_t p0 = 0; p0 < P; p0 += 512) {
-    const int64_t pc = std::min<int64_t>(512, P - p0);
-    const dim3 grid(nblocks(H.cols, 4));
-    const double* Mp = M + p0;
-    double* op = out + p0;
-    const int pr = (int)cdiv(pc, 64);
-    if (pr <= 2)
-      hipLaunchKernelGGL(k_left_all_dense<2>, grid, dim3(256), 0, st, H.ptr, H.row, H.val, H.cols, Mp, ldm, pc, cw,
-                         window, op, ldo);
-    else if (pr <= 4)
-      hipLaunchKernelGGL(k_left_all_dense<4>, grid, dim3(256), 0, st, H.ptr, H.row, H.val, H.cols, Mp, ldm, pc, cw,
-                         window, op, ldo);
-    else
-      hipLaunchKernelGGL(k_left_all_dense<8>, grid, dim3(256), 0, st, H.ptr, H.row, H.val, H.cols, Mp, ldm, pc, cw,
-                         window, op, ldo);
-    check_launch("k_left_all_dense");
-  }
-}
-
 }  // namespace
 
-void update_csr_all(Sketch& sk, const int64_t* rowptr, const int32_t* col, const double* val, const int64_t* ends) {
+void update_csr_all(Sketch& sk, const int64_t* rowptr, const int32_t* col, const double* val, int64_t nnz) {
   Ctx* c = sk.ctx;
   hipStream_t st = c->stream;
   const int64_t k = sk.k, s = sk.s, m = sk.p.m, n = sk.p.n;
@@ -805,19 +722,13 @@ void update_csr_all(Sketch& sk, const int64_t* rowptr, const int32_t* col, const
   double* Wm = nullptr;
   {
     Timed t(c, "window");
-    scr.reserve(align_up((size_t)W * sizeof(double), 256) + align_up((size_t)s * n * sizeof(double), 256) + 256);
+    scr.reserve(align_up((size_t)W * sizeof(double), 256) + (size_t)s * n * sizeof(double));
     cw = scr.as<double>();
     Wm = reinterpret_cast<double*>(scr.as<char>() + align_up((size_t)W * sizeof(double), 256));
-    int* flag = reinterpret_cast<int*>(scr.as<char>() + align_up((size_t)W * sizeof(double), 256) +
-                                       align_up((size_t)s * n * sizeof(double), 256));
     SKEMA_HIP(hipMemcpyAsync(cw, hw.data(), (size_t)W * sizeof(double), hipMemcpyHostToDevice, st));
-    bool done = false;
-    if (sk.sparse_maps) {
-      // the fixed-point products take the column entries in any order
-      const int64_t nnz = validate_csr_window(st, rowptr, col, m, n, flag, ends);
-      done = csc_by_buckets(st, rowptr, col, val, m, n, nnz, sk.win, H);
-    }
-    if (!done) H = csr_window_to_csc(st, rowptr, col, val, m, n, sk.win, /*sorted=*/true);
+    // the fixed-point products take the column entries in any order
+    if (!sk.sparse_maps || !csc_by_buckets(st, rowptr, col, val, m, n, nnz, sk.win, H))
+      H = csr_window_to_csc(st, rowptr, col, val, m, n, nnz, sk.win, /*sorted=*/true);
   }
   double* X = sk.X.as<double>();
   double* Y = sk.Y.as<double>();
@@ -842,27 +753,15 @@ void update_csr_all(Sketch& sk, const int64_t* rowptr, const int32_t* col, const
   }
   {
     Timed t(c, "sketch_left");
-    left_dense(st, H, sk.upsL, sk.ldups, k, cw, window, X, k);
-    left_dense(st, H, sk.phiL, sk.ldphi, s, cw, window, Wm, s);
+    csc_left_dense(st, H, sk.upsL, sk.ldups, 0, k, 1.0, 0.0, X, k, cw, window);
+    csc_left_dense(st, H, sk.phiL, sk.ldphi, 0, s, 1.0, 0.0, Wm, s, cw, window);
   }
   {
     Timed t(c, "sketch_right");
-    const double* Om = sk.omps.as<double>();  // Omega = rows 0..k-1 of [Omega; Psi], ld k+s
-    for (int64_t p0 = 0; p0 < k; p0 += 512) {
-      const int64_t pc = std::min<int64_t>(512, k - p0);
-      const dim3 grid(nblocks(m, 4));
-      const int pr = (int)cdiv(pc, 64);
-      if (pr <= 2)
-        hipLaunchKernelGGL(k_right_all_dense<2>, grid, dim3(256), 0, st, rowptr, col, val, m, Om + p0, k + s, pc, eta,
-                           0.0, Y + p0 * m, m);
-      else if (pr <= 4)
-        hipLaunchKernelGGL(k_right_all_dense<4>, grid, dim3(256), 0, st, rowptr, col, val, m, Om + p0, k + s, pc, eta,
-                           0.0, Y + p0 * m, m);
-      else
-        hipLaunchKernelGGL(k_right_all_dense<8>, grid, dim3(256), 0, st, rowptr, col, val, m, Om + p0, k + s, pc, eta,
-                           0.0, Y + p0 * m, m);
-      check_launch("k_right_all_dense");
-    }
+    GemmOut o;  // Omega = rows 0..k-1 of [Omega; Psi], ld k+s
+    o.C1 = Y; o.ldc1 = m; o.alpha1 = eta; o.beta1 = 0.0; o.nsplit = k;
+    o.C2 = Y; o.ldc2 = m;
+    csr_right_dense(st, rowptr, col, val, m, sk.omps.as<double>(), k + s, k, o);
   }
   {
     Timed t(c, "sketch_core");

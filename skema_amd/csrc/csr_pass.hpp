@@ -5,7 +5,7 @@
 
 namespace skema {
 
-// ends: rowptr[0] and rowptr[m] as already read by the caller.
-void update_csr_all(Sketch& sk, const int64_t* rowptr, const int32_t* col, const double* val, const int64_t* ends);
+// nnz: the nonzeros, as inspect_csr found them.
+void update_csr_all(Sketch& sk, const int64_t* rowptr, const int32_t* col, const double* val, int64_t nnz);
 
 }  // namespace skema

@@ -113,7 +113,7 @@ void residuals_dense(Ctx* c, int64_t m, int64_t n, int64_t r, const double* A, i
   norms_to_host(st, r, m, AV.as<double>(), m, U, ldu, n, AtU.as<double>(), n, V, ldv, S, rnorms);
 }
 
-void residuals_csr(Ctx* c, int64_t m, int64_t n, int64_t r, const int64_t* rowptr, const int32_t* col,
+void residuals_csr(Ctx* c, int64_t m, int64_t n, int64_t r, int64_t nnz, const int64_t* rowptr, const int32_t* col,
                    const double* val, const double* U, int64_t ldu, const double* S, const double* V, int64_t ldv,
                    double* rnorms) {
   if (r == 0) return;
@@ -128,7 +128,7 @@ void residuals_csr(Ctx* c, int64_t m, int64_t n, int64_t r, const int64_t* rowpt
   csr_right_dense(st, rowptr, col, val, m, Vt.as<double>(), r, r, o);
   // (A^T U)^T = U^T A: column products over the CSC copy (rows in order)
   transpose(st, m, r, U, ldu, Ut.as<double>(), r);
-  const CscWindow H = csr_window_to_csc(st, rowptr, col, val, m, n, scratch, true);
+  const CscWindow H = csr_window_to_csc(st, rowptr, col, val, m, n, nnz, scratch, true);
   csc_left_dense(st, H, Ut.as<double>(), r, 0, r, 1.0, 0.0, AtUt.as<double>(), r);
   transpose(st, r, n, AtUt.as<double>(), r, AtU.as<double>(), n);
   norms_to_host(st, r, m, AV.as<double>(), m, U, ldu, n, AtU.as<double>(), n, V, ldv, S, rnorms);

@@ -8,7 +8,7 @@ namespace skema {
 // U (m x r), S (r), V (n x r) on the device; rnorms on the host.
 void residuals_dense(Ctx* c, int64_t m, int64_t n, int64_t r, const double* A, int64_t lda, const double* U,
                      int64_t ldu, const double* S, const double* V, int64_t ldv, double* rnorms);
-void residuals_csr(Ctx* c, int64_t m, int64_t n, int64_t r, const int64_t* rowptr, const int32_t* col,
+void residuals_csr(Ctx* c, int64_t m, int64_t n, int64_t r, int64_t nnz, const int64_t* rowptr, const int32_t* col,
                    const double* val, const double* U, int64_t ldu, const double* S, const double* V, int64_t ldv,
                    double* rnorms);
 // A = the n x n Gaussian RBF matrix of the point set (generated by row

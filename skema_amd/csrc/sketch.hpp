@@ -26,6 +26,17 @@ struct KernelStats {
   ~KernelStats();
 };
 
+// Pinned host memory owned by a library object.
+struct HostBuf {
+  void* p = nullptr;
+  HostBuf() = default;
+  HostBuf(const HostBuf&) = delete;
+  HostBuf& operator=(const HostBuf&) = delete;
+  ~HostBuf() {
+    if (p) (void)hipHostFree(p);
+  }
+};
+
 struct Ctx {
   int device = 0;
   hipStream_t stream = nullptr;
@@ -36,6 +47,8 @@ struct Ctx {
   DevBuf scratch;  // general grow-only scratch
   DevBuf qr;       // blocked QR workspace (panel reflectors, T, products)
   DevBuf kwin;     // rows of an RBF matrix, a range of points at a time (at most 1 GiB)
+  DevBuf csr_dev;    // inspect_csr's result (three 8-byte words), its flags zero between calls
+  HostBuf csr_host;  // the same, pinned
   KernelStats stats;
   void sync_if_needed() {
     if (!async_calls) SKEMA_HIP(hipStreamSynchronize(stream));
@@ -149,8 +162,9 @@ double now_seconds();
 
 // Update kernels (per window); implemented in update.hip.
 void update_dense_window(Sketch& sk, const double* H, int64_t ldh, int64_t row0, int64_t rows);
+// nnz: the window's nonzeros, as inspect_csr found them.
 void update_csr_window(Sketch& sk, const int64_t* rowptr, const int32_t* col, const double* val, int64_t row0,
-                       int64_t rows);
+                       int64_t rows, int64_t nnz);
 // again: a later window of one linear_update (what an earlier one derived from
 // the points, in the sketch's scratch, still holds).
 void update_rbf_window(Sketch& sk, const double* points, int64_t ldp, int64_t row0, int64_t rows, bool again = false);

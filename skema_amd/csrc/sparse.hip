@@ -2,6 +2,7 @@
 // Bandwidth-bound gathers: consecutive lanes own consecutive output rows of a
 // column-major result, so stores and the dense-operand loads coalesce, and
 // no two threads ever accumulate into the same element.
+#include <algorithm>
 #include <vector>
 
 #include "sparse.hpp"
@@ -88,16 +89,23 @@ __global__ void k_spmm_dense_csrT(int64_t M, const double* B, int64_t ldb, const
 }
 
 // ---- CSR window -> CSC ----------------------------------------------------
-// flag bit 0: rowptr decreasing, bit 1: column index outside [0, cols).
-__global__ void k_validate_csr(const int64_t* rowptr, int64_t rows, const int32_t* col, int64_t cols, int* flag) {
-  const int64_t base = rowptr[0];
-  const int64_t nnz = rowptr[rows] - base;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < rows; i += (int64_t)gridDim.x * blockDim.x)
-    if (rowptr[i + 1] < rowptr[i]) atomicOr(flag, 1);
-  for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < nnz; e += (int64_t)gridDim.x * blockDim.x) {
-    const int32_t c = col[base + e];
-    if (c < 0 || c >= cols) atomicOr(flag, 2);
+__global__ void k_inspect_csr(const int64_t* rowptr, int64_t rows, const int32_t* col, int64_t cols, int64_t room,
+                              int64_t* out) {
+  const int64_t base = rowptr[0], end = rowptr[rows];
+  const int64_t i0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, step = (int64_t)gridDim.x * blockDim.x;
+  if (i0 == 0) {
+    out[0] = base;
+    out[1] = end;
   }
+  unsigned long long bad = 0;
+  for (int64_t i = i0; i < rows; i += step)
+    if (rowptr[i + 1] < rowptr[i]) bad |= 1;
+  if (base >= 0 && end >= base && end <= room && end - base < ((int64_t)1 << 31))
+    for (int64_t e = base + i0; e < end; e += step) {
+      const int32_t c = col[e];
+      if (c < 0 || c >= cols) bad |= 2;
+    }
+  if (bad) atomicOr(reinterpret_cast<unsigned long long*>(out + 2), bad);
 }
 
 __global__ void k_count_cols(const int64_t* rowptr, int64_t rows, const int32_t* col, int* counts) {
@@ -302,16 +310,59 @@ __global__ __launch_bounds__(64) void k_sort_columns(const int64_t* ptr, int32_t
   }
 }
 
-__global__ void k_csc_left_dense(const int64_t* ptr, const int32_t* row, const double* val, int64_t cols,
-                                 const double* M, int64_t ldm, int64_t row0, int64_t k, double eta, double nu,
-                                 double* X, int64_t ldx) {
-  const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (g >= k * cols) return;
-  const int64_t p = g % k, j = g / k;
-  double acc = 0.0;
-  for (int64_t e = ptr[j]; e < ptr[j + 1]; ++e) acc += val[e] * M[p + (row0 + row[e]) * ldm];
-  double* x = X + p + j * ldx;
-  *x = (nu != 0.0) ? nu * *x + eta * acc : eta * acc;
+// X(p, j) = nu X + eta sum over column j's entries (i, a) of a M(p, row0 + i): one
+// wave per column and 64 PR rows p, the entries in order, four of them (and their
+// map columns) in flight at a time.  With cw, a is weighted by cw[i / window].
+template <int PR, bool CW>
+__global__ __launch_bounds__(256) void k_csc_left_dense(const int64_t* __restrict__ ptr, const int32_t* __restrict__ row,
+                                                        const double* __restrict__ val, int64_t cols,
+                                                        const double* __restrict__ M, int64_t ldm, int64_t row0,
+                                                        int64_t k, const double* __restrict__ cw, uint32_t window,
+                                                        double eta, double nu, double* __restrict__ X, int64_t ldx) {
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t j = (int64_t)blockIdx.x * 4 + wave, p0 = (int64_t)blockIdx.y * (64 * PR);
+  if (j >= cols) return;
+  const int64_t lo = ptr[j], hi = ptr[j + 1];
+  int64_t at[PR];  // this lane's rows (past k: the last one's, not stored)
+#pragma unroll
+  for (int r = 0; r < PR; ++r) at[r] = p0 + lane + 64 * r < k ? p0 + lane + 64 * r : k - 1;
+  double acc[PR];
+#pragma unroll
+  for (int r = 0; r < PR; ++r) acc[r] = 0.0;
+  auto term = [&](int64_t e, const double*& m) {
+    const int32_t i = row[e];
+    m = M + (row0 + i) * ldm;
+    return CW ? val[e] * cw[(uint32_t)i / window] : val[e];
+  };
+  int64_t e = lo;
+  for (; e + 4 <= hi; e += 4) {
+    const double* m[4];
+    double a[4], v[4][PR];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) a[q] = term(e + q, m[q]);
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int r = 0; r < PR; ++r) v[q][r] = m[q][at[r]];
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int r = 0; r < PR; ++r) acc[r] += a[q] * v[q][r];
+  }
+  for (; e < hi; ++e) {
+    const double* m;
+    const double a = term(e, m);
+#pragma unroll
+    for (int r = 0; r < PR; ++r) acc[r] += a * m[at[r]];
+  }
+#pragma unroll
+  for (int r = 0; r < PR; ++r) {
+    const int64_t p = p0 + lane + 64 * r;
+    if (p < k) {
+      double* x = X + p + j * ldx;
+      *x = (nu != 0.0) ? nu * *x + eta * acc[r] : eta * acc[r];
+    }
+  }
 }
 
 __global__ void k_csc_left_sparse(const int64_t* ptr, const int32_t* row, const double* val, int64_t cols,
@@ -329,14 +380,62 @@ __global__ void k_csc_left_sparse(const int64_t* ptr, const int32_t* row, const 
   }
 }
 
-__global__ void k_csr_right_dense(const int64_t* rowptr, const int32_t* col, const double* val, int64_t rows,
-                                  const double* M, int64_t ldm, int64_t kk, GemmOut o) {
-  const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (g >= kk * rows) return;
-  const int64_t p = g % kk, i = g / kk;
-  double acc = 0.0;
-  for (int64_t e = rowptr[i]; e < rowptr[i + 1]; ++e) acc += val[e] * M[p + (int64_t)col[e] * ldm];
-  put(o, i, p, acc);
+// out(i, p) = sum over row i's entries (j, a) of a M(p, j): 16 rows and 64 PR
+// map rows p a block, each wave four rows one after another (entries in order,
+// four and their map columns in flight), then through LDS so that a column of
+// the output is written 16 rows (128 bytes) at a time.  One thread per output
+// with p fastest wrote every 8 bytes to a line of its own: 4096 x 304 outputs
+// with 15 entries a row took 48 us, 24 here.
+constexpr int kRightTile = 16;
+template <int PR>
+__global__ __launch_bounds__(256) void k_csr_right_dense(const int64_t* __restrict__ rowptr, const int32_t* __restrict__ col,
+                                                         const double* __restrict__ val, int64_t rows,
+                                                         const double* __restrict__ M, int64_t ldm, int64_t kk, GemmOut o) {
+  __shared__ double tile[64 * PR][kRightTile + 1];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int64_t r0 = (int64_t)blockIdx.x * kRightTile, p0 = (int64_t)blockIdx.y * (64 * PR);
+  int64_t at[PR];
+#pragma unroll
+  for (int r = 0; r < PR; ++r) at[r] = p0 + lane + 64 * r < kk ? p0 + lane + 64 * r : kk - 1;
+  for (int q = 0; q < kRightTile / 4; ++q) {
+    const int64_t i = r0 + 4 * q + wave;
+    if (i >= rows) break;
+    const int64_t lo = rowptr[i], hi = rowptr[i + 1];
+    double acc[PR];
+#pragma unroll
+    for (int r = 0; r < PR; ++r) acc[r] = 0.0;
+    int64_t e = lo;
+    for (; e + 4 <= hi; e += 4) {
+      const double* m[4];
+      double a[4], v[4][PR];
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        a[t] = val[e + t];
+        m[t] = M + (int64_t)col[e + t] * ldm;
+      }
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int r = 0; r < PR; ++r) v[t][r] = m[t][at[r]];
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int r = 0; r < PR; ++r) acc[r] += a[t] * v[t][r];
+    }
+    for (; e < hi; ++e) {
+      const double a = val[e];
+      const double* m = M + (int64_t)col[e] * ldm;
+#pragma unroll
+      for (int r = 0; r < PR; ++r) acc[r] += a * m[at[r]];
+    }
+#pragma unroll
+    for (int r = 0; r < PR; ++r) tile[lane + 64 * r][4 * q + wave] = acc[r];
+  }
+  __syncthreads();
+  for (int x = tid; x < 64 * PR * kRightTile; x += 256) {
+    const int ii = x % kRightTile, pp = x / kRightTile;
+    if (r0 + ii < rows && p0 + pp < kk) put(o, r0 + ii, p0 + pp, tile[pp][ii]);
+  }
 }
 
 __global__ void k_csr_right_sparse(const int64_t* rowptr, const int32_t* col, const double* val, int64_t rows,
@@ -413,50 +512,42 @@ void spmm_dense_csrT(hipStream_t st, int64_t M, const double* B, int64_t ldb, co
   check_launch("k_spmm_dense_csrT");
 }
 
-int64_t validate_csr_window(hipStream_t st, const int64_t* rowptr, const int32_t* col, int64_t rows, int64_t cols,
-                            int* flag, const int64_t* known) {
-  int64_t ends[2] = {0, 0};
-  if (known) {
-    ends[0] = known[0];
-    ends[1] = known[1];
-  } else {
-    SKEMA_HIP(hipMemcpyAsync(&ends[0], rowptr, sizeof(int64_t), hipMemcpyDeviceToHost, st));
-    SKEMA_HIP(hipMemcpyAsync(&ends[1], rowptr + rows, sizeof(int64_t), hipMemcpyDeviceToHost, st));
-    SKEMA_HIP(hipStreamSynchronize(st));
+CsrInfo inspect_csr(Ctx* c, const int64_t* rowptr, const int32_t* col, int64_t rows, int64_t cols, int64_t room) {
+  hipStream_t st = c->stream;
+  constexpr size_t kBytes = 3 * sizeof(int64_t);
+  if (!c->csr_dev.p) {
+    c->csr_dev.alloc(kBytes);
+    fill_i32(st, c->csr_dev.as<int>(), kBytes / sizeof(int), 0);
   }
-  const int64_t nnz = ends[1] - ends[0];
-  SKEMA_REQUIRE(nnz >= 0 && nnz < ((int64_t)1 << 31), kErrArg, "CSR window: bad rowptr range");
-  // Reject malformed windows before any kernel indexes with them.
-  fill_i32(st, flag, 1, 0);
-  const int64_t work = nnz > rows ? nnz : rows;
-  const unsigned nb = blocks_for(work) > 65536 ? 65536 : blocks_for(work);
-  hipLaunchKernelGGL(k_validate_csr, dim3(nb), dim3(256), 0, st, rowptr, rows, col, cols, flag);
-  check_launch("k_validate_csr");
-  int h = 0;
-  SKEMA_HIP(hipMemcpyAsync(&h, flag, sizeof(int), hipMemcpyDeviceToHost, st));
+  if (!c->csr_host.p) SKEMA_HIP(hipHostMalloc(&c->csr_host.p, kBytes, hipHostMallocDefault));
+  int64_t* dev = c->csr_dev.as<int64_t>();
+  const int64_t work = std::max(rows, room);
+  const unsigned nb = (unsigned)std::max<int64_t>(1, std::min<int64_t>(cdiv(work, 256), 2048));
+  hipLaunchKernelGGL(k_inspect_csr, dim3(nb), dim3(256), 0, st, rowptr, rows, col, cols, room, dev);
+  check_launch("k_inspect_csr");
+  SKEMA_HIP(hipMemcpyAsync(c->csr_host.p, dev, kBytes, hipMemcpyDeviceToHost, st));
   SKEMA_HIP(hipStreamSynchronize(st));
-  SKEMA_REQUIRE(!(h & 1), kErrArg, "CSR window: rowptr is not non-decreasing");
-  SKEMA_REQUIRE(!(h & 2), kErrArg, "CSR window: column index outside [0, n)");
-  return nnz;
+  const int64_t* h = static_cast<const int64_t*>(c->csr_host.p);
+  const CsrInfo info{h[0], h[1], h[2]};
+  if (info.flags) fill_i32(st, reinterpret_cast<int*>(dev + 2), 2, 0);
+  return info;
 }
 
 CscWindow csr_window_to_csc(hipStream_t st, const int64_t* rowptr, const int32_t* col, const double* val,
-                            int64_t rows, int64_t cols, DevBuf& scratch, bool sorted) {
-  int64_t nnz = 0;
-  {
-    DevBuf flag(sizeof(int));
-    nnz = validate_csr_window(st, rowptr, col, rows, cols, flag.as<int>());
-  }
+                            int64_t rows, int64_t cols, int64_t nnz, DevBuf& scratch, bool sorted) {
   const size_t o_cnt = 0;
   const size_t o_ptr = align_up((size_t)cols * sizeof(int) * 2, 256);
   const size_t o_row = o_ptr + align_up((size_t)(cols + 1) * sizeof(int64_t), 256);
   const size_t o_val = o_row + align_up((size_t)nnz * sizeof(int32_t), 256);
-  // Row-blocked counts and placement in LDS when the columns fit (512 row
-  // blocks; no global atomics); global atomic counters otherwise.
-  const int64_t nbk = 512, R = cdiv(rows, nbk);
+  // Row-blocked counts and placement in LDS when the columns fit (no global
+  // atomics; one block per about 2048 nonzeros, 16 to 512 of them: the scan of
+  // the blocks' counts reads cols ints a block, 35 us for 512 blocks of 3001
+  // columns, 4 us for the 30 that 61000 nonzeros take); global atomic counters
+  // otherwise.
+  const int64_t nbk = std::max<int64_t>(16, std::min<int64_t>(512, cdiv(nnz, (int64_t)2048))), R = cdiv(rows, nbk);
   // (the fill keeps cols cursors and the R + 1 row starts of its slice in LDS)
   const bool blocked =
-      cols <= kHistCols && rows >= 4096 && nnz > 0 && (size_t)(cols + R + 1) * sizeof(int) <= 160 * 1024;
+      cols <= kHistCols && rows >= 256 && nnz > 0 && (size_t)(cols + R + 1) * sizeof(int) <= 160 * 1024;
   const size_t o_T = o_val + align_up((size_t)nnz * sizeof(double), 256);
   const size_t total = o_T + (blocked ? align_up((size_t)nbk * cols * sizeof(int), 256) : 0);
   scratch.reserve(total);
@@ -497,10 +588,23 @@ CscWindow csr_window_to_csc(hipStream_t st, const int64_t* rowptr, const int32_t
 }
 
 void csc_left_dense(hipStream_t st, const CscWindow& H, const double* M, int64_t ldm, int64_t row0, int64_t k,
-                    double eta, double nu, double* X, int64_t ldx) {
+                    double eta, double nu, double* X, int64_t ldx, const double* cw, int64_t window) {
   if (k == 0 || H.cols == 0) return;
-  hipLaunchKernelGGL(k_csc_left_dense, dim3(blocks_for(k * H.cols)), dim3(256), 0, st, H.ptr, H.row, H.val, H.cols,
-                     M, ldm, row0, k, eta, nu, X, ldx);
+  const int pr = k <= 128 ? 2 : k <= 256 ? 4 : 8;  // map rows per lane
+  const dim3 grid(blocks_for(H.cols, 4), (unsigned)cdiv(k, (int64_t)64 * pr));
+#define SKEMA_LEFT(PR, CW)                                                                                            \
+  hipLaunchKernelGGL((k_csc_left_dense<PR, CW>), grid, dim3(256), 0, st, H.ptr, H.row, H.val, H.cols, M, ldm, row0, k, \
+                     cw, (uint32_t)window, eta, nu, X, ldx)
+  if (cw) {
+    if (pr == 2) SKEMA_LEFT(2, true);
+    else if (pr == 4) SKEMA_LEFT(4, true);
+    else SKEMA_LEFT(8, true);
+  } else {
+    if (pr == 2) SKEMA_LEFT(2, false);
+    else if (pr == 4) SKEMA_LEFT(4, false);
+    else SKEMA_LEFT(8, false);
+  }
+#undef SKEMA_LEFT
   check_launch("k_csc_left_dense");
 }
 
@@ -515,8 +619,16 @@ void csc_left_sparse(hipStream_t st, const CscWindow& H, const Csr& Mt, int64_t 
 void csr_right_dense(hipStream_t st, const int64_t* rowptr, const int32_t* col, const double* val, int64_t rows,
                      const double* M, int64_t ldm, int64_t kk, const GemmOut& out) {
   if (rows == 0 || kk == 0) return;
-  hipLaunchKernelGGL(k_csr_right_dense, dim3(blocks_for(kk * rows)), dim3(256), 0, st, rowptr, col, val, rows, M,
-                     ldm, kk, out);
+  const int pr = (int)std::min<int64_t>(5, cdiv(kk, (int64_t)64));  // 5: the 304 rows of a rank-25 [Omega; Psi]
+  const dim3 grid(blocks_for(rows, kRightTile), (unsigned)cdiv(kk, (int64_t)64 * pr));
+#define SKEMA_RIGHT(PR) \
+  hipLaunchKernelGGL(k_csr_right_dense<PR>, grid, dim3(256), 0, st, rowptr, col, val, rows, M, ldm, kk, out)
+  if (pr == 1) SKEMA_RIGHT(1);
+  else if (pr == 2) SKEMA_RIGHT(2);
+  else if (pr == 3) SKEMA_RIGHT(3);
+  else if (pr == 4) SKEMA_RIGHT(4);
+  else SKEMA_RIGHT(5);
+#undef SKEMA_RIGHT
   check_launch("k_csr_right_dense");
 }
 

@@ -19,12 +19,15 @@ void spmm_csr_rows(hipStream_t st, const Csr& S, int64_t r0, int64_t r1, int64_t
 void spmm_dense_csrT(hipStream_t st, int64_t M, const double* B, int64_t ldb, const Csr& S, const GemmOut& out,
                      DevBuf* ws = nullptr);
 
-// Checks a device CSR window (rowptr non-decreasing, column indices in
-// [0, cols)) and returns its nonzero count; flag is one device int of
-// scratch; ends (optional): rowptr[0] and rowptr[rows] already read on the
-// host.  Throws on a malformed window before any kernel indexes with it.
-int64_t validate_csr_window(hipStream_t st, const int64_t* rowptr, const int32_t* col, int64_t rows, int64_t cols,
-                            int* flag, const int64_t* ends = nullptr);
+// What a device CSR window holds, in one launch and one small copy back:
+// rowptr[0] and rowptr[rows], and flags (1: rowptr decreases somewhere, 2: a
+// column index outside [0, cols)).  Column indices are read only where the ends
+// lie in order within [0, room], room the entries that col's and val's
+// allocations hold, and below 2^31 of them.
+struct CsrInfo {
+  int64_t first = 0, last = 0, flags = 0;
+};
+CsrInfo inspect_csr(Ctx* c, const int64_t* rowptr, const int32_t* col, int64_t rows, int64_t cols, int64_t room);
 
 // Column-compressed copy of a CSR window (rowptr may start at an offset).
 struct CscWindow {
@@ -35,14 +38,15 @@ struct CscWindow {
 };
 // sorted: rows ascending within each column (a deterministic summation
 // order for the kernels that walk a column in order); callers that only
-// accumulate with atomics pass false.
+// accumulate with atomics pass false.  The window has been inspected (nnz).
 CscWindow csr_window_to_csc(hipStream_t st, const int64_t* rowptr, const int32_t* col, const double* val,
-                            int64_t rows, int64_t cols, DevBuf& scratch, bool sorted = true);
+                            int64_t rows, int64_t cols, int64_t nnz, DevBuf& scratch, bool sorted = true);
 
 // X[p,j] = nu*X[p,j] + eta * sum_{(i,a) in column j of H} a * M[p, row0+i]
 // with M a dense k x * logical map (ldm).
+// cw: when not null, a is weighted by cw[i / window] first.
 void csc_left_dense(hipStream_t st, const CscWindow& H, const double* M, int64_t ldm, int64_t row0, int64_t k,
-                    double eta, double nu, double* X, int64_t ldx);
+                    double eta, double nu, double* X, int64_t ldx, const double* cw = nullptr, int64_t window = 1);
 // Same with a sparse logical map given as the CSR of its transpose (row
 // c of Mt = column c of the map).
 void csc_left_sparse(hipStream_t st, const CscWindow& H, const Csr& Mt, int64_t row0, int64_t k, double eta,

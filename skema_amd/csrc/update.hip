@@ -183,7 +183,7 @@ void update_dense_window(Sketch& sk, const double* H, int64_t ldh, int64_t row0,
 }
 
 void update_csr_window(Sketch& sk, const int64_t* rowptr, const int32_t* col, const double* val, int64_t row0,
-                       int64_t rows) {
+                       int64_t rows, int64_t nnz) {
   Ctx* c = sk.ctx;
   hipStream_t st = c->stream;
   const int64_t k = sk.k, s = sk.s, m = sk.p.m, n = sk.p.n;
@@ -206,7 +206,7 @@ void update_csr_window(Sketch& sk, const int64_t* rowptr, const int32_t* col, co
   CscWindow Hc;
   {
     Timed t(c, "window");
-    Hc = csr_window_to_csc(st, rowptr, col, val, rows, n, sk.win);
+    Hc = csr_window_to_csc(st, rowptr, col, val, rows, n, nnz, sk.win);
   }
   if (sk.sparse_maps) {
     {
