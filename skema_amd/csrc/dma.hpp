@@ -86,6 +86,21 @@ __device__ __forceinline__ void wait_vm_upto(int n) {
   }
 }
 
+// The copy through a buffer resource instead: lane l fetches 16 (4) bytes at
+// base + off, base the same in the whole wave and off its own.  The address
+// is a scalar base with a 32-bit lane offset, and, no flat instruction, it
+// leaves the compiler free to wait for LDS reads one by one: with
+// global_load_lds in flight it waits for all of them at every use.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t wave_buffer(const void* base) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, -1, 0x00020000);  // raw, 32-bit data format
+}
+__device__ __forceinline__ void copy16_to_lds(const void* base, uint32_t off, void* lds) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(wave_buffer(base), (SKEMA_LDS void*)lds, 16, (int)off, 0, 0, 0);
+}
+__device__ __forceinline__ void copy4_to_lds(const void* base, uint32_t off, void* lds) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(wave_buffer(base), (SKEMA_LDS void*)lds, 4, (int)off, 0, 0, 0);
+}
+
 // Barrier that orders this wave's LDS accesses around it in the compiler's
 // view (memory clobber) without the fence of __syncthreads, which would wait
 // for every copy in flight.

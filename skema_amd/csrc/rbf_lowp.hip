@@ -260,14 +260,21 @@ __global__ __launch_bounds__(kThreadsR) void k_rbf_right_bf16(RbfLpArgs g) {
 // exactly points 8 (l/16) .. +7 of row l%16 after the two sub-tiles: the
 // A-operand layout of the sketch MFMA, in natural point order.  The
 // [Omega; Psi] slice (208 x 32 points, 64-byte rows), the step's points
-// (32 x DP) and their norms stream global -> LDS through global_load_lds
-// into a kRingSlots-slot ring, so four steps of loads are in flight while
-// one is consumed; one barrier per step.  16-byte chunks are XOR-swizzled
+// (32 x DP) and their norms stream global -> LDS (copy16_to_lds) into a
+// kRingSlots-slot ring, so four steps of loads are in flight while one is
+// consumed; one barrier per step.  16-byte chunks are XOR-swizzled
 // within rows so the 16 rows a lane group reads at one chunk hit distinct
 // banks.
-// kTallXT 16-row tiles per wave: 4 (one wave per SIMD, accumulators in
-// AGPRs) halves the LDS reads of the [Omega; Psi] operands per MFMA against 2.
-constexpr int kTallRows = 256, kTallCols = 208, kRingSlots = 6, kTallXT = 4;
+// kTallXT 16-row tiles per wave.  A step is a chain (LDS reads, Gram,
+// exponentials, sketch) in which a wave alone on its SIMD leaves the matrix
+// cores idle three cycles in four: with 4 tiles a wave (4 waves) 5000 cycles
+// a step for 1345 of MFMA.  2 tiles (8 waves, two a SIMD, LDS reads doubled)
+// overlap one wave's exponentials with the other's MFMAs.  A window of 2048
+// rows of 100000 points in d = 128, k + s = 604: 666 us with 4 tiles, 516
+// with 2, 486 with LDS reads two tiles ahead and waited for one by one (no
+// flat copies), 455 with the slot offsets, step counts and waits kept scalar
+// and simple.  Reading the Gram's operands before the barrier spills (573).
+constexpr int kTallRows = 256, kTallCols = 208, kRingSlots = 6, kTallXT = 2;
 
 // chunk-position swizzle of a points row with CPR 16-byte chunks, for the
 // rows 8a + 4h + t (a, t < 4) of either sub-tile
@@ -285,7 +292,7 @@ __device__ __forceinline__ int os_swz(int r) { return (r >> 2) & 3; }
 // log2(e): u <= 0 exactly when D >= 0.
 __device__ __forceinline__ float rbf_exp2(float g, float ab, float kappa) {
   const float u = fmaf(g, kappa, ab);
-  return __builtin_amdgcn_exp2f(u < 0.f ? u : 0.f);
+  return __builtin_amdgcn_exp2f(fminf(u, 0.f));
 }
 
 template <int DP>
@@ -333,61 +340,55 @@ __global__ __launch_bounds__(64 * (kTallRows / (16 * kTallXT)), 1) void k_rbf_ri
     al[x] = (i < g.M) ? -lg * g.nrm[g.row0 + i] : 0.f;
   }
 
-  // Per-lane sources of the wave's copies at the first step; a step moves
-  // each by BK points (2 BK bytes along an [Omega; Psi] row, BK points rows,
-  // 4 BK bytes of norms).  Near the end of the split the points rows and
+  // The wave's copies: a scalar base that moves by BK points a step (2 BK
+  // bytes along an [Omega; Psi] row, BK points rows, 4 BK bytes of norms) and
+  // a lane offset that stays.  Near the end of the split the points rows and
   // norms are clamped to the last point instead.
-  const char* dsrc[IPW];
+  uint32_t doff[IPW];
 #pragma unroll
   for (int s = 0; s < IPW; ++s) {
     const int it = wave + NW * s;
     if (it < I_OS) {  // 16 rows of the [Omega; Psi] slice
       const int r = 16 * it + (lane >> 2), p = lane & 3;
-      int64_t col = c0 + r;
-      col = col < g.N ? col : g.N - 1;
-      dsrc[s] = reinterpret_cast<const char*>(g.OP + col * g.ldop + kbeg + 8 * (p ^ os_swz(r)));
+      const int64_t cb = c0 + 16 * it < g.N ? c0 + 16 * it : g.N - 1, col = c0 + r < g.N ? c0 + r : g.N - 1;
+      doff[s] = (uint32_t)(2 * ((col - cb) * g.ldop + 8 * (p ^ os_swz(r))));
     } else if (it < I_OS + I_XS) {  // RPI points rows
-      const int x = it - I_OS;
-      const int r = RPI * x + lane / CPR, p = lane % CPR;
-      dsrc[s] = reinterpret_cast<const char*>(g.P + (kbeg + r) * g.ldpb + 8 * (p ^ xs_swz<CPR>(r)));
+      const int r = RPI * (it - I_OS) + lane / CPR, p = lane % CPR;
+      doff[s] = (uint32_t)(2 * (r * DP + 8 * (p ^ xs_swz<CPR>(r))));
     } else {  // norms of the step's points (lanes >= 32 duplicate, unused)
-      dsrc[s] = reinterpret_cast<const char*>(g.nrm + kbeg + (lane & 31));
+      doff[s] = 4 * (lane & 31);
     }
   }
-  auto issue = [&](int u) {
-    uint8_t* slot = ring + (u % NS) * SLOT;
-    const bool tail = kbeg + (int64_t)(u + 1) * BK > kend;
+  auto issue = [&](int u, int at) {  // at: the step's slot, in bytes
+    uint8_t* slot = ring + at;
+    const int64_t j0 = kbeg + (int64_t)u * BK;
+    const bool tail = j0 + BK > kend;
+    const int last = (int)(kend - j0) - 1;  // the step's last point
 #pragma unroll
     for (int s = 0; s < IPW; ++s) {
       const int it = wave + NW * s;
       if (it < I_OS) {
-        __builtin_amdgcn_global_load_lds((const void*)(dsrc[s] + (int64_t)u * (2 * BK)),
-                                         (SKEMA_LDS void*)(slot + 1024 * it), 16, 0, 0);
+        const int64_t cb = c0 + 16 * it < g.N ? c0 + 16 * it : g.N - 1;
+        copy16_to_lds(g.OP + cb * g.ldop + j0, doff[s], slot + 1024 * it);
       } else if (it < I_OS + I_XS) {
         const int x = it - I_OS;
-        const char* src = dsrc[s] + (int64_t)u * BK * (2 * DP);
+        uint32_t off = doff[s];
         if (tail) {
           const int r = RPI * x + lane / CPR, p = lane % CPR;
-          int64_t j = kbeg + (int64_t)u * BK + r;
-          j = j < kend ? j : kend - 1;
-          src = reinterpret_cast<const char*>(g.P + j * g.ldpb + 8 * (p ^ xs_swz<CPR>(r)));
+          off = (uint32_t)(2 * ((r < last ? r : last) * DP + 8 * (p ^ xs_swz<CPR>(r))));
         }
-        __builtin_amdgcn_global_load_lds((const void*)src, (SKEMA_LDS void*)(slot + OS_BYTES + 1024 * x), 16, 0, 0);
+        copy16_to_lds(g.P + j0 * DP, off, slot + OS_BYTES + 1024 * x);
       } else if (it == I_OS + I_XS) {
-        const char* src = dsrc[s] + (int64_t)u * (4 * BK);
-        if (tail) {
-          int64_t j = kbeg + (int64_t)u * BK + (lane & 31);
-          j = j < kend ? j : kend - 1;
-          src = reinterpret_cast<const char*>(g.nrm + j);
-        }
-        __builtin_amdgcn_global_load_lds((const void*)src, (SKEMA_LDS void*)(slot + NJ_OFF), 4, 0, 0);
+        uint32_t off = doff[s];
+        if (tail) off = 4 * ((lane & 31) < last ? (lane & 31) : last);
+        copy4_to_lds(g.nrm + j0, off, slot + NJ_OFF);
       }
     }
   };
 
   // Gram tiles of step u (transposed: points x the wave's window rows)
-  auto gram = [&](int u, f4v (&gr)[2][XT]) {
-    const uint8_t* xs = ring + (u % NS) * SLOT + OS_BYTES;
+  auto gram = [&](int at, f4v (&gr)[2][XT]) {
+    const uint8_t* xs = ring + at + OS_BYTES;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       const int r = 8 * (l16 >> 2) + 4 * h + (l16 & 3);  // points row read by this lane
@@ -405,8 +406,8 @@ __global__ __launch_bounds__(64 * (kTallRows / (16 * kTallXT)), 1) void k_rbf_ri
   // K of step u from its Gram tiles, in registers (A operands of the
   // sketch), without checks: interior steps (every row and point in range,
   // the window's diagonal not among them)
-  auto exp_fast = [&](int u, const f4v (&gr)[2][XT], bf16x8 (&kv)[XT]) {
-    const float* nj = reinterpret_cast<const float*>(ring + (u % NS) * SLOT + NJ_OFF);
+  auto exp_fast = [&](int at, const f4v (&gr)[2][XT], bf16x8 (&kv)[XT]) {
+    const float* nj = reinterpret_cast<const float*>(ring + at + NJ_OFF);
     f4v be[2];
     be[0] = *reinterpret_cast<const f4v*>(nj + 8 * lq);
     be[1] = *reinterpret_cast<const f4v*>(nj + 8 * lq + 4);
@@ -417,13 +418,15 @@ __global__ __launch_bounds__(64 * (kTallRows / (16 * kTallXT)), 1) void k_rbf_ri
 #pragma unroll
         for (int v = 0; v < 4; ++v) kv[x][4 * h + v] = (__bf16)rbf_exp2(gr[h][x][v], al[x] - lg * be[h][v], kappa);
   };
-  auto interior = [&](int u) {
-    const int64_t j0 = kbeg + (int64_t)u * BK, gi0 = g.row0 + wr0;
-    return rows_full && j0 + BK <= kend && (j0 + BK <= gi0 || j0 >= gi0 + 16 * XT);
-  };
+  // interior steps: every point in range and none of the wave's own rows
+  // among them (the diagonal lies in steps dlo .. dhi - 1)
+  const int64_t dg = g.row0 + wr0 - kbeg;
+  const int full = rows_full ? (int)((kend - kbeg) / BK) : 0;
+  const int dlo = dg > 0 ? (int)(dg / BK) : 0, dhi = dg + 16 * XT > 0 ? (int)((dg + 16 * XT + BK - 1) / BK) : 0;
+  auto interior = [&](int u) { return u < full && (u < dlo || u >= dhi); };
   // the same with the range and diagonal checks
-  auto exp_edge = [&](int u, const f4v (&gr)[2][XT], bf16x8 (&kv)[XT]) {
-    const float* nj = reinterpret_cast<const float*>(ring + (u % NS) * SLOT + NJ_OFF);
+  auto exp_edge = [&](int u, int at, const f4v (&gr)[2][XT], bf16x8 (&kv)[XT]) {
+    const float* nj = reinterpret_cast<const float*>(ring + at + NJ_OFF);
     const int64_t j0 = kbeg + (int64_t)u * BK;
 #pragma unroll
     for (int x = 0; x < XT; ++x) {
@@ -450,43 +453,46 @@ __global__ __launch_bounds__(64 * (kTallRows / (16 * kTallXT)), 1) void k_rbf_ri
   bf16x8 kv[XT];
 #pragma unroll
   for (int p = 0; p < NS - 1; ++p)
-    if (p < steps) issue(p);
+    if (p < steps) issue(p, p * SLOT);
   if (steps > 0) {
     wait_vm_upto(((NS - 2) < (steps - 1) ? (NS - 2) : (steps - 1)) * dw);  // step 0 complete
     lds_barrier();
     f4v gr[2][XT];
     gram(0, gr);
     if (interior(0)) exp_fast(0, gr, kv);
-    else exp_edge(0, gr, kv);
+    else exp_edge(0, 0, gr, kv);
   }
-  for (int u = 0; u < steps; ++u) {
-    if (u + 1 < steps) {  // step u + 1 complete: at most steps u+2 .. min(u+NS-2, steps-1) in flight
-      const int last = (u + NS - 2 < steps - 1) ? u + NS - 2 : steps - 1;
-      wait_vm_upto((last - (u + 1)) * dw);
+  for (int u = 0, at = 0, atn = SLOT, fill = (NS - 1) * SLOT; u < steps; ++u) {  // slots of u, u + 1, u + NS - 1
+    if (u + NS - 1 <= steps) {  // step u + 1 complete: steps u+2 .. u+NS-2 in flight
+      if (dw == IPW) wait_vm<(NS - 3) * IPW>();
+      else wait_vm<(NS - 3) * (IPW - 1)>();
+    } else if (u + 1 < steps) {  // steps u+2 .. steps-1
+      wait_vm_upto((steps - 2 - u) * dw);
     }
     lds_barrier();  // every wave's copies of step u+1 landed; slot (u-1) % NS is free
-    if (u + NS - 1 < steps) issue(u + NS - 1);
-    const int un = (u + 1 < steps) ? u + 1 : u;  // the last step forms a Gram it does not use
+    if (u + NS - 1 < steps) issue(u + NS - 1, fill);
+    const int un = u + 1;  // past the last step: a Gram of the slot's older contents, not used
     f4v gr[2][XT];
-    gram(un, gr);
+    gram(atn, gr);
     // the sketch MFMAs of step u, column tile by column tile, each followed
     // by a share of the exponentials of step u+1 (which need only the Gram
     // above): the matrix cores run one tile while the VALU forms the next
     // K values (sched_barrier keeps the compiler from regrouping them)
-    const uint8_t* os = ring + (u % NS) * SLOT;
-    const float* nj = reinterpret_cast<const float*>(ring + (un % NS) * SLOT + NJ_OFF);
+    const uint8_t* os = ring + at;
+    const float* nj = reinterpret_cast<const float*>(ring + atn + NJ_OFF);
     f4v be[2];
     be[0] = *reinterpret_cast<const f4v*>(nj + 8 * lq);
     be[1] = *reinterpret_cast<const f4v*>(nj + 8 * lq + 4);
     bf16x8 kn[XT];
-    bf16x8 o = *reinterpret_cast<const bf16x8*>(os + 64 * l16 + 16 * (lq ^ os_swz(l16)));
+    auto op_at = [&](int y) {
+      const int r = 16 * y + l16;
+      return *reinterpret_cast<const bf16x8*>(os + 64 * r + 16 * (lq ^ os_swz(r)));
+    };
+    bf16x8 o = op_at(0), o1 = op_at(1);  // read two column tiles ahead
 #pragma unroll
     for (int y = 0; y < TNC; ++y) {
-      bf16x8 on = o;
-      if (y + 1 < TNC) {
-        const int r = 16 * (y + 1) + l16;
-        on = *reinterpret_cast<const bf16x8*>(os + 64 * r + 16 * (lq ^ os_swz(r)));
-      }
+      bf16x8 o2 = o1;
+      if (y + 2 < TNC) o2 = op_at(y + 2);
 #pragma unroll
       for (int x = 0; x < XT; ++x) acc[x][y] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kv[x], o, acc[x][y], 0, 0, 0);
       // K values e in [32 y / TNC, 32 (y + 1) / TNC) of this lane's 32 (x, h, v)
@@ -498,11 +504,15 @@ __global__ __launch_bounds__(64 * (kTallRows / (16 * kTallXT)), 1) void k_rbf_ri
         kn[x][4 * h + v] = (__bf16)k;
       }
       __builtin_amdgcn_sched_barrier(0);
-      o = on;
+      o = o1;
+      o1 = o2;
     }
-    if (!interior(un)) exp_edge(un, gr, kn);
+    if (!interior(un) && un < steps) exp_edge(un, atn, gr, kn);
 #pragma unroll
     for (int x = 0; x < XT; ++x) kv[x] = kn[x];
+    fill = at;
+    at = atn;
+    atn = atn + SLOT == NS * SLOT ? 0 : atn + SLOT;
   }
 #pragma unroll
   for (int x = 0; x < XT; ++x)
@@ -541,10 +551,13 @@ __global__ __launch_bounds__(64 * (kTallRows / (16 * kTallXT)), 1) void k_rbf_ri
 // the sketch MFMA in natural row order, matched by one 16-byte read of the
 // Upsilon slice.  The step's window rows (32 x DP), their norms and the
 // Upsilon slice (16 TP rows x 32 window rows, 64-byte rows) stream global ->
-// LDS through global_load_lds into a kRingSlots-slot ring shared by all
-// waves, one barrier per step.  Needs row0 a multiple of 8 (16-byte aligned
-// slices).
-constexpr int kLeftRingWaves = 4, kLeftJT = 4;
+// LDS (copy16_to_lds) into a kRingSlots-slot ring shared by all waves, one
+// barrier per step.  Needs row0 a multiple of 8 (16-byte aligned slices).
+// Two waves a SIMD as in the right product; k = 201, 2048 rows, 100000
+// points in d = 128: 564 us with 4 waves of 4 tiles and X updated lane by
+// lane, 476 with X in column runs, 285 with 8 waves of 2 tiles.  391 blocks
+// take two rounds over 256 CUs; the X update, 0.32 GB, is 75 us of it.
+constexpr int kLeftRingWaves = 8, kLeftJT = 2;
 
 template <int DP, int TP>
 __global__ __launch_bounds__(64 * kLeftRingWaves, 1) void k_rbf_left_bf16_ring(RbfLpArgs g) {
@@ -559,7 +572,9 @@ __global__ __launch_bounds__(64 * kLeftRingWaves, 1) void k_rbf_left_bf16_ring(R
   constexpr int I_US = US_BYTES / 1024, I_XS = XS_BYTES / 1024, ITEMS = I_US + I_XS + 1;
   constexpr int IPW = (ITEMS + NW - 1) / NW;
   static_assert(US_BYTES % 1024 == 0 && XS_BYTES % 1024 == 0 && (NS - 2) * IPW <= 62, "copy items");
-  __shared__ __attribute__((aligned(1024))) uint8_t ring[NS * SLOT];
+  constexpr int LT = PR + 4;                        // floats a point of the epilogue's tiles
+  constexpr int TILES = NW * 16 * LT * 4;
+  __shared__ __attribute__((aligned(1024))) uint8_t ring[NS * SLOT > TILES ? NS * SLOT : TILES];
   // wave index as a scalar: the copy items, their counts and the vmcnt waits
   // below branch on it, and a per-lane value would turn every wave-uniform
   // branch into exec-masked code that runs each wait case in turn
@@ -585,65 +600,60 @@ __global__ __launch_bounds__(64 * kLeftRingWaves, 1) void k_rbf_left_bf16_ring(R
     be[y] = (jp < g.N) ? -lg * g.nrm[jp] : 0.f;
   }
 
-  // Per-lane sources of the wave's copies at the first step; a step moves
-  // each by BK window rows (2 BK bytes along an Upsilon row, BK points rows,
-  // 4 BK bytes of norms).  Past the window's end the sources are clamped.
-  const char* dsrc[IPW];
+  // The wave's copies: a scalar base that moves by BK window rows a step
+  // (2 BK bytes along an Upsilon row, BK points rows, 4 BK bytes of norms)
+  // and a lane offset that stays.  Past the window's end the sources are
+  // clamped.
+  uint32_t doff[IPW];
 #pragma unroll
   for (int s = 0; s < IPW; ++s) {
     const int it = wave + NW * s;
     if (it < I_US) {  // 16 map rows of the Upsilon slice
       const int r = 16 * it + (lane >> 2), p = lane & 3;
-      int64_t row = p0 + r;
-      row = row < g.M ? row : g.M - 1;
-      dsrc[s] = reinterpret_cast<const char*>(g.U + row * g.ldu + g.row0 + 8 * (p ^ os_swz(r)));
+      const int64_t rb = p0 + 16 * it < g.M ? p0 + 16 * it : g.M - 1, row = p0 + r < g.M ? p0 + r : g.M - 1;
+      doff[s] = (uint32_t)(2 * ((row - rb) * g.ldu + 8 * (p ^ os_swz(r))));
     } else if (it < I_US + I_XS) {  // RPI window rows
-      const int x = it - I_US;
-      const int r = RPI * x + lane / CPR, p = lane % CPR;
-      dsrc[s] = reinterpret_cast<const char*>(g.P + (g.row0 + r) * g.ldpb + 8 * (p ^ xs_swz<CPR>(r)));
+      const int r = RPI * (it - I_US) + lane / CPR, p = lane % CPR;
+      doff[s] = (uint32_t)(2 * (r * DP + 8 * (p ^ xs_swz<CPR>(r))));
     } else {  // norms of the step's window rows (lanes >= 32 duplicate, unused)
-      dsrc[s] = reinterpret_cast<const char*>(g.nrm + g.row0 + (lane & 31));
+      doff[s] = 4 * (lane & 31);
     }
   }
-  auto issue = [&](int u) {
-    uint8_t* slot = ring + (u % NS) * SLOT;
+  auto issue = [&](int u, int at) {  // at: the step's slot, in bytes
+    uint8_t* slot = ring + at;
     const int64_t i0 = (int64_t)u * BK;
     const bool tail = i0 + BK > g.K;
+    const int last = (int)(g.K - i0) - 1;  // the step's last window row
 #pragma unroll
     for (int s = 0; s < IPW; ++s) {
       const int it = wave + NW * s;
       if (it < I_US) {
-        const char* src = dsrc[s] + i0 * 2;
-        if (tail) {  // a chunk starting past the window reads the row's first chunk (finite, multiplied by zero)
-          const int r = 16 * it + (lane >> 2), p = lane & 3;
-          if (i0 + 8 * (p ^ os_swz(r)) >= g.K) src = dsrc[s] - 16 * (p ^ os_swz(r));
+        uint32_t off = doff[s];
+        if (tail) {  // a chunk starting past the window reads the step's first chunk (finite, multiplied by zero)
+          const int r = 16 * it + (lane >> 2), p = lane & 3, c = p ^ os_swz(r);
+          if (8 * c > last) off -= 16 * c;
         }
-        __builtin_amdgcn_global_load_lds((const void*)src, (SKEMA_LDS void*)(slot + 1024 * it), 16, 0, 0);
+        const int64_t rb = p0 + 16 * it < g.M ? p0 + 16 * it : g.M - 1;
+        copy16_to_lds(g.U + rb * g.ldu + g.row0 + i0, off, slot + 1024 * it);
       } else if (it < I_US + I_XS) {
         const int x = it - I_US;
-        const char* src = dsrc[s] + i0 * (2 * DP);
+        uint32_t off = doff[s];
         if (tail) {
           const int r = RPI * x + lane / CPR, p = lane % CPR;
-          int64_t i = i0 + r;
-          i = i < g.K ? i : g.K - 1;
-          src = reinterpret_cast<const char*>(g.P + (g.row0 + i) * g.ldpb + 8 * (p ^ xs_swz<CPR>(r)));
+          off = (uint32_t)(2 * ((r < last ? r : last) * DP + 8 * (p ^ xs_swz<CPR>(r))));
         }
-        __builtin_amdgcn_global_load_lds((const void*)src, (SKEMA_LDS void*)(slot + US_BYTES + 1024 * x), 16, 0, 0);
+        copy16_to_lds(g.P + (g.row0 + i0) * DP, off, slot + US_BYTES + 1024 * x);
       } else if (it == I_US + I_XS) {
-        const char* src = dsrc[s] + i0 * 4;
-        if (tail) {
-          int64_t i = i0 + (lane & 31);
-          i = i < g.K ? i : g.K - 1;
-          src = reinterpret_cast<const char*>(g.nrm + g.row0 + i);
-        }
-        __builtin_amdgcn_global_load_lds((const void*)src, (SKEMA_LDS void*)(slot + NI_OFF), 4, 0, 0);
+        uint32_t off = doff[s];
+        if (tail) off = 4 * ((lane & 31) < last ? (lane & 31) : last);
+        copy4_to_lds(g.nrm + g.row0 + i0, off, slot + NI_OFF);
       }
     }
   };
 
   // Gram tiles of step u (window rows x the wave's points)
-  auto gram = [&](int u, f4v (&gr)[2][JT]) {
-    const uint8_t* xs = ring + (u % NS) * SLOT + US_BYTES;
+  auto gram = [&](int at, f4v (&gr)[2][JT]) {
+    const uint8_t* xs = ring + at + US_BYTES;
 #pragma unroll
     for (int x = 0; x < 2; ++x) {
       const int r = 8 * (l16 >> 2) + 4 * x + (l16 & 3);
@@ -658,14 +668,16 @@ __global__ __launch_bounds__(64 * kLeftRingWaves, 1) void k_rbf_left_bf16_ring(R
       }
     }
   };
-  auto interior = [&](int u) {
-    const int64_t i0 = (int64_t)u * BK, gi0 = g.row0 + i0;  // the step's window rows, as point indices
-    return pts_full && i0 + BK <= g.K && (gi0 + BK <= wj0 || gi0 >= wj0 + 16 * JT);
-  };
+  // interior steps: every window row in range and none of the wave's own
+  // points among them (the diagonal lies in steps dlo .. dhi - 1)
+  const int64_t dg = wj0 - g.row0;
+  const int full = pts_full ? (int)(g.K / BK) : 0;
+  const int dlo = dg > 0 ? (int)(dg / BK) : 0, dhi = dg + 16 * JT > 0 ? (int)((dg + 16 * JT + BK - 1) / BK) : 0;
+  auto interior = [&](int u) { return u < full && (u < dlo || u >= dhi); };
   // K of step u (B operands: lane l holds point l%16 of tile y, window rows
   // 8 (l/16) .. +7 of the step) with the range and diagonal checks
-  auto exp_edge = [&](int u, const f4v (&gr)[2][JT], bf16x8 (&kb)[JT]) {
-    const float* ni = reinterpret_cast<const float*>(ring + (u % NS) * SLOT + NI_OFF);
+  auto exp_edge = [&](int u, int at, const f4v (&gr)[2][JT], bf16x8 (&kb)[JT]) {
+    const float* ni = reinterpret_cast<const float*>(ring + at + NI_OFF);
     const int64_t i0 = (int64_t)u * BK;
 #pragma unroll
     for (int y = 0; y < JT; ++y) {
@@ -682,8 +694,8 @@ __global__ __launch_bounds__(64 * kLeftRingWaves, 1) void k_rbf_left_bf16_ring(R
         }
     }
   };
-  auto exp_fast = [&](int u, const f4v (&gr)[2][JT], bf16x8 (&kb)[JT]) {
-    const float* ni = reinterpret_cast<const float*>(ring + (u % NS) * SLOT + NI_OFF);
+  auto exp_fast = [&](int at, const f4v (&gr)[2][JT], bf16x8 (&kb)[JT]) {
+    const float* ni = reinterpret_cast<const float*>(ring + at + NI_OFF);
     const f4v m0 = *reinterpret_cast<const f4v*>(ni + 8 * lq);
     const f4v m1 = *reinterpret_cast<const f4v*>(ni + 8 * lq + 4);
 #pragma unroll
@@ -704,41 +716,44 @@ __global__ __launch_bounds__(64 * kLeftRingWaves, 1) void k_rbf_left_bf16_ring(R
   bf16x8 kb[JT];
 #pragma unroll
   for (int p = 0; p < NS - 1; ++p)
-    if (p < steps) issue(p);
+    if (p < steps) issue(p, p * SLOT);
   if (steps > 0) {
     wait_vm_upto(((NS - 2) < (steps - 1) ? (NS - 2) : (steps - 1)) * dw);  // step 0 complete
     lds_barrier();
     f4v gr[2][JT];
     gram(0, gr);
     if (interior(0)) exp_fast(0, gr, kb);
-    else exp_edge(0, gr, kb);
+    else exp_edge(0, 0, gr, kb);
   }
-  for (int u = 0; u < steps; ++u) {
-    if (u + 1 < steps) {  // step u + 1 complete: at most steps u+2 .. min(u+NS-2, steps-1) in flight
-      const int last = (u + NS - 2 < steps - 1) ? u + NS - 2 : steps - 1;
-      wait_vm_upto((last - (u + 1)) * dw);
+  for (int u = 0, at = 0, atn = SLOT, fill = (NS - 1) * SLOT; u < steps; ++u) {  // slots of u, u + 1, u + NS - 1
+    if (u + NS - 1 <= steps) {  // step u + 1 complete: steps u+2 .. u+NS-2 in flight
+      if (dw == IPW) wait_vm<(NS - 3) * IPW>();
+      else wait_vm<(NS - 3) * (IPW - 1)>();
+    } else if (u + 1 < steps) {  // steps u+2 .. steps-1
+      wait_vm_upto((steps - 2 - u) * dw);
     }
     lds_barrier();  // every wave's copies of step u+1 landed; slot (u-1) % NS is free
-    if (u + NS - 1 < steps) issue(u + NS - 1);
-    const int un = (u + 1 < steps) ? u + 1 : u;  // the last step forms a Gram it does not use
+    if (u + NS - 1 < steps) issue(u + NS - 1, fill);
+    const int un = u + 1;  // past the last step: a Gram of the slot's older contents, not used
     f4v gr[2][JT];
-    gram(un, gr);
+    gram(atn, gr);
     // the sketch MFMAs of step u, map-row tile by map-row tile, each
     // followed by a share of the exponentials of step u+1
-    const uint8_t* us = ring + (u % NS) * SLOT;
-    const float* ni = reinterpret_cast<const float*>(ring + (un % NS) * SLOT + NI_OFF);
+    const uint8_t* us = ring + at;
+    const float* ni = reinterpret_cast<const float*>(ring + atn + NI_OFF);
     f4v mi[2];
     mi[0] = *reinterpret_cast<const f4v*>(ni + 8 * lq);
     mi[1] = *reinterpret_cast<const f4v*>(ni + 8 * lq + 4);
     bf16x8 kn[JT];
-    bf16x8 a = *reinterpret_cast<const bf16x8*>(us + 64 * l16 + 16 * (lq ^ os_swz(l16)));
+    auto up_at = [&](int z) {
+      const int r = 16 * z + l16;
+      return *reinterpret_cast<const bf16x8*>(us + 64 * r + 16 * (lq ^ os_swz(r)));
+    };
+    bf16x8 a = up_at(0), a1 = up_at(1);  // read two map-row tiles ahead
 #pragma unroll
     for (int z = 0; z < TP; ++z) {
-      bf16x8 an = a;
-      if (z + 1 < TP) {
-        const int r = 16 * (z + 1) + l16;
-        an = *reinterpret_cast<const bf16x8*>(us + 64 * r + 16 * (lq ^ os_swz(r)));
-      }
+      bf16x8 a2 = a1;
+      if (z + 2 < TP) a2 = up_at(z + 2);
 #pragma unroll
       for (int y = 0; y < JT; ++y) acc[y][z] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, kb[y], acc[y][z], 0, 0, 0);
 #pragma unroll
@@ -749,22 +764,51 @@ __global__ __launch_bounds__(64 * kLeftRingWaves, 1) void k_rbf_left_bf16_ring(R
         kn[y][4 * x + v] = (__bf16)k;
       }
       __builtin_amdgcn_sched_barrier(0);
-      a = an;
+      a = a1;
+      a1 = a2;
     }
-    if (!interior(un)) exp_edge(un, gr, kn);
+    if (!interior(un) && un < steps) exp_edge(un, atn, gr, kn);
 #pragma unroll
     for (int y = 0; y < JT; ++y) kb[y] = kn[y];
+    fill = at;
+    at = atn;
+    atn = atn + SLOT == NS * SLOT ? 0 : atn + SLOT;
   }
+  // X is read and written in column runs of 64 rows: the wave turns
+  // each 16-point tile round in its own part of the ring (16 TP + 4 floats a
+  // point), then keeps 4 columns of loads in flight.  Stored straight from
+  // the MFMA layout, every lane's read, multiply and write of 8 bytes waited
+  // for the one before it.
+  lds_barrier();  // every wave is done with the ring
+  constexpr int RC = (PR + 63) / 64, CB = 4;
+  float* tile = reinterpret_cast<float*>(ring) + wave * (16 * LT);
+  const GemmOut& o = g.out;
 #pragma unroll
   for (int y = 0; y < JT; ++y) {
-    const int64_t jp = wj0 + 16 * y + l16;
 #pragma unroll
-    for (int z = 0; z < TP; ++z)
+    for (int z = 0; z < TP; ++z) *reinterpret_cast<f4v*>(tile + l16 * LT + 16 * z + 4 * lq) = acc[y][z];
+    const int64_t j0 = wj0 + 16 * y;
+    const int nj = g.N - j0 < 16 ? (int)(g.N - j0) : 16;  // <= 0 past the last point
+    for (int q0 = 0; q0 < nj; q0 += CB) {
+      double old[CB][RC];
 #pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int64_t p = p0 + 16 * z + 4 * lq + v;
-        if (p < g.M && jp < g.N) store_out(g.out, p, jp, (double)acc[y][z][v]);
-      }
+      for (int q = 0; q < CB; ++q)
+#pragma unroll
+        for (int r = 0; r < RC; ++r) {
+          const int64_t p = p0 + 64 * r + lane;
+          const bool in = q0 + q < nj && 64 * r + lane < PR && p < g.M;
+          old[q][r] = (in && o.beta1 != 0.0) ? o.C1[p + (j0 + q0 + q) * o.ldc1] : 0.0;
+        }
+#pragma unroll
+      for (int q = 0; q < CB; ++q)
+#pragma unroll
+        for (int r = 0; r < RC; ++r) {
+          const int64_t p = p0 + 64 * r + lane;
+          if (q0 + q < nj && 64 * r + lane < PR && p < g.M)
+            o.C1[p + (j0 + q0 + q) * o.ldc1] =
+                o.alpha1 * (double)tile[(q0 + q) * LT + 64 * r + lane] + o.beta1 * old[q][r];
+        }
+    }
   }
 }
 
@@ -896,6 +940,9 @@ __global__ __launch_bounds__(64 * NW) void k_rbf_left_bf16(RbfLpArgs g) {
     }
 }
 
+// the ring kernels reach 16 rows of a map at 32-bit byte offsets
+constexpr int64_t kLdsCopyLd = (int64_t)1 << 26;
+
 constexpr int kTnChoices[] = {1, 2, 3, 4, 5};
 constexpr int kTpChoices[] = {1, 2, 4, 8, 13};
 
@@ -955,7 +1002,7 @@ void rbf_right_bf16(Ctx* c, const __bf16* P, int dp, const float* nrm, float gam
   a.G = G; a.ldg = ldg;
   // tall tiles (256 rows x 208 columns) once the window fills them;
   // otherwise 64 rows x all columns
-  const bool tall = a.M >= 128;
+  const bool tall = a.M >= 128 && ldop < kLdsCopyLd;
   const int tn = pick(kTnChoices, cdiv(cdiv(a.N, 16), 8));
   const int64_t col_blocks = tall ? cdiv(a.N, kTallCols) : cdiv(a.N, 128 * tn);
   a.tiles_m = (int)cdiv(a.M, tall ? kTallRows : 64);
@@ -1022,7 +1069,7 @@ void update_rbf_window_bf16(Sketch& sk, const double* points, int64_t ldp, int64
     a.out.C1 = sk.X.as<double>(); a.out.ldc1 = k; a.out.alpha1 = eta; a.out.beta1 = nu; a.out.nsplit = n;
     a.out.C2 = a.out.C1; a.out.ldc2 = k;
     const int tp = pick(kTpChoices, cdiv(k, 16));
-    if (tp >= 8 && row0 % 8 == 0) {  // long map-row tiles on aligned windows: the ring kernel
+    if (tp >= 8 && row0 % 8 == 0 && sk.lp_ldups < kLdsCopyLd) {  // long map-row tiles on aligned windows: the ring kernel
       const dim3 grid((unsigned)cdiv(n, 16 * kLeftJT * kLeftRingWaves), (unsigned)cdiv(k, 16 * tp));
       const dim3 block(64 * kLeftRingWaves);
 #define SKEMA_LEFT_RING(DP, TP) hipLaunchKernelGGL((k_rbf_left_bf16_ring<DP, TP>), grid, block, 0, st, a)
