@@ -618,6 +618,156 @@ __global__ __launch_bounds__(kThreads) void k_nt_bf16(NtArgs g) {
   nt_epilogue<TM, TN, BM, BN, false>(g, acc, m0, n0, wm, wn, lane);
 }
 
+// ---- split-BF16 ring kernel ------------------------------------------------
+// The split-BF16 product for the K ranges k_mx does not take (not whole
+// 64-element steps), 2 x 4 waves of (16 TM) x 32, block tile 32 TM x 128.
+// Steps of 32 K elements, the order of k_nt_bf16 (hi.hi, hi.lo, lo.hi per
+// step), so the two give the same bits.  Both planes of both tiles go global
+// -> LDS (64-byte rows, 16-byte chunk c of row r at c ^ ((r >> 2) & 3)) into
+// an NS-slot ring; a step's fragments are read into registers during the
+// step before, so its slot is free again when its products start and NS - 1
+// steps of copies are in flight.  The last step of a K range zeroes what lies
+// past the range; its copies past the range repeat the row's first chunk.
+// Right product of a 2048 x 5003 window, k + s = 604: 102 us on k_nt_bf16
+// (64 x 64 tiles, each load waited for before the next step's barrier), 71 us
+// here with 4 waves of (16 TM) x 64 (one a SIMD: nothing runs beside its
+// waits and scalar work), 63 with 8 waves, 56 with the partial step out of
+// the loop (its merge made the compiler wait for the next step's fragments).
+// The matrix cores are busy 40% of that; copies are 64-byte row pieces, half
+// an L2 line a request.
+constexpr int kRingThreads = 512;
+template <int TM>
+__global__ __launch_bounds__(kRingThreads, 1) void k_ring_bf16x3(NtArgs g) {
+  constexpr int TN = 2, BM = 32 * TM, BN = 64 * TN, BK = 32, NS = 4, NW = 8;
+  constexpr int ROWS = BM + BN, SLOT = 2 * ROWS * 2 * BK;  // A hi | B hi | A lo | B lo
+  constexpr int IA = BM / 16, ITEMS = 2 * ROWS / 16, IPW = (ITEMS + NW - 1) / NW;
+  static_assert(ITEMS > (IPW - 1) * NW && (NS - 1) * IPW < 63, "every wave has IPW copies or one less");
+  __shared__ __attribute__((aligned(1024))) uint8_t ring[NS * SLOT];
+  const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, q = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave & 1, wn = wave >> 1;
+  const int t = xcd_remap(blockIdx.x, gridDim.x);
+  const int64_t m0 = (int64_t)(t % g.tiles_m) * BM;
+  const int64_t n0 = (int64_t)(t / g.tiles_m) * BN;
+  const int64_t kbeg = (int64_t)blockIdx.z * g.k_per_split;
+  const int64_t kend = (g.K < kbeg + g.k_per_split) ? g.K : kbeg + g.k_per_split;
+  const int steps = (int)((kend - kbeg + BK - 1) / BK);
+
+  const int dw = (ITEMS - wave + NW - 1) / NW;  // copies this wave issues per step
+  // Copy items of 16 rows, wave w's at w + NW s: a scalar base (the item's
+  // first row) and the lane's byte offset; rows past M / N repeat the last
+  // row (computed, never stored).
+  const __bf16* base[IPW];
+  uint32_t off[IPW];
+#pragma unroll
+  for (int s = 0; s < IPW; ++s) {
+    const int at = wave + NW * s, it = at < ITEMS ? at : 0;  // past the last: not issued
+    const int plane = it / (ITEMS / 2), i = it % (ITEMS / 2);
+    const bool isa = i < IA;
+    const int64_t lim = isa ? g.M : g.N, ld = isa ? g.lda : g.ldb;
+    const int64_t first = isa ? m0 + 16 * i : n0 + 16 * (i - IA), r = first + (lane >> 2);
+    const int64_t rb = first < lim ? first : lim - 1, row = r < lim ? r : lim - 1;
+    const void* p = isa ? (plane ? g.al : g.ah) : (plane ? g.bl : g.bh);
+    base[s] = static_cast<const __bf16*>(p) + rb * ld + (isa ? g.koff_a : 0) + kbeg;
+    off[s] = (uint32_t)(2 * (row - rb) * ld) + 16 * ((lane & 3) ^ (lane >> 4));
+  }
+  auto issue = [&](int st) {
+    uint8_t* slot = ring + (st % NS) * SLOT;
+    const int64_t k0 = (int64_t)st * BK, left = kend - kbeg - k0;
+#pragma unroll
+    for (int s = 0; s < IPW; ++s) {
+      if (s >= dw) break;
+      uint32_t o = off[s];
+      if (left < BK) {
+        const int c = (lane & 3) ^ (lane >> 4);
+        if (8 * c >= left) o -= 16 * c;
+      }
+      copy16_to_lds(base[s] + k0, o, slot + 1024 * (wave + NW * s));
+    }
+  };
+  // fragments of step st: hi in [0], lo in [1]
+  struct Frags { bf16x8 a[2][TM], b[2][TN]; };
+  const int so = 64 * l16 + 16 * (q ^ (l16 >> 2));
+  auto read = [&](int st, Frags& f) {
+    const uint8_t* slot = ring + (st % NS) * SLOT;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+#pragma unroll
+      for (int x = 0; x < TM; ++x)
+        f.a[h][x] = *reinterpret_cast<const bf16x8*>(slot + h * (SLOT / 2) + 64 * (16 * (wm * TM + x)) + so);
+#pragma unroll
+      for (int y = 0; y < TN; ++y)
+        f.b[h][y] = *reinterpret_cast<const bf16x8*>(slot + h * (SLOT / 2) + 64 * (BM + 16 * (wn * TN + y)) + so);
+    }
+  };
+
+  f4v acc[TM][TN];
+#pragma unroll
+  for (int x = 0; x < TM; ++x)
+#pragma unroll
+    for (int y = 0; y < TN; ++y) acc[x][y] = f4v{0.f, 0.f, 0.f, 0.f};
+  auto products = [&](const Frags& f) {
+#pragma unroll
+    for (int z = 0; z < 3; ++z)  // hi.hi, hi.lo, lo.hi
+#pragma unroll
+      for (int y = 0; y < TN; ++y)
+#pragma unroll
+        for (int x = 0; x < TM; ++x)
+          acc[x][y] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.a[z == 2][x], f.b[z == 1][y], acc[x][y], 0, 0, 0);
+  };
+  // a step that is not the last one
+  auto step = [&](int st, const Frags& f, Frags& nf) {
+    if (st + NS <= steps) {  // step st + 1 complete: steps st+2 .. st+NS-1 in flight
+      if (dw == IPW) wait_vm<(NS - 2) * IPW>();
+      else wait_vm<(NS - 2) * (IPW - 1)>();
+    } else {  // steps st+2 .. steps-1
+      wait_vm_upto((steps - 2 - st) * dw);
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this step's fragments are in: its slot is free
+    lds_barrier();
+    if (st + NS < steps) issue(st + NS);
+    read(st + 1, nf);
+    products(f);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto last_step = [&](Frags& f) {
+    const int64_t left = kend - kbeg - (int64_t)(steps - 1) * BK;
+    if (left < BK) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const bool in = 8 * q + e < left;
+#pragma unroll
+          for (int x = 0; x < TM; ++x) f.a[h][x][e] = in ? f.a[h][x][e] : (__bf16)0.f;
+#pragma unroll
+          for (int y = 0; y < TN; ++y) f.b[h][y][e] = in ? f.b[h][y][e] : (__bf16)0.f;
+        }
+      }
+    }
+    products(f);
+  };
+
+#pragma unroll
+  for (int p = 0; p < NS; ++p)
+    if (p < steps) issue(p);
+  Frags f0, f1;
+  wait_vm_upto(((NS < steps ? NS : steps) - 1) * dw);  // step 0 complete
+  lds_barrier();
+  read(0, f0);
+  int st = 0;
+  for (; st + 2 < steps; st += 2) {
+    step(st, f0, f1);
+    step(st + 1, f1, f0);
+  }
+  if (st + 1 < steps) {
+    step(st, f0, f1);
+    last_step(f1);
+  } else {
+    last_step(f0);
+  }
+  nt_epilogue_at<TM, TN, false, false>(g, acc, m0 + wm * (16 * TM), n0 + wn * (16 * TN), lane);
+}
+
 // FP32 NT GEMM on v_mfma_f32_16x16x4_f32.  Each lane reads 4 consecutive K
 // elements of its row (K quarter l/16 of a 16-wide chunk) with one 16-byte LDS
 // read and issues 4 MFMAs, element q of A with element q of B: every K index
@@ -1851,6 +2001,25 @@ bool nt_picks_mx(int prec, const NtArgs& a) {
   return pl.ns > 0 && ntx_eligible(prec, a) && a.K % kstep_mx == 0 && launch_mx(0, prec, a, pl, dim3(), true);
 }
 
+// Row tiles (16 rows) a wave of k_ring_bf16x3, or 0 for the 2 x 2 kernel,
+// which takes rows off the 16-byte boundaries (windows that start off a
+// multiple of 8): fewest rounds x rows over the 256 CUs.  The ring kernel is
+// the faster one at every size measured; whole updates in windows, 2 x 2
+// kernel -> ring: 500 x 301 in 64 rows 310 -> 275 us, 2000 x 1003 in 100 rows
+// 1125 -> 999, 3000 x 5003 in 500 rows 966 -> 588, 6000 x 20001 in 1111 rows
+// 3596 -> 2574.
+int ring_tile(const NtArgs& a, int splits) {
+  const int64_t far = (int64_t)1 << 27;  // 16 rows of an operand at 32-bit byte offsets
+  if (!ntx_eligible(SKEMA_PREC_BF16X3, a) || a.lda >= far || a.ldb >= far) return 0;
+  int best = 0;
+  int64_t best_cost = INT64_MAX;
+  for (int tm = 4; tm >= 2; --tm) {
+    const int64_t cost = cdiv(cdiv(a.M, 32 * tm) * cdiv(a.N, 128) * splits, 256) * tm;
+    if (cost < best_cost) { best_cost = cost; best = tm; }
+  }
+  return best;
+}
+
 // t (optional): a timing scope closed right after the product kernel, so
 // it covers that kernel and not the split-K reduction that follows.
 // ws = nullptr: no K split.  fill: as many K splits as fill the 256 CUs
@@ -1899,8 +2068,17 @@ void gemm_nt(hipStream_t st, int prec, NtArgs a, DevBuf* ws, Timed* t = nullptr,
   SKEMA_REQUIRE(!a.seg_steps || (prec == SKEMA_PREC_BF16 && pl.ns == 2 && pl.tm == 8 && pl.tn == 4 && pl.wm == 2 &&
                                  pl.wn == 4),
                 kErrUnsupported, "K segments need the 256 x 256 bf16 k_mx");
-  const dim3 grid((unsigned)(a.tiles_m * cdiv(a.N, pl.bn)), 1, (unsigned)splits);
-  launch_nt(st, prec, a, pl, grid);
+  const int rtm = (prec == SKEMA_PREC_BF16X3 && pl.ns == 0) ? ring_tile(a, splits) : 0;
+  if (rtm) {
+    a.tiles_m = (int)cdiv(a.M, 32 * rtm);
+    const dim3 grid((unsigned)(a.tiles_m * cdiv(a.N, 128)), 1, (unsigned)splits);
+    if (rtm == 4) hipLaunchKernelGGL(k_ring_bf16x3<4>, grid, dim3(kRingThreads), 0, st, a);
+    else if (rtm == 3) hipLaunchKernelGGL(k_ring_bf16x3<3>, grid, dim3(kRingThreads), 0, st, a);
+    else hipLaunchKernelGGL(k_ring_bf16x3<2>, grid, dim3(kRingThreads), 0, st, a);
+  } else {
+    const dim3 grid((unsigned)(a.tiles_m * cdiv(a.N, pl.bn)), 1, (unsigned)splits);
+    launch_nt(st, prec, a, pl, grid);
+  }
   check_launch("k_nt");
   if (t) t->stop();
   if (splits > 1) {
