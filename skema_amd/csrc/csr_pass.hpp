@@ -5,6 +5,9 @@
 
 namespace skema {
 
+// What the pass keeps of a sketch's sparse maps (Sketch::ell_pair).
+void prepare_csr_maps(Sketch& sk);
+
 // nnz: the nonzeros, as inspect_csr found them.
 void update_csr_all(Sketch& sk, const int64_t* rowptr, const int32_t* col, const double* val, int64_t nnz);
 

@@ -138,6 +138,9 @@ struct Sketch {
   int64_t ldphi = 0;
   // Sparse maps: [Omega; Psi] as CSR (rows p) and as CSR of its transpose.
   Csr sp_omps, sp_ompsT;
+  // Sparse maps: [Upsilon; Phi] column by column, 8 + 8 packed ELL entries
+  // (csr_pass.hip); empty when a map has no packed form.
+  DevBuf ell_pair;
   // Low-precision map copies (precision forms).
   DevBuf lp_ups, lp_omps, lp_phi;
   // fp8 E8M0 block scales of the window copies (L then R), kept apart from the

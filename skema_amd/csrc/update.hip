@@ -12,6 +12,7 @@
 // disappears.  The nu/eta axpy's are folded into the GEMM epilogues.
 #include <cmath>
 
+#include "csr_pass.hpp"
 #include "linalg.hpp"
 #include "lowp.hpp"
 #include "rbf.hpp"
@@ -100,6 +101,7 @@ void prepare_sketch_maps(Sketch& sk) {
       rp[j + 1] = (int64_t)ci.size();
     }
     upload_csr(sk.sp_ompsT, n, k + s, (int64_t)ci.size(), rp.data(), ci.data(), v.data(), st);
+    prepare_csr_maps(sk);
     return;
   }
   auto logical = [&](Map* m, DevBuf& own, const double*& ptr, int64_t& ld) {

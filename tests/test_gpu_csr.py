@@ -75,3 +75,24 @@ def test_inspection_after_a_bad_window(S):
         g.linear_update(good)
         for a, b in zip(g.state(), (osk.X, osk.Y, osk.Z)):
             assert O.rel_err(a, b) <= TOL
+
+
+# Sparse-sign maps with fewer than 8 entries a column and with 8, columns with
+# more nonzeros than a wave keeps (256) and with one, k + s past the joint
+# pass's 512 rows, rows of Psi long enough (64) to be split over blocks with a
+# remainder of the 8 loads in flight.
+@pytest.mark.parametrize("m,n,k,s,density,window", [(60, 40, 3, 5, 0.1, 60), (900, 130, 21, 43, 0.4, 250),
+                                                    (500, 1500, 60, 121, 0.004, 125), (400, 700, 200, 401, 0.02, 400)])
+@pytest.mark.parametrize("conv", ["cols", "rows"])
+def test_csr_sign_maps(S, m, n, k, s, density, window, conv):
+    print(f"case csr sign maps {conv} {m}x{n} k={k} s={s} w={window}", flush=True)
+    A = _matrix(m, n, density, n)
+    p = O.AlgParams(matrix_m=m, matrix_n=n, rank=2, sketch_range=k, sketch_core=s, window=window,
+                    dim_redux="sparse-sign", issparse=True, sketch_nu=0.9, sketch_eta=1.2)
+    osk = O.SketchySVD(p, sparse_convention=conv)
+    osk.linear_update(A)
+    g = S.SketchySVD(to_gpu_params(p), maps=gpu_maps({"Upsilon": osk.Upsilon, "Omega": osk.Omega, "Phi": osk.Phi,
+                                                      "Psi": osk.Psi}))
+    g.linear_update(S.CrsMatrix.from_scipy(A))
+    for a, b in zip(g.state(), (osk.X, osk.Y, osk.Z)):
+        assert O.rel_err(a, b) <= TOL
