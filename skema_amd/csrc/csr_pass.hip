@@ -10,11 +10,12 @@
 // ones, with no host synchronisation between windows.
 //
 // Sparse (sparse-sign) maps:
-//   CSC of A in two bucketing levels (column tiles, then columns) with LDS
-//   cursors, so the entries of a column come in no fixed order;
-//   left  (X and W = Phi diag(c) A in one pass): one wave per column of A,
-//         lanes over its nonzeros, each nonzero's term c_i a added into the
-//         rows p of the maps' column i;
+//   A bucketed by column tiles with LDS cursors, so the entries of a tile come
+//   in no fixed order;
+//   left  (X and W = Phi diag(c) A in one pass): one block per tile, each
+//         nonzero's term c_i a added into the rows p of the maps' column i.
+//         Maps or sizes this does not fit: a second bucketing level makes the
+//         CSC of A, and one wave per column of it, lanes over its nonzeros;
 //   right (Y): one block per 32 rows of A, threads over their nonzeros.
 //   Both accumulate in LDS in int64 fixed point (fixedpoint.hpp),
 //   so every sum is the same whatever order the atomics land in: X, Y, Z
@@ -43,7 +44,8 @@ namespace {
 // Runs are filled through LDS cursors, so the entries of a column come in no
 // fixed order; the products below do not depend on it.
 constexpr int kL1Rows = 256;
-constexpr int kMaxTiles = 256;
+constexpr int kMaxTiles = 512;
+constexpr int kCscTiles = 256;  // tiles of the CSC build (two levels)
 constexpr int kMaxTileCols = 4096;
 
 __global__ __launch_bounds__(256) void k_l1_count(const int64_t* rowptr, int64_t rows, const int32_t* col, int tc,
@@ -130,15 +132,15 @@ __global__ __launch_bounds__(256) void k_l1_scatter(const int64_t* rowptr, int64
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int64_t r0 = (int64_t)blockIdx.x * kL1Rows;
   const int nr = (int)((r0 + kL1Rows < rows) ? kL1Rows : rows - r0);
-  static_assert(kMaxTiles == 256, "one thread per tile");
-  cur[tid] = (tid < nt) ? base[tid] + off[(int64_t)tid * nb + blockIdx.x] : 0;
+  static_assert(kMaxTiles == 2 * 256, "two tiles a thread in the scan");
+  for (int t = tid; t < kMaxTiles; t += 256) cur[t] = (t < nt) ? base[t] + off[(int64_t)t * nb + blockIdx.x] : 0;
   for (int i = tid; i <= nr; i += 256) rp[i] = rowptr[r0 + i];
   __syncthreads();
   const int64_t e_end = rp[nr];
   static_assert(kL1Rows <= 256, "rows of a block fit a byte");
   for (int64_t b0 = rp[0]; b0 < e_end; b0 += kL1Batch) {
     const int nbat = (int)((e_end - b0 < kL1Batch) ? e_end - b0 : kL1Batch);
-    cnt[tid] = 0;  // nt <= 256 = blockDim
+    cnt[tid] = cnt[tid + 256] = 0;
     if (tid < nr) {  // thread t labels the entries of row t that fall in this batch
       const int64_t a = rp[tid] > b0 ? rp[tid] : b0;
       const int64_t b = rp[tid + 1] < b0 + nbat ? rp[tid + 1] : b0 + nbat;
@@ -161,8 +163,8 @@ __global__ __launch_bounds__(256) void k_l1_scatter(const int64_t* rowptr, int64
     for (int q = 0; q < E; ++q)
       if (tid + 256 * q < nbat) slot[q] = atomicAdd(&cnt[rec[q].col / tc], 1);
     __syncthreads();
-    {  // exclusive scan of cnt over the tiles, one thread per tile
-      const int v = cnt[tid];
+    {  // exclusive scan of cnt over the tiles, two per thread
+      const int v0 = cnt[2 * tid], v = v0 + cnt[2 * tid + 1];
       int x = v;
       for (int d = 1; d < 64; d <<= 1) {
         const int y = __shfl_up(x, d);
@@ -172,7 +174,8 @@ __global__ __launch_bounds__(256) void k_l1_scatter(const int64_t* rowptr, int64
       __syncthreads();
       int before = 0;
       for (int i = 0; i < w; ++i) before += wsum[i];
-      lst[tid] = before + x - v;
+      lst[2 * tid] = before + x - v;
+      lst[2 * tid + 1] = before + x - v + v0;
     }
     __syncthreads();
 #pragma unroll
@@ -185,7 +188,8 @@ __global__ __launch_bounds__(256) void k_l1_scatter(const int64_t* rowptr, int64
       brec[cur[t] + (x - lst[t])] = e;
     }
     __syncthreads();
-    cur[tid] += cnt[tid];  // cur has kMaxTiles = blockDim entries; tiles >= nt unused
+    cur[tid] += cnt[tid];
+    cur[tid + 256] += cnt[tid + 256];
     __syncthreads();
   }
 }
@@ -462,6 +466,118 @@ __global__ __launch_bounds__(256, PAIR ? 5 : 1) void k_left_fx(const int64_t* cp
   }
 }
 
+// The same from the column tiles of the level-1 buckets, for maps with joint
+// records: one block per tile of tc columns keeps all its accumulators in LDS,
+// so the tile's nonzeros are used in the order they lie in and the CSC is not
+// built.  A first pass takes each column's largest |c_i a| and its count, a
+// second adds the terms; the first kTileCache records a thread stay in
+// registers between the two.  Same scales, so the same sums as k_left_fx.
+// Bound by the LDS atomics and the gathers of the records' map columns, which
+// one block a CU (106 KB) overlaps only within itself: 65 us at 200000 x 20000,
+// 4e6 nonzeros, k + s = 304, against 45 (second bucketing level) + 56.
+constexpr int kTileSlots = 12288, kTileCols = 512, kTileCache = 8, kTileThreads = 1024;
+
+__global__ __launch_bounds__(kTileThreads) void k_left_tile(const int* base, const CooRec* brec, int tc, int64_t ncols,
+                                                            const double* cw, int64_t window, const uint4* pair,
+                                                            SpMapCols M1, int n1, double* out1, SpMapCols M2, int n2,
+                                                            double* out2) {
+  __shared__ unsigned long long acc[kTileSlots];  // tc columns x (n1 + n2)
+  __shared__ unsigned long long cmax[kTileCols];  // bits of a column's largest |term|
+  __shared__ int cnt[kTileCols];
+  __shared__ FxScale cs[kTileCols];
+  const int tid = threadIdx.x, na = n1 + n2;
+  const int64_t j0 = (int64_t)blockIdx.x * tc;
+  const int w = (int)((j0 + tc < ncols) ? tc : ncols - j0);
+  const int64_t b0 = base[blockIdx.x], b1 = base[blockIdx.x + 1];
+  const uint32_t wdw = (uint32_t)window;
+  auto record = [&](int64_t e) {
+    const uint4 x = reinterpret_cast<const uint4*>(brec)[e];
+    CooRec r;
+    r.row = (int32_t)x.x;
+    r.col = (int32_t)x.y;
+    r.val = __longlong_as_double((long long)(((unsigned long long)x.w << 32) | x.z));
+    return r;
+  };
+  CooRec rec[kTileCache];
+#pragma unroll
+  for (int q = 0; q < kTileCache; ++q) {
+    const int64_t e = b0 + tid + kTileThreads * q;
+    rec[q].col = -1;
+    if (e < b1) rec[q] = record(e);
+  }
+  for (int i = tid; i < w * na; i += kTileThreads) acc[i] = 0ull;
+  for (int i = tid; i < w; i += kTileThreads) {
+    cmax[i] = 0ull;
+    cnt[i] = 0;
+  }
+  __syncthreads();
+  auto take = [&](const CooRec& r, double t) {
+    const int c = (int)(r.col - j0);
+    atomicMax(&cmax[c], (unsigned long long)__double_as_longlong(fabs(t)));  // NaN orders above inf
+    atomicAdd(&cnt[c], 1);
+  };
+#pragma unroll
+  for (int q = 0; q < kTileCache; ++q) {
+    if (rec[q].col < 0) continue;
+    rec[q].val *= cw[(uint32_t)rec[q].row / wdw];
+    take(rec[q], rec[q].val);
+  }
+  for (int64_t e = b0 + kTileThreads * kTileCache + tid; e < b1; e += kTileThreads) {
+    const CooRec r = record(e);
+    take(r, r.val * cw[(uint32_t)r.row / wdw]);
+  }
+  __syncthreads();
+  for (int i = tid; i < w; i += kTileThreads)
+    cs[i] = fx_scale(__longlong_as_double((long long)cmax[i]),
+                     (int64_t)cnt[i] * (M1.zmax > M2.zmax ? M1.zmax : M2.zmax));
+  __syncthreads();
+  auto add = [&](const CooRec& r, const uint32_t (&a)[8], const uint32_t (&b)[8]) {
+    const int c = (int)(r.col - j0);
+    const FxScale fs = cs[c];
+    if (!fs.finite) return;
+    const long long V = fx_term(r.val, fs);
+    const unsigned long long vp = (unsigned long long)V, vn = (unsigned long long)(-V);
+    unsigned long long* d1 = acc + c * na;
+    unsigned long long* d2 = d1 + n1;
+#pragma unroll
+    for (int f = 0; f < 8; ++f)
+      if (f < M1.z) {
+        const uint32_t x = ell_entry<8, false, true>(a, 8, f);
+        atomicAdd(d1 + (x & 0x7fffffffu), (x >> 31) ? vn : vp);
+      }
+#pragma unroll
+    for (int f = 0; f < 8; ++f)
+      if (f < M2.z) {
+        const uint32_t x = ell_entry<8, false, true>(b, 8, f);
+        atomicAdd(d2 + (x & 0x7fffffffu), (x >> 31) ? vn : vp);
+      }
+  };
+#pragma unroll
+  for (int h = 0; h < kTileCache; h += 4) {  // the map columns of four records in flight
+    uint32_t u1[4][8], u2[4][8];
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      if (rec[h + q].col >= 0) ell_pair_load(pair, rec[h + q].row, u1[q], u2[q]);
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      if (rec[h + q].col >= 0) add(rec[h + q], u1[q], u2[q]);
+  }
+  for (int64_t e = b0 + kTileThreads * kTileCache + tid; e < b1; e += kTileThreads) {
+    CooRec r = record(e);
+    r.val *= cw[(uint32_t)r.row / wdw];
+    uint32_t a[8], b[8];
+    ell_pair_load(pair, r.row, a, b);
+    add(r, a, b);
+  }
+  __syncthreads();
+  for (int i = tid; i < w * na; i += kTileThreads) {
+    const int c = i / na, p = i - c * na;
+    const double v = fx_value((long long)acc[i], cs[c]);
+    if (p < n1) out1[p + (j0 + c) * n1] = M1.mag * v;
+    else out2[(p - n1) + (j0 + c) * n2] = M2.mag * v;
+  }
+}
+
 // Y(i, p) = eta * sum over row i's nonzeros (j, a) of a * M(p, j) for p in
 // [p0, p0 + pn), pn <= kRightSlots.  One block per kRightRows rows; each
 // thread takes the block's nonzeros tid, tid + 256, ... (kRightCache of them
@@ -669,45 +785,82 @@ void right_sparse_fx(hipStream_t st, const int64_t* rowptr, const int32_t* col, 
   }
 }
 
-// CSC of the whole CSR by the two bucketing levels (entries of a column in no
-// fixed order); false when a column tile would exceed kMaxTileCols.
-bool csc_by_buckets(hipStream_t st, const int64_t* rowptr, const int32_t* col, const double* val, int64_t m,
-                    int64_t n, int64_t nnz, DevBuf& scratch, CscWindow& H) {
-  int64_t nt = std::min<int64_t>(kMaxTiles, n);
-  const int64_t tc = cdiv(n, nt);
-  nt = cdiv(n, tc);
-  if (tc > kMaxTileCols || nnz <= 0 || nnz >= ((int64_t)1 << 31)) return false;  // int positions
-  const int64_t nb = cdiv(m, kL1Rows);
+// The nonzeros as (row, column, value) records bucketed by tiles of tc columns
+// (level 1): tile t's at brec[base[t] .. base[t + 1]), in no fixed order.
+// `more` further bytes of the scratch follow at `rest`.
+struct Buckets {
+  int64_t nt = 0, tc = 0;
+  int* base = nullptr;
+  CooRec* brec = nullptr;
+  char* rest = nullptr;
+};
+Buckets bucket_columns(hipStream_t st, const int64_t* rowptr, const int32_t* col, const double* val, int64_t m,
+                       int64_t n, int64_t nnz, int64_t tc, size_t more, DevBuf& scratch) {
+  Buckets B;
+  B.tc = tc;
+  B.nt = cdiv(n, tc);
+  const int64_t nt = B.nt, nb = cdiv(m, kL1Rows);
   SKEMA_REQUIRE(nt * nb < ((int64_t)1 << 31), kErrShape, "linear_update_csr: too many row blocks");
   const size_t o_off = align_up((size_t)nt * nb * sizeof(int), 256);
   const size_t o_tot = o_off + align_up((size_t)nt * nb * sizeof(int), 256);
   const size_t o_base = o_tot + align_up((size_t)nt * sizeof(int), 256);
   const size_t o_brec = o_base + align_up((size_t)(nt + 1) * sizeof(int), 256);
-  const size_t o_ptr = o_brec + align_up((size_t)nnz * sizeof(CooRec), 256);
-  const size_t o_row = o_ptr + align_up((size_t)(n + 1) * sizeof(int64_t), 256);
-  const size_t o_val = o_row + align_up((size_t)nnz * sizeof(int32_t), 256);
-  scratch.reserve(o_val + (size_t)nnz * sizeof(double));
+  const size_t o_rest = o_brec + align_up((size_t)nnz * sizeof(CooRec), 256);
+  scratch.reserve(o_rest + more);
   char* b = scratch.as<char>();
   int* cnt = reinterpret_cast<int*>(b);
   int* off = reinterpret_cast<int*>(b + o_off);
   int* tot = reinterpret_cast<int*>(b + o_tot);
-  int* base = reinterpret_cast<int*>(b + o_base);
-  CooRec* brec = reinterpret_cast<CooRec*>(b + o_brec);
+  B.base = reinterpret_cast<int*>(b + o_base);
+  B.brec = reinterpret_cast<CooRec*>(b + o_brec);
+  B.rest = b + o_rest;
+  hipLaunchKernelGGL(k_l1_count, dim3((unsigned)nb), dim3(256), 0, st, rowptr, m, col, (int)tc, (int)nt, (int)nb, cnt);
+  hipLaunchKernelGGL(k_tile_scan, dim3((unsigned)nt), dim3(1024), 0, st, cnt, (int)nb, off, tot);
+  hipLaunchKernelGGL(k_tile_base, dim3(1), dim3(1024), 0, st, tot, (int)nt, B.base);
+  hipLaunchKernelGGL(k_l1_scatter, dim3((unsigned)nb), dim3(256), 0, st, rowptr, m, col, val, (int)tc, (int)nt,
+                     (int)nb, off, B.base, B.brec);
+  check_launch("bucket_columns");
+  return B;
+}
+// int positions
+bool buckets_fit(int64_t nnz) { return nnz > 0 && nnz < ((int64_t)1 << 31); }
+
+// CSC of the whole CSR by the two bucketing levels (entries of a column in no
+// fixed order); false when a column tile would exceed kMaxTileCols.
+bool csc_by_buckets(hipStream_t st, const int64_t* rowptr, const int32_t* col, const double* val, int64_t m,
+                    int64_t n, int64_t nnz, DevBuf& scratch, CscWindow& H) {
+  const int64_t tc = cdiv(n, std::min<int64_t>(kCscTiles, n));
+  if (tc > kMaxTileCols || !buckets_fit(nnz)) return false;
+  const size_t o_row = align_up((size_t)(n + 1) * sizeof(int64_t), 256);
+  const size_t o_val = o_row + align_up((size_t)nnz * sizeof(int32_t), 256);
+  const Buckets B =
+      bucket_columns(st, rowptr, col, val, m, n, nnz, tc, o_val + (size_t)nnz * sizeof(double), scratch);
   H.rows = m;
   H.cols = n;
   H.nnz = nnz;
-  H.ptr = reinterpret_cast<int64_t*>(b + o_ptr);
-  H.row = reinterpret_cast<int32_t*>(b + o_row);
-  H.val = reinterpret_cast<double*>(b + o_val);
-  hipLaunchKernelGGL(k_l1_count, dim3((unsigned)nb), dim3(256), 0, st, rowptr, m, col, (int)tc, (int)nt, (int)nb, cnt);
-  hipLaunchKernelGGL(k_tile_scan, dim3((unsigned)nt), dim3(1024), 0, st, cnt, (int)nb, off, tot);
-  hipLaunchKernelGGL(k_tile_base, dim3(1), dim3(1024), 0, st, tot, (int)nt, base);
-  hipLaunchKernelGGL(k_l1_scatter, dim3((unsigned)nb), dim3(256), 0, st, rowptr, m, col, val, (int)tc, (int)nt,
-                     (int)nb, off, base, brec);
-  hipLaunchKernelGGL(k_l2_place, dim3((unsigned)nt), dim3(1024), 0, st, base, (int)nt, (int)tc, n, nnz, brec, H.ptr,
-                     H.row, H.val);
-  check_launch("csc_by_buckets");
+  H.ptr = reinterpret_cast<int64_t*>(B.rest);
+  H.row = reinterpret_cast<int32_t*>(B.rest + o_row);
+  H.val = reinterpret_cast<double*>(B.rest + o_val);
+  hipLaunchKernelGGL(k_l2_place, dim3((unsigned)B.nt), dim3(1024), 0, st, B.base, (int)B.nt, (int)tc, n, nnz, B.brec,
+                     H.ptr, H.row, H.val);
+  check_launch("k_l2_place");
   return true;
+}
+
+// Columns a tile for k_left_tile, 0 when it does not apply: the tile's
+// accumulators fit its LDS, at most kMaxTiles tiles, and of those the fewest
+// rounds x columns over the 256 CUs (one block each).  Whole passes, CSC ->
+// tiles: 500 x 300 with 3000 nonzeros 98 -> 93 us, 100000 x 200 with 2e5
+// 131 -> 96, 20000 x 50000 with 1e5 166 -> 140, 200000 x 20000 with 4e6
+// 309 -> 278: the faster one wherever it fits.
+int64_t left_tile_cols(int64_t n, int64_t na) {
+  const int64_t lo = cdiv(n, kMaxTiles), hi = std::min<int64_t>(kTileSlots / na, kTileCols);
+  int64_t best = 0, best_cost = INT64_MAX;
+  for (int64_t tc = lo; tc <= hi; ++tc) {
+    const int64_t cost = cdiv(cdiv(n, tc), 256) * tc;
+    if (cost <= best_cost) { best_cost = cost; best = tc; }
+  }
+  return best;
 }
 
 // Joint records of two maps' packed ELL columns: entry f of column c of the
@@ -760,6 +913,7 @@ void update_csr_all(Sketch& sk, const int64_t* rowptr, const int32_t* col, const
   }
   DevBuf& scr = c->scratch;
   CscWindow H;
+  Buckets tiles;
   double* cw = nullptr;
   double* Wm = nullptr;
   {
@@ -769,7 +923,10 @@ void update_csr_all(Sketch& sk, const int64_t* rowptr, const int32_t* col, const
     Wm = reinterpret_cast<double*>(scr.as<char>() + align_up((size_t)W * sizeof(double), 256));
     SKEMA_HIP(hipMemcpyAsync(cw, hw.data(), (size_t)W * sizeof(double), hipMemcpyHostToDevice, st));
     // the fixed-point products take the column entries in any order
-    if (!sk.sparse_maps || !csc_by_buckets(st, rowptr, col, val, m, n, nnz, sk.win, H))
+    const int64_t tc = sk.ell_pair.p && buckets_fit(nnz) ? left_tile_cols(n, k + s) : 0;
+    if (tc > 0)
+      tiles = bucket_columns(st, rowptr, col, val, m, n, nnz, tc, 0, sk.win);
+    else if (!sk.sparse_maps || !csc_by_buckets(st, rowptr, col, val, m, n, nnz, sk.win, H))
       H = csr_window_to_csc(st, rowptr, col, val, m, n, nnz, sk.win, /*sorted=*/true);
   }
   double* X = sk.X.as<double>();
@@ -778,8 +935,15 @@ void update_csr_all(Sketch& sk, const int64_t* rowptr, const int32_t* col, const
   if (sk.sparse_maps) {
     {
       Timed t(c, "sketch_left");
-      left_sparse_fx(st, H, *sk.maps[0], k, X, k, *sk.maps[2], s, Wm, s, cw, window,
-                     sk.ell_pair.p ? sk.ell_pair.as<uint4>() : nullptr);
+      const uint4* pair = sk.ell_pair.p ? sk.ell_pair.as<uint4>() : nullptr;
+      if (tiles.nt > 0) {
+        hipLaunchKernelGGL(k_left_tile, dim3((unsigned)tiles.nt), dim3(kTileThreads), 0, st, tiles.base, tiles.brec,
+                           (int)tiles.tc, n, cw, window, pair, map_cols(*sk.maps[0]), (int)k, X, map_cols(*sk.maps[2]),
+                           (int)s, Wm);
+        check_launch("k_left_tile");
+      } else {
+        left_sparse_fx(st, H, *sk.maps[0], k, X, k, *sk.maps[2], s, Wm, s, cw, window, pair);
+      }
     }
     {
       Timed t(c, "sketch_right");

@@ -78,11 +78,14 @@ def test_inspection_after_a_bad_window(S):
 
 
 # Sparse-sign maps with fewer than 8 entries a column and with 8, columns with
-# more nonzeros than a wave keeps (256) and with one, k + s past the joint
-# pass's 512 rows, rows of Psi long enough (64) to be split over blocks with a
+# more nonzeros than a wave (256) or a tile's block (8192) keeps and with one,
+# too many columns for 512 tiles, with k + s within a wave's 512 accumulators
+# and past them, rows of Psi long enough (64) to be split over blocks with a
 # remainder of the 8 loads in flight.
 @pytest.mark.parametrize("m,n,k,s,density,window", [(60, 40, 3, 5, 0.1, 60), (900, 130, 21, 43, 0.4, 250),
-                                                    (500, 1500, 60, 121, 0.004, 125), (400, 700, 200, 401, 0.02, 400)])
+                                                    (500, 1500, 60, 121, 0.004, 125), (400, 700, 200, 401, 0.02, 400),
+                                                    (18100, 7, 9, 19, 0.5, 6000), (300, 14400, 150, 301, 0.003, 100),
+                                                    (200, 11000, 200, 401, 0.004, 200)])
 @pytest.mark.parametrize("conv", ["cols", "rows"])
 def test_csr_sign_maps(S, m, n, k, s, density, window, conv):
     print(f"case csr sign maps {conv} {m}x{n} k={k} s={s} w={window}", flush=True)
