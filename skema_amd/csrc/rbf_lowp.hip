@@ -814,12 +814,36 @@ __global__ __launch_bounds__(64 * kLeftRingWaves, 1) void k_rbf_left_bf16_ring(R
 
 // Sum of the FP32 partials of the point splits (fixed order), then the
 // epilogue; consecutive threads own consecutive rows, so the stores coalesce.
+// Four partials are in flight at a time, of four rows each where the window
+// has a multiple of four: 10 partials of 2048 x 604 in 19 us, 27 one by one.
+template <int V>
 __global__ void k_rbf_right_bf16_reduce(RbfLpArgs g, int splits) {
-  const int64_t total = g.M * g.N;
-  for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < total; e += (int64_t)gridDim.x * blockDim.x) {
-    double v = 0.0;
-    for (int z = 0; z < splits; ++z) v += (double)g.part[(int64_t)z * total + e];
-    store_right(g, e % g.M, e / g.M, v);
+  typedef float fv __attribute__((ext_vector_type(V)));
+  const int64_t total = g.M * g.N, items = total / V;
+  for (int64_t it = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; it < items;
+       it += (int64_t)gridDim.x * blockDim.x) {
+    const int64_t e = it * V;
+    double v[V];
+#pragma unroll
+    for (int q = 0; q < V; ++q) v[q] = 0.0;
+    int z = 0;
+    for (; z + 4 <= splits; z += 4) {
+      fv x[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) x[u] = *reinterpret_cast<const fv*>(g.part + (int64_t)(z + u) * total + e);
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int q = 0; q < V; ++q) v[q] += (double)x[u][q];
+    }
+    for (; z < splits; ++z) {
+      const fv x = *reinterpret_cast<const fv*>(g.part + (int64_t)z * total + e);
+#pragma unroll
+      for (int q = 0; q < V; ++q) v[q] += (double)x[q];
+    }
+    const int64_t i = e % g.M, j = e / g.M;
+#pragma unroll
+    for (int q = 0; q < V; ++q) store_right(g, i + q, j, v[q]);
   }
 }
 
@@ -1033,8 +1057,10 @@ void rbf_right_bf16(Ctx* c, const __bf16* P, int dp, const float* nrm, float gam
   else launch_right<128>(st, a, grid, tn);
   check_launch("k_rbf_right_bf16");
   if (splits > 1) {
-    const int blocks = (int)std::min<int64_t>(cdiv(a.M * a.N, 256), 8192);
-    hipLaunchKernelGGL(k_rbf_right_bf16_reduce, dim3(blocks), dim3(256), 0, st, a, (int)splits);
+    const bool four = a.M % 4 == 0;
+    const int blocks = (int)std::min<int64_t>(cdiv(a.M * a.N / (four ? 4 : 1), 256), 8192);
+    if (four) hipLaunchKernelGGL(k_rbf_right_bf16_reduce<4>, dim3(blocks), dim3(256), 0, st, a, (int)splits);
+    else hipLaunchKernelGGL(k_rbf_right_bf16_reduce<1>, dim3(blocks), dim3(256), 0, st, a, (int)splits);
     check_launch("k_rbf_right_bf16_reduce");
   }
 }

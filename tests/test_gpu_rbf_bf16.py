@@ -26,9 +26,10 @@ BOUND = 2e-2
 
 # Features padded to 32, 64 and 128; 256-point and 256-row blocks and one past
 # them; 32-point steps with one, two and many in the last window and a
-# remainder; 8, 13 and 2 x 13 map-row tiles; window starts off a multiple of 8
+# remainder; 8, 13 and 2 x 13 map-row tiles; window starts off a multiple of 8;
+# the points split over blocks, with windows off a multiple of 4 rows
 @pytest.mark.parametrize("n,d,w,rank", [(257, 32, 128, 25), (512, 33, 129, 50), (300, 65, 136, 25), (641, 128, 256, 50),
-                                        (513, 64, 168, 60), (1100, 100, 544, 51), (385, 20, 384, 50)])
+                                        (513, 64, 168, 60), (1100, 100, 544, 51), (385, 20, 384, 50), (2101, 32, 131, 25)])
 def test_rbf_bf16_products_by_column(S, n, d, w, rank):
     print(f"case rbf bf16 columns n={n} d={d} w={w} r={rank}", flush=True)
     rng = np.random.default_rng(n * d)
