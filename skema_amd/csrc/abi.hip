@@ -636,7 +636,15 @@ int skema_linear_update_dense(skema_sketch* h, const double* A, int64_t lda) {
       sk.finalized = false;
     } else {
       zero_state(sk);
-      for_each_window(sk, [&](int64_t r0, int64_t w) { update_dense_window(sk, A + r0, lda, r0, w); });
+      int64_t next = 0;  // first row of the windows not taken in groups
+      for (const int64_t w = sk.p.window; w < sk.p.m;) {
+        const int64_t took = update_dense_windows(sk, A + next, lda, next, w, (sk.p.m - next) / w);
+        if (took == 0) break;
+        next += took * w;
+      }
+      for_each_window(sk, [&](int64_t r0, int64_t w) {
+        if (r0 >= next) update_dense_window(sk, A + r0, lda, r0, w);
+      });
     }
     sk.ctx->sync_if_needed();
   });

@@ -40,6 +40,11 @@ struct KArgs {
   int64_t k_per_split;
   double* partial;  // split-K slices [z][M x N], nullptr -> direct epilogue
   int tiles_t, tiles_s;
+  // k_gemm_ksplit<..., true>: `chain` products one after the other into the same output,
+  // A and B stepA and stepB elements further each time (blockIdx.y = 0), or
+  // as many products as gridDim.y, each into its own output
+  int chain = 1;
+  int64_t stepA = 0, stepB = 0, stepC1 = 0, stepC2 = 0;
 };
 
 // Workgroup ids are dealt round-robin to the 8 XCDs; give each XCD a
@@ -329,7 +334,7 @@ __global__ __launch_bounds__(kWideThreads) void k_gemm_wide(KArgs g) {
 // partial tiles summed through LDS in wave order.  These products are bound by
 // the latency of their K loop: 64 x 98 x 300 took 26 us with 64 x 64 tiles and a
 // barrier pair per 16 of K, and takes 5 us here; 803 x 803 x 4096 124 us.
-template <int KW, bool TA, bool TB>
+template <int KW, bool TA, bool TB, bool SERIES = false>
 __global__ __launch_bounds__(64 * KW) void k_gemm_ksplit(KArgs g) {
   __shared__ double part[KW][32][33];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -345,14 +350,15 @@ __global__ __launch_bounds__(64 * KW) void k_gemm_ksplit(KArgs g) {
     int64_t i = m0 + 16 * x + l16, j = n0 + 16 * x + l16;
     i = i < g.M ? i : g.M - 1;  // rows past the end: results not stored
     j = j < g.N ? j : g.N - 1;
-    pa[x] = g.A + (TA ? i * g.lda : i) + (kbeg + 2 * lq) * sa;
-    pb[x] = g.B + (TB ? j : j * g.ldb) + (kbeg + 2 * lq) * sb;
+    pa[x] = g.A + (SERIES ? blockIdx.y * g.stepA : 0) + (TA ? i * g.lda : i) + (kbeg + 2 * lq) * sa;
+    pb[x] = g.B + (SERIES ? blockIdx.y * g.stepB : 0) + (TB ? j : j * g.ldb) + (kbeg + 2 * lq) * sb;
+  }
+  GemmOut out = g.out;
+  if (SERIES) {
+    out.C1 += blockIdx.y * g.stepC1;
+    out.C2 += blockIdx.y * g.stepC2;
   }
   d4 acc[2][2];
-#pragma unroll
-  for (int x = 0; x < 2; ++x)
-#pragma unroll
-    for (int y = 0; y < 2; ++y) acc[x][y] = d4{0.0, 0.0, 0.0, 0.0};
   struct Frags {
     double a[2][4], b[2][4];
   };
@@ -396,54 +402,68 @@ __global__ __launch_bounds__(64 * KW) void k_gemm_ksplit(KArgs g) {
   const int64_t full = (kend - kbeg) / 16;
   const int left = (int)((kend - kbeg) % 16);
   Frags f0, f1;
-  if (wave < full) {
-    int64_t n = (full - 1 - wave) / KW + 1;
-    const int64_t last = wave + (n - 1) * KW;
-    auto at = [&](int64_t c) { return c < last ? c : last; };
-    int64_t c = wave;
-    load(f0, c);
-    load(f1, at(c + KW));
-    for (; n > 1; n -= 2) {
-      mma(f0);
-      load(f0, at(c + 2 * KW));
-      mma(f1);
-      load(f1, at(c + 3 * KW));
-      c += 2 * KW;
+  for (int link = 0; link < (SERIES ? g.chain : 1); ++link) {
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+      for (int y = 0; y < 2; ++y) acc[x][y] = d4{0.0, 0.0, 0.0, 0.0};
+    if (wave < full) {
+      int64_t n = (full - 1 - wave) / KW + 1;
+      const int64_t last = wave + (n - 1) * KW;
+      auto at = [&](int64_t c) { return c < last ? c : last; };
+      int64_t c = wave;
+      load(f0, c);
+      load(f1, at(c + KW));
+      for (; n > 1; n -= 2) {
+        mma(f0);
+        load(f0, at(c + 2 * KW));
+        mma(f1);
+        load(f1, at(c + 3 * KW));
+        c += 2 * KW;
+      }
+      if (n) mma(f0);
     }
-    if (n) mma(f0);
-  }
-  if (left > 0 && wave == (int)(full % KW)) {
+    if (left > 0 && wave == (int)(full % KW)) {
 #pragma unroll
-    for (int kk = 0; kk < 4; ++kk) {
-      const int kc = 8 * (kk / 2) + kk % 2;
-      const bool ok = kc + 2 * lq < left;
-      const int64_t k = 16 * full + (ok ? kc : -2 * lq);  // else this chunk's first
+      for (int kk = 0; kk < 4; ++kk) {
+        const int kc = 8 * (kk / 2) + kk % 2;
+        const bool ok = kc + 2 * lq < left;
+        const int64_t k = 16 * full + (ok ? kc : -2 * lq);  // else this chunk's first
 #pragma unroll
-      for (int x = 0; x < 2; ++x) {
-        const double va = pa[x][k * sa], vb = pb[x][k * sb];
-        f0.a[x][kk] = ok ? va : 0.0;
-        f0.b[x][kk] = ok ? vb : 0.0;
+        for (int x = 0; x < 2; ++x) {
+          const double va = pa[x][k * sa], vb = pb[x][k * sb];
+          f0.a[x][kk] = ok ? va : 0.0;
+          f0.b[x][kk] = ok ? vb : 0.0;
+        }
+      }
+      mma(f0);
+    }
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+      for (int y = 0; y < 2; ++y)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) part[wave][16 * y + lq + 4 * v][16 * x + l16] = acc[x][y][v];
+    __syncthreads();
+#pragma unroll
+    for (int e = tid; e < 1024; e += 64 * KW) {
+      const int ii = e & 31, jj = e >> 5;
+      double s = 0.0;
+#pragma unroll
+      for (int w = 0; w < KW; ++w) s += part[w][jj][ii];
+      const int64_t i = m0 + ii, j = n0 + jj;
+      if (i < g.M && j < g.N) {
+        if (g.partial) g.partial[(int64_t)blockIdx.z * g.M * g.N + i + j * g.M] = s;
+        else store_out(out, i, j, s);
       }
     }
-    mma(f0);
-  }
+    if (SERIES && link + 1 < g.chain) {
 #pragma unroll
-  for (int x = 0; x < 2; ++x)
-#pragma unroll
-    for (int y = 0; y < 2; ++y)
-#pragma unroll
-      for (int v = 0; v < 4; ++v) part[wave][16 * y + lq + 4 * v][16 * x + l16] = acc[x][y][v];
-  __syncthreads();
-#pragma unroll
-  for (int e = tid; e < 1024; e += 64 * KW) {
-    const int ii = e & 31, jj = e >> 5;
-    double s = 0.0;
-#pragma unroll
-    for (int w = 0; w < KW; ++w) s += part[w][jj][ii];
-    const int64_t i = m0 + ii, j = n0 + jj;
-    if (i < g.M && j < g.N) {
-      if (g.partial) g.partial[(int64_t)blockIdx.z * g.M * g.N + i + j * g.M] = s;
-      else store_out(g.out, i, j, s);
+      for (int x = 0; x < 2; ++x) {
+        pa[x] += g.stepA;
+        pb[x] += g.stepB;
+      }
+      __syncthreads();  // the partial tiles have been read
     }
   }
 }
@@ -509,6 +529,12 @@ void launch_ksplit(hipStream_t st, bool ta, bool tb, const KArgs& a, dim3 grid) 
   else hipLaunchKernelGGL((k_gemm_ksplit<KW, true, true>), grid, block, 0, st, a);
 }
 
+template <int KW>
+void launch_series(hipStream_t st, bool tb, const KArgs& a, dim3 grid) {
+  if (tb) hipLaunchKernelGGL((k_gemm_ksplit<KW, false, true, true>), grid, dim3(64 * KW), 0, st, a);
+  else hipLaunchKernelGGL((k_gemm_ksplit<KW, false, false, true>), grid, dim3(64 * KW), 0, st, a);
+}
+
 // One way to run a product, with its estimated time in CU cycles.
 struct Plan {
   bool wide = false;
@@ -564,6 +590,35 @@ void try_ksplit(Plan& best, int64_t M, int64_t N, int64_t K, bool may_split) {
 }
 
 }  // namespace
+
+bool gemm_f64_one_pass(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb) {
+  if (M <= 0 || N <= 0 || K <= 0) return false;
+  Plan p;
+  try_ksplit(p, M, N, K, true);
+  if (lda <= (int64_t)1 << 21 && ldb <= (int64_t)1 << 21) try_wide(p, M, N, K, true);
+  return p.cost < 1e300 && !p.wide && p.splits == 1;
+}
+
+void gemm_f64_series(hipStream_t stream, char transB, int64_t M, int64_t N, int64_t K, const double* A,
+                     int64_t lda, const double* B, int64_t ldb, const GemmOut& out, const GemmSeries& sr) {
+  const bool tb = (transB == 'T' || transB == 't');
+  SKEMA_REQUIRE(gemm_f64_one_pass(M, N, K, lda, ldb) && sr.count > 0 && (sr.chain || sr.count <= 65535), kErrShape,
+                "gemm_f64_series: not products of one pass");
+  SKEMA_REQUIRE(lda >= M && ldb >= (tb ? N : K), kErrShape, "gemm_f64_series: leading dimension too small");
+  Plan p;
+  try_ksplit(p, M, N, K, true);
+  KArgs a;
+  a.M = M; a.N = N; a.K = K; a.A = A; a.lda = lda; a.B = B; a.ldb = ldb; a.out = out;
+  a.tiles_t = (int)p.tiles_t; a.tiles_s = (int)p.tiles_s;
+  a.partial = nullptr;
+  a.k_per_split = cdiv(K, kBK) * kBK;
+  a.stepA = sr.stepA; a.stepB = sr.stepB; a.stepC1 = sr.stepC1; a.stepC2 = sr.stepC2;
+  a.chain = sr.chain ? (int)sr.count : 1;
+  const dim3 grid((unsigned)(p.tiles_t * p.tiles_s), sr.chain ? 1u : (unsigned)sr.count, 1);
+  if (p.wm == 16) launch_series<16>(stream, tb, a, grid);
+  else launch_series<8>(stream, tb, a, grid);
+  check_launch("k_gemm_ksplit (series)");
+}
 
 void gemm_f64(hipStream_t stream, char transA, char transB, int64_t M, int64_t N, int64_t K,
               const double* A, int64_t lda, const double* B, int64_t ldb, const GemmOut& out,

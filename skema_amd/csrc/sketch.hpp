@@ -165,6 +165,7 @@ double now_seconds();
 
 // Update kernels (per window); implemented in update.hip.
 void update_dense_window(Sketch& sk, const double* H, int64_t ldh, int64_t row0, int64_t rows);
+int64_t update_dense_windows(Sketch& sk, const double* H, int64_t ldh, int64_t row0, int64_t w, int64_t count);
 // nnz: the window's nonzeros, as inspect_csr found them.
 void update_csr_window(Sketch& sk, const int64_t* rowptr, const int32_t* col, const double* val, int64_t row0,
                        int64_t rows, int64_t nnz);

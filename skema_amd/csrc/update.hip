@@ -10,6 +10,7 @@
 // Phi[:,idx]*(H*Psi^T) so H*Omega^T and H*Psi^T share one pass over H
 // (one GEMM against Omega stacked over Psi) and the s x n intermediate
 // disappears.  The nu/eta axpy's are folded into the GEMM epilogues.
+#include <algorithm>
 #include <cmath>
 
 #include "csr_pass.hpp"
@@ -182,6 +183,54 @@ void update_dense_window(Sketch& sk, const double* H, int64_t ldh, int64_t row0,
     Timed t(c, "sketch_core");
     gemm_f64(st, 'N', 'N', s, s, rows, eta, sk.phiL + row0 * sk.ldphi, sk.ldphi, G, rows, nu, Z, s, &c->gws);
   }
+}
+
+// Up to `count` windows of w rows from row0 in three launches: all right
+// products at once, then the left and the core products as chains over the
+// windows.  Returns the windows taken, 0 where one of the products is not a
+// single launch by itself.  Small windows are bound by launches and by the few
+// blocks of one product: the 60 products of 20 windows of 100 x 1000, k = 41,
+// s = 83, take 0.5 ms one by one and 0.15 ms so.  A group's rows of A and G stay
+// within 128 MiB, so that the second pass over them finds them in the last-level
+// cache.
+int64_t update_dense_windows(Sketch& sk, const double* H, int64_t ldh, int64_t row0, int64_t w, int64_t count) {
+  const int64_t k = sk.k, s = sk.s, m = sk.p.m, n = sk.p.n;
+  if (sk.sparse_maps || sk.p.precision != SKEMA_PREC_FP64 || count < 2) return 0;
+  if (!gemm_f64_one_pass(k, n, w, sk.ldups, ldh) || !gemm_f64_one_pass(w, k + s, n, ldh, k + s) ||
+      !gemm_f64_one_pass(s, s, w, sk.ldphi, w))
+    return 0;
+  count = std::min<int64_t>({count, ((int64_t)128 << 20) / (w * (n + s) * 8), (int64_t)65535});
+  if (count < 2) return 0;
+  Ctx* c = sk.ctx;
+  hipStream_t st = c->stream;
+  const double eta = sk.p.eta, nu = sk.p.nu;
+  sk.G.reserve((size_t)count * w * s * sizeof(double));
+  double* G = sk.G.as<double>();
+  GemmSeries sr;
+  sr.count = count;
+  GemmOut o;
+  {
+    Timed t(c, "sketch_right");
+    o.C1 = sk.Y.as<double>() + row0; o.ldc1 = m; o.alpha1 = eta; o.beta1 = nu; o.nsplit = k;
+    o.C2 = G; o.ldc2 = w; o.alpha2 = 1.0; o.beta2 = 0.0;
+    sr.stepA = w; sr.stepB = 0; sr.stepC1 = w; sr.stepC2 = w * s;
+    gemm_f64_series(st, 'T', w, k + s, n, H, ldh, sk.omps.as<double>(), k + s, o, sr);
+  }
+  sr.chain = true;
+  sr.stepC1 = sr.stepC2 = 0;
+  {
+    Timed t(c, "sketch_left");
+    o.C1 = o.C2 = sk.X.as<double>(); o.ldc1 = o.ldc2 = k; o.nsplit = n;
+    sr.stepA = w * sk.ldups; sr.stepB = w;
+    gemm_f64_series(st, 'N', k, n, w, sk.upsL + row0 * sk.ldups, sk.ldups, H, ldh, o, sr);
+  }
+  {
+    Timed t(c, "sketch_core");
+    o.C1 = o.C2 = sk.Z.as<double>(); o.ldc1 = o.ldc2 = s; o.nsplit = s;
+    sr.stepA = w * sk.ldphi; sr.stepB = w * s;
+    gemm_f64_series(st, 'N', s, s, w, sk.phiL + row0 * sk.ldphi, sk.ldphi, G, w, o, sr);
+  }
+  return count;
 }
 
 void update_csr_window(Sketch& sk, const int64_t* rowptr, const int32_t* col, const double* val, int64_t row0,

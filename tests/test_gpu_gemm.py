@@ -71,3 +71,24 @@ def test_rbf_rows_in_ranges(S, n, d, window):
         K = np.exp(-0.5 / d * torch.cdist(X.cpu(), X.cpu()).numpy() ** 2)
         om = whole.maps["Omega"].download()
         assert np.linalg.norm(whole.state()[1] - K @ om.T) <= TOL * np.linalg.norm(K @ om.T)
+
+
+@pytest.mark.parametrize("m,n,w,k,s,nu", [(64, 33, 32, 3, 7, 1.0), (200, 129, 33, 21, 43, 0.7), (1000, 300, 64, 41, 83, 0.0),
+                                          (960, 20000, 64, 5, 11, 0.9), (2049, 1000, 100, 41, 83, 1.0)])
+def test_grouped_windows_equal_single_ones(S, m, n, w, k, s, nu):
+    """linear_update takes small windows in groups of one launch per product:
+    two windows, a shorter one after them, more than 128 MiB of rows (two
+    groups), and nu = 0, where no output is read.  Bit for bit the windows' own
+    updates."""
+    print(f"case grouped windows {m}x{n} w={w} nu={nu}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(m)
+    A = torch.randn((n, m), dtype=torch.float64, device="cuda", generator=g).t()
+    p = S.AlgParams(matrix_m=m, matrix_n=n, rank=2, sketch_range=k, sketch_core=s, window=w, sketch_nu=nu,
+                    sketch_eta=1.3)
+    maps = S.make_maps(p, dist="normal")
+    whole, parts = S.SketchySVD(p, maps=maps), S.SketchySVD(p, maps=maps)
+    whole.linear_update(A)
+    for r0 in range(0, m, w):
+        parts.update(A, (r0, min(m, r0 + w)))
+    for a, b in zip(whole.state(), parts.state()):
+        assert np.array_equal(a, b)
