@@ -891,6 +891,7 @@ void prepare_csr_maps(Sketch& sk) {
                      u.ell16.as<uint16_t>(), u.ell_zeta, f.ell16.as<uint16_t>(), f.ell_zeta, m,
                      sk.ell_pair.as<uint16_t>());
   check_launch("k_pair_ell");
+  SKEMA_HIP(hipStreamSynchronize(st));  // whatever stream the context uses later
 }
 
 void update_csr_all(Sketch& sk, const int64_t* rowptr, const int32_t* col, const double* val, int64_t nnz) {
