@@ -544,7 +544,12 @@ CsrInfo inspect_csr(Ctx* c, const int64_t* rowptr, const int32_t* col, int64_t r
   SKEMA_HIP(hipStreamSynchronize(st));
   const int64_t* h = static_cast<const int64_t*>(c->csr_host.p);
   const CsrInfo info{h[0], h[1], h[2]};
-  if (info.flags) fill_i32(st, reinterpret_cast<int*>(dev + 2), 2, 0);
+  if (info.flags) {
+    // The caller refuses the window, so nothing after this waits for the clearing,
+    // and the context's next inspection may run on another stream.
+    fill_i32(st, reinterpret_cast<int*>(dev + 2), 2, 0);
+    SKEMA_HIP(hipStreamSynchronize(st));
+  }
   return info;
 }
 

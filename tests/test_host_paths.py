@@ -1,0 +1,114 @@
+"""Host code of the library without a GPU: which kernels a call launches, what
+it leaves on its stream, and what it does where device memory runs short.  The
+library runs in a process of its own on tests/host_runtime.cpp, whose kernels do
+nothing and whose allocations can be limited."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+LIB = os.path.join(ROOT, "skema_amd", "libskema_mi355x.so")
+pytestmark = pytest.mark.skipif(not os.path.exists(LIB), reason="library not built")
+
+# The binding is loaded by its path: the package would bring torch, and its own
+# HIP runtime, into the process.
+PRELUDE = r"""
+import ctypes as C, importlib.util, os, sys
+rt = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
+rt.rt_used.restype = C.c_size_t
+rt.rt_set_limit.argtypes = [C.c_size_t]
+rt.rt_queued.restype, rt.rt_queued.argtypes = C.c_long, [C.c_void_p]
+rt.rt_launches.restype = C.c_char_p
+rt.rt_inspection.argtypes = [C.c_int64] * 3
+spec = importlib.util.spec_from_file_location("binding", os.path.join(sys.argv[2], "skema_amd", "_lib.py"))
+L = importlib.util.module_from_spec(spec)
+spec.loader.exec_module(L)
+L.load()
+MiB = 1 << 20
+
+def device(count, item=8):
+    p = C.c_void_p()
+    assert rt.hipMalloc(C.byref(p), C.c_size_t(count * item)) == 0
+    return p.value
+
+def context():
+    h = C.c_void_p()
+    L.call("skema_ctx_create", 0, C.byref(h))
+    return h
+
+def dense_map(ctx, rows, cols):
+    h = C.c_void_p()
+    L.call("skema_map_gauss_seeded", ctx, rows, cols, 1, L.DIST_NORMAL, 0, C.byref(h))
+    return h
+
+def sign_map(ctx, rows, cols, zeta=8):
+    h = C.c_void_p()
+    L.call("skema_map_sparse_sign_seeded", ctx, rows, cols, 1, L.SSIGN_COLS, zeta, 0, C.byref(h))
+    return h
+
+def sketch(ctx, m, n, k, s, sign=False, **more):
+    p = L.skema_params()
+    L.load().skema_params_default(C.byref(p))
+    p.m, p.n, p.rank, p.range, p.core, p.window = m, n, 2, k, s, m
+    p.dim_redux = L.MAP_SPARSE_SIGN if sign else L.MAP_GAUSS
+    for name, value in more.items():
+        setattr(p, name, value)
+    make = sign_map if sign else dense_map
+    maps = [make(ctx, *shape) for shape in ((k, m), (k, n), (s, m), (s, n))]
+    h = C.c_void_p()
+    L.call("skema_sketch_create", ctx, C.byref(p), *maps, C.byref(h))
+    return h
+
+def launched():
+    out = [line.rsplit(" ", 3) for line in rt.rt_launches().decode().splitlines()]
+    rt.rt_forget()
+    return [(name, tuple(map(int, grid))) for name, *grid in out]
+
+def names():
+    return [name for name, grid in launched()]
+
+def refused(name, *args):
+    try:
+        L.call(name, *args)
+    except L.SkemaError as e:
+        return e.code
+    return 0
+
+rt.rt_forget()
+"""
+
+
+@pytest.fixture(scope="module")
+def runtime(tmp_path_factory):
+    out = str(tmp_path_factory.mktemp("rt") / "libhostrt.so")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-o", out,
+                    os.path.join(ROOT, "tests", "host_runtime.cpp")], check=True, timeout=120)
+    return out
+
+
+def run(runtime, code):
+    r = subprocess.run([sys.executable, "-c", PRELUDE + code, runtime, ROOT], capture_output=True, text=True,
+                       timeout=300)
+    assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-4000:]
+
+
+def test_refused_window_leaves_nothing_on_the_stream(runtime):
+    """A refused window's call returns with its stream empty: the clearing of
+    the inspection's flags has no successor that would wait for it, and the next
+    call may come on another stream."""
+    run(runtime, r"""
+ctx = context()
+m, n = 300, 40
+sk = sketch(ctx, m, n, 9, 19)
+rowptr, col, val = device(m + 1), device(1000, 4), device(1000)
+stream = C.c_void_p(0x1000)
+L.call("skema_ctx_set_stream", ctx, stream)
+for flags in (1, 2, 3):
+    rt.rt_inspection(0, 1000, flags)
+    assert refused("skema_update_csr", sk, rowptr, col, val, 0, m) == 1
+    assert rt.rt_queued(stream) == 0, (flags, launched())
+rt.rt_inspection(0, 1000, 0)
+L.call("skema_update_csr", sk, rowptr, col, val, 0, m)
+""")
