@@ -39,7 +39,7 @@ void gemm_f64(hipStream_t stream, char transA, char transB, int64_t M, int64_t N
 // series of them, the operands stepA and stepB elements apart, can run in one:
 // each into its own output (stepC1, stepC2 apart), or as a chain, one after the
 // other into the same one.  Every product takes the order it would take alone.
-bool gemm_f64_one_pass(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb);
+bool gemm_f64_one_pass(char transB, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb);
 struct GemmSeries {
   int64_t count = 1, stepA = 0, stepB = 0, stepC1 = 0, stepC2 = 0;
   bool chain = false;

@@ -102,7 +102,9 @@ struct Slice {
 // Measured: 4096 x 1204 x 16384 (NT) 3.78 -> 2.64 ms (61 TF of the 78.6 TF
 // peak), 401 x 16384 x 4096 (NN) 1.35 -> 0.90 ms, 8192^3 69 TF; before, 64 x 64
 // tiles of 4 waves with two barriers per slice.
-template <int WM, int TM, int TN, bool TA, bool TB>
+// FAR: 64-bit offsets, for leading dimensions whose slices span 4 GiB or more
+// (near_enough below).
+template <int WM, int TM, int TN, bool TA, bool TB, bool FAR>
 __device__ __forceinline__ void wide_tile(const KArgs& g, double* lds, int64_t m0, int64_t n0, int64_t m1, int64_t n1,
                                           int64_t kbeg, int64_t kend, int split) {
   constexpr int RA = WM * TM * 16, RB = (8 / WM) * TN * 16;
@@ -113,20 +115,21 @@ __device__ __forceinline__ void wide_tile(const KArgs& g, double* lds, int64_t m
   const int l16 = lane & 15, lq = lane >> 4;
   const int wm = WM == 8 ? wave : 0, wn = WM == 8 ? 0 : wave;
 
-  uint32_t oa[SA::E], ob[SB::E];  // byte offsets from the slice's first element
+  using Off = std::conditional_t<FAR, uint64_t, uint32_t>;
+  Off oa[SA::E], ob[SB::E];  // byte offsets from the slice's first element
 #pragma unroll
   for (int e = 0; e < SA::E; ++e) {
     const int idx = SA::clip(tid + e * kWideThreads);
     const int64_t last = g.M - 1 - m0;
     const int64_t r = SA::r_of(idx) < last ? SA::r_of(idx) : last;
-    oa[e] = (uint32_t)((TA ? SA::k_of(idx) + r * g.lda : r + SA::k_of(idx) * g.lda) * 8);
+    oa[e] = (Off)((TA ? SA::k_of(idx) + r * g.lda : r + SA::k_of(idx) * g.lda) * 8);
   }
 #pragma unroll
   for (int e = 0; e < SB::E; ++e) {
     const int idx = SB::clip(tid + e * kWideThreads);
     const int64_t last = g.N - 1 - n0;
     const int64_t r = SB::r_of(idx) < last ? SB::r_of(idx) : last;
-    ob[e] = (uint32_t)((TB ? r + SB::k_of(idx) * g.ldb : SB::k_of(idx) + r * g.ldb) * 8);
+    ob[e] = (Off)((TB ? r + SB::k_of(idx) * g.ldb : SB::k_of(idx) + r * g.ldb) * 8);
   }
   const char* pa = reinterpret_cast<const char*>(g.A + (TA ? m0 * g.lda + kbeg : m0 + kbeg * g.lda));
   const char* pb = reinterpret_cast<const char*>(g.B + (TB ? n0 + kbeg * g.ldb : n0 * g.ldb + kbeg));
@@ -148,14 +151,14 @@ __device__ __forceinline__ void wide_tile(const KArgs& g, double* lds, int64_t m
 #pragma unroll
     for (int e = 0; e < SA::E; ++e) {
       const int k = SA::k_of(SA::clip(tid + e * kWideThreads));
-      const uint32_t back = k < left ? 0u : (uint32_t)(k * (TA ? 1 : g.lda) * 8);
+      const Off back = k < left ? 0 : (Off)(k * (TA ? 1 : g.lda) * 8);
       const double v = *reinterpret_cast<const double*>(qa + (oa[e] - back));
       ra[e] = k < left ? v : 0.0;
     }
 #pragma unroll
     for (int e = 0; e < SB::E; ++e) {
       const int k = SB::k_of(SB::clip(tid + e * kWideThreads));
-      const uint32_t back = k < left ? 0u : (uint32_t)(k * (TB ? g.ldb : 1) * 8);
+      const Off back = k < left ? 0 : (Off)(k * (TB ? g.ldb : 1) * 8);
       const double v = *reinterpret_cast<const double*>(qb + (ob[e] - back));
       rb[e] = k < left ? v : 0.0;
     }
@@ -302,7 +305,7 @@ __device__ __forceinline__ void wide_tile(const KArgs& g, double* lds, int64_t m
 // it each; all of them share the block's part of S, which is cut into tiles_s
 // nearly equal parts of at most TS MFMA tiles (401 rows are 7 + 7 + 6 + 6
 // tiles, not 8 + 8 + 8 + 2); a part below TS is multiplied as TS - 1 tiles.
-template <int WM, int TT, int TS, bool TA, bool TB>
+template <int WM, int TT, int TS, bool TA, bool TB, bool FAR>
 __global__ __launch_bounds__(kWideThreads) void k_gemm_wide(KArgs g) {
   constexpr int RT = 8 * TT * 16, RS = TS * 16;
   constexpr int SZ_T = WM == 8 ? Slice<TA, RT>::SIZE : Slice<!TB, RT>::SIZE;
@@ -318,13 +321,14 @@ __global__ __launch_bounds__(kWideThreads) void k_gemm_wide(KArgs g) {
   const int64_t e1 = s1 * 16;
   const int64_t m1 = WM == 8 || e1 > g.M ? g.M : e1, n1 = WM == 8 && e1 < g.N ? e1 : g.N;
   if constexpr (TS == 1) {
-    wide_tile<WM, WM == 8 ? TT : 1, WM == 8 ? 1 : TT, TA, TB>(g, lds, m0, n0, m1, n1, kbeg, kend, blockIdx.z);
+    wide_tile<WM, WM == 8 ? TT : 1, WM == 8 ? 1 : TT, TA, TB, FAR>(g, lds, m0, n0, m1, n1, kbeg, kend, blockIdx.z);
   } else {
     if (s1 - s0 == TS)
-      wide_tile<WM, WM == 8 ? TT : TS, WM == 8 ? TS : TT, TA, TB>(g, lds, m0, n0, m1, n1, kbeg, kend, blockIdx.z);
+      wide_tile<WM, WM == 8 ? TT : TS, WM == 8 ? TS : TT, TA, TB, FAR>(g, lds, m0, n0, m1, n1, kbeg, kend,
+                                                                      blockIdx.z);
     else
-      wide_tile<WM, WM == 8 ? TT : TS - 1, WM == 8 ? TS - 1 : TT, TA, TB>(g, lds, m0, n0, m1, n1, kbeg, kend,
-                                                                         blockIdx.z);
+      wide_tile<WM, WM == 8 ? TT : TS - 1, WM == 8 ? TS - 1 : TT, TA, TB, FAR>(g, lds, m0, n0, m1, n1, kbeg, kend,
+                                                                              blockIdx.z);
   }
 }
 
@@ -504,20 +508,21 @@ __global__ __launch_bounds__(256) void k_splitk_reduce(const double* part, int s
   }
 }
 
-template <int WM, int TT, int TS>
+template <int WM, int TT, int TS, bool FAR>
 void launch_wide_t(hipStream_t st, bool ta, bool tb, const KArgs& a, dim3 grid) {
-  if (!ta && !tb) hipLaunchKernelGGL((k_gemm_wide<WM, TT, TS, false, false>), grid, dim3(kWideThreads), 0, st, a);
-  else if (!ta && tb) hipLaunchKernelGGL((k_gemm_wide<WM, TT, TS, false, true>), grid, dim3(kWideThreads), 0, st, a);
-  else if (ta && !tb) hipLaunchKernelGGL((k_gemm_wide<WM, TT, TS, true, false>), grid, dim3(kWideThreads), 0, st, a);
-  else hipLaunchKernelGGL((k_gemm_wide<WM, TT, TS, true, true>), grid, dim3(kWideThreads), 0, st, a);
+  const dim3 block(kWideThreads);
+  if (!ta && !tb) hipLaunchKernelGGL((k_gemm_wide<WM, TT, TS, false, false, FAR>), grid, block, 0, st, a);
+  else if (!ta && tb) hipLaunchKernelGGL((k_gemm_wide<WM, TT, TS, false, true, FAR>), grid, block, 0, st, a);
+  else if (ta && !tb) hipLaunchKernelGGL((k_gemm_wide<WM, TT, TS, true, false, FAR>), grid, block, 0, st, a);
+  else hipLaunchKernelGGL((k_gemm_wide<WM, TT, TS, true, true, FAR>), grid, block, 0, st, a);
 }
-template <int WM, int TT>
+template <int WM, int TT, bool FAR>
 void launch_wide_s(hipStream_t st, bool ta, bool tb, const KArgs& a, dim3 grid, int ts) {
-  if (ts == 8) launch_wide_t<WM, TT, 8>(st, ta, tb, a, grid);
-  else if (ts >= 6) launch_wide_t<WM, TT, 7>(st, ta, tb, a, grid);
-  else if (ts >= 4) launch_wide_t<WM, TT, 5>(st, ta, tb, a, grid);
-  else if (ts >= 2) launch_wide_t<WM, TT, 3>(st, ta, tb, a, grid);
-  else launch_wide_t<WM, TT, 1>(st, ta, tb, a, grid);
+  if (ts == 8) launch_wide_t<WM, TT, 8, FAR>(st, ta, tb, a, grid);
+  else if (ts >= 6) launch_wide_t<WM, TT, 7, FAR>(st, ta, tb, a, grid);
+  else if (ts >= 4) launch_wide_t<WM, TT, 5, FAR>(st, ta, tb, a, grid);
+  else if (ts >= 2) launch_wide_t<WM, TT, 3, FAR>(st, ta, tb, a, grid);
+  else launch_wide_t<WM, TT, 1, FAR>(st, ta, tb, a, grid);
 }
 
 template <int KW>
@@ -537,7 +542,7 @@ void launch_series(hipStream_t st, bool tb, const KArgs& a, dim3 grid) {
 
 // One way to run a product, with its estimated time in CU cycles.
 struct Plan {
-  bool wide = false;
+  bool wide = false, far = false;
   int wm = 8;  // wide: waves along M (8) or N (1); else the block's waves
   int tt = 2, ts = 8, splits = 1;
   int64_t tiles_t = 1, tiles_s = 1;
@@ -547,10 +552,12 @@ struct Plan {
 // Estimated cycles of the wide kernel: rounds of 256 blocks, a slice costing
 // the most of its MFMA, LDS and L2 time, plus writing and reading the K
 // splits' partials at about 4 TB/s and the launch that adds them.
-void try_wide(Plan& best, int64_t M, int64_t N, int64_t K, bool may_split) {
+// far: the 64-bit form, built for TT = 2 only.
+void try_wide(Plan& best, int64_t M, int64_t N, int64_t K, bool may_split, bool far) {
   for (int wm : {8, 1}) {
     const int64_t T = wm == 8 ? M : N, ns = cdiv(wm == 8 ? N : M, 16);
     for (int tt : {2, 1}) {
+      if (far && tt == 1) continue;
       const int64_t tiles_t = cdiv(T, 128 * tt), tiles_s = cdiv(ns, 8);
       if (tiles_t * tiles_s >= (int64_t)1 << 31) continue;
       const int ts = (int)cdiv(ns, tiles_s);
@@ -564,7 +571,7 @@ void try_wide(Plan& best, int64_t M, int64_t N, int64_t K, bool may_split) {
         const double rounds = (double)cdiv(tiles_t * tiles_s * sp, kCUs);
         double cost = rounds * ((double)(per / kBK) * slice + 5000.0 + 40.0 * tt * ts);
         if (sp > 1) cost += 8000.0 + 16.0 * (double)sp * (double)M * (double)N / 1700.0;
-        if (cost < best.cost) best = Plan{true, wm, tt, ts, (int)sp, tiles_t, tiles_s, cost};
+        if (cost < best.cost) best = Plan{true, far, wm, tt, ts, (int)sp, tiles_t, tiles_s, cost};
       }
     }
   }
@@ -585,24 +592,36 @@ void try_ksplit(Plan& best, int64_t M, int64_t N, int64_t K, bool may_split) {
     const double rounds = (double)cdiv(blocks, kCUs), chunk = kw == 16 ? 4600.0 : blocks <= kCUs ? 3000.0 : 4500.0;
     double cost = rounds * ((double)cdiv(per, 16 * kw) * chunk + 4000.0);
     if (sp > 1) cost += 8000.0 + 16.0 * (double)sp * (double)M * (double)N / 1700.0;
-    if (cost < best.cost) best = Plan{false, kw, 1, 1, (int)sp, tm, tn, cost};
+    if (cost < best.cost) best = Plan{false, false, kw, 1, 1, (int)sp, tm, tn, cost};
   }
+}
+
+// Whether a slice of an operand spans less than 4 GiB, 32-bit byte offsets: up to
+// 256 rows ld apart where K is contiguous, 16 of K ld apart where the rows are.
+// Past that the 64-bit form, at the same speed: windows of 200000 rows of a
+// column-major 2200000 x 256 matrix, k = 201, s = 403 3.07 ms, as at 2000000 rows
+// (5.38 on the small kernel).
+bool near_enough(bool k_contiguous, int64_t ld) { return ld <= (int64_t)1 << (k_contiguous ? 21 : 25); }
+
+Plan choose(bool ta, bool tb, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, bool may_split) {
+  Plan p;
+  try_ksplit(p, M, N, K, may_split);
+  try_wide(p, M, N, K, may_split, !near_enough(ta, lda) || !near_enough(!tb, ldb));
+  return p;
 }
 
 }  // namespace
 
-bool gemm_f64_one_pass(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb) {
+bool gemm_f64_one_pass(char transB, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb) {
   if (M <= 0 || N <= 0 || K <= 0) return false;
-  Plan p;
-  try_ksplit(p, M, N, K, true);
-  if (lda <= (int64_t)1 << 21 && ldb <= (int64_t)1 << 21) try_wide(p, M, N, K, true);
+  const Plan p = choose(false, transB == 'T' || transB == 't', M, N, K, lda, ldb, true);
   return p.cost < 1e300 && !p.wide && p.splits == 1;
 }
 
 void gemm_f64_series(hipStream_t stream, char transB, int64_t M, int64_t N, int64_t K, const double* A,
                      int64_t lda, const double* B, int64_t ldb, const GemmOut& out, const GemmSeries& sr) {
   const bool tb = (transB == 'T' || transB == 't');
-  SKEMA_REQUIRE(gemm_f64_one_pass(M, N, K, lda, ldb) && sr.count > 0 && (sr.chain || sr.count <= 65535), kErrShape,
+  SKEMA_REQUIRE(gemm_f64_one_pass(transB, M, N, K, lda, ldb) && sr.count > 0 && (sr.chain || sr.count <= 65535), kErrShape,
                 "gemm_f64_series: not products of one pass");
   SKEMA_REQUIRE(lda >= M && ldb >= (tb ? N : K), kErrShape, "gemm_f64_series: leading dimension too small");
   Plan p;
@@ -634,10 +653,7 @@ void gemm_f64(hipStream_t stream, char transA, char transB, int64_t M, int64_t N
   SKEMA_REQUIRE(out.nsplit == N || out.ldc2 >= M, kErrShape, "gemm_f64: ldc too small");
   SKEMA_REQUIRE(M * N < (int64_t)1 << 40, kErrShape, "gemm_f64: output too large");
 
-  Plan p;
-  try_ksplit(p, M, N, K, ws != nullptr);
-  // the wide kernel's element offsets within a slice are 32-bit byte offsets
-  if (lda <= (int64_t)1 << 21 && ldb <= (int64_t)1 << 21) try_wide(p, M, N, K, ws != nullptr);
+  const Plan p = choose(ta, tb, M, N, K, lda, ldb, ws != nullptr);
   SKEMA_REQUIRE(p.cost < 1e300, kErrShape, "gemm_f64: too many tiles");
 
   KArgs a;
@@ -651,10 +667,12 @@ void gemm_f64(hipStream_t stream, char transA, char transB, int64_t M, int64_t N
   }
   dim3 grid((unsigned)(p.tiles_t * p.tiles_s), 1, (unsigned)p.splits);
   if (p.wide) {
-    if (p.wm == 8 && p.tt == 2) launch_wide_s<8, 2>(stream, ta, tb, a, grid, p.ts);
-    else if (p.wm == 8) launch_wide_s<8, 1>(stream, ta, tb, a, grid, p.ts);
-    else if (p.tt == 2) launch_wide_s<1, 2>(stream, ta, tb, a, grid, p.ts);
-    else launch_wide_s<1, 1>(stream, ta, tb, a, grid, p.ts);
+    if (p.far && p.wm == 8) launch_wide_s<8, 2, true>(stream, ta, tb, a, grid, p.ts);
+    else if (p.far) launch_wide_s<1, 2, true>(stream, ta, tb, a, grid, p.ts);
+    else if (p.wm == 8 && p.tt == 2) launch_wide_s<8, 2, false>(stream, ta, tb, a, grid, p.ts);
+    else if (p.wm == 8) launch_wide_s<8, 1, false>(stream, ta, tb, a, grid, p.ts);
+    else if (p.tt == 2) launch_wide_s<1, 2, false>(stream, ta, tb, a, grid, p.ts);
+    else launch_wide_s<1, 1, false>(stream, ta, tb, a, grid, p.ts);
     check_launch("k_gemm_wide");
   } else {
     if (p.wm == 16) launch_ksplit<16>(stream, ta, tb, a, grid);

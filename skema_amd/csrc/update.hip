@@ -196,8 +196,8 @@ void update_dense_window(Sketch& sk, const double* H, int64_t ldh, int64_t row0,
 int64_t update_dense_windows(Sketch& sk, const double* H, int64_t ldh, int64_t row0, int64_t w, int64_t count) {
   const int64_t k = sk.k, s = sk.s, m = sk.p.m, n = sk.p.n;
   if (sk.sparse_maps || sk.p.precision != SKEMA_PREC_FP64 || count < 2) return 0;
-  if (!gemm_f64_one_pass(k, n, w, sk.ldups, ldh) || !gemm_f64_one_pass(w, k + s, n, ldh, k + s) ||
-      !gemm_f64_one_pass(s, s, w, sk.ldphi, w))
+  if (!gemm_f64_one_pass('N', k, n, w, sk.ldups, ldh) || !gemm_f64_one_pass('T', w, k + s, n, ldh, k + s) ||
+      !gemm_f64_one_pass('N', s, s, w, sk.ldphi, w))
     return 0;
   count = std::min<int64_t>({count, ((int64_t)128 << 20) / (w * (n + s) * 8), (int64_t)65535});
   if (count < 2) return 0;

@@ -92,3 +92,29 @@ def test_grouped_windows_equal_single_ones(S, m, n, w, k, s, nu):
         parts.update(A, (r0, min(m, r0 + w)))
     for a, b in zip(whole.state(), parts.state()):
         assert np.array_equal(a, b)
+
+
+# Operand slices just within 4 GiB (32-bit offsets) and just past it (64-bit):
+# 256 rows 2^21 apart where K is contiguous, 16 of K 2^25 apart where the rows are.
+@pytest.mark.parametrize("side,trans,M,N,K,ld", [
+    ("B", "N", 2000, 300, 1003, 1 << 21), ("B", "N", 2000, 300, 1003, (1 << 21) + 3),
+    ("A", "T", 301, 3000, 1003, 1 << 21), ("A", "T", 301, 3000, 1003, (1 << 21) + 3),
+    ("A", "N", 401, 3000, 43, 1 << 25), ("A", "N", 4001, 4003, 43, (1 << 25) + 3),
+    ("B", "T", 401, 3000, 43, 1 << 25), ("B", "T", 4001, 4003, 43, (1 << 25) + 3)])
+def test_leading_dimensions_around_32_bit_slices(S, side, trans, M, N, K, ld):
+    print(f"case gemm ld={ld} {side}{trans} {M}x{N}x{K}", flush=True)
+    rng = np.random.default_rng(K)
+    A, B = rng.standard_normal((M, K)), rng.standard_normal((K, N))
+    far = A if side == "A" else B
+    far = far if trans == "N" else far.T
+    rows, cols = far.shape
+    buf = torch.empty(ld * (cols - 1) + rows, dtype=torch.float64, device="cuda")
+    X = buf.as_strided((rows, cols), (1, ld))
+    X.copy_(torch.as_tensor(far, device="cuda"))
+    out = dev(np.full((M, N), np.nan))
+    if side == "A":
+        S.GaussDimRedux(K, N, data=B).rmap(1.0, X, 0.0, trans, "N", C_out=out)
+    else:
+        S.GaussDimRedux(M, K, data=A).lmap(1.0, X, 0.0, "N", trans, C_out=out)
+    want = A @ B
+    assert np.linalg.norm(host(out) - want) <= TOL * np.linalg.norm(want)

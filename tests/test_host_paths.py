@@ -112,3 +112,22 @@ for flags in (1, 2, 3):
 rt.rt_inspection(0, 1000, 0)
 L.call("skema_update_csr", sk, rowptr, col, val, 0, m)
 """)
+
+
+@pytest.mark.parametrize("transB", ["N", "T"])
+@pytest.mark.parametrize("ld", [5000, (1 << 21) + 3, (1 << 25) + 3])
+def test_large_products_take_the_wide_kernel_at_any_leading_dimension(runtime, transB, ld):
+    """With 32-bit offsets where the operand's slices allow them (rows of the
+    operand contiguous: up to 2^25), 64-bit ones past that."""
+    run(runtime, rf"""
+ctx = context()
+M, N, K, ld, tb = 800, 4000, 1000, {ld}, {transB!r}
+mp, out = dense_map(ctx, M, K), device(M * N)
+rows, cols = (K, N) if tb == "N" else (N, K)
+B = device(ld * (cols - 1) + rows)
+rt.rt_forget()
+L.call("skema_map_lmap", mp, 1.0, B, rows, cols, ld, 0.0, b"N", tb.encode(), 0, 0, out, M)
+wide = [n for n in names() if "k_gemm_wide" in n]
+far = ld > 1 << (25 if tb == "T" else 21)
+assert len(wide) == 1 and ("ELb1EEEv" in wide[0]) == far, wide
+""")
