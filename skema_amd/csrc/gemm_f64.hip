@@ -14,10 +14,11 @@
 //
 // Two kernels.  k_gemm_wide: one 8-wave block per CU on a 256 x 128 tile, for
 // products with enough tiles (or K to split) to fill the chip.
-// k_gemm_ksplit: 32 x 32 tiles whose 8 or 16 waves split K, for small products.
+// k_gemm_ksplit: 32 x 32 tiles whose 2, 8 or 16 waves split K, for small products.
 #include "gemm.hpp"
 
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 namespace skema {
@@ -402,7 +403,7 @@ __global__ __launch_bounds__(64 * KW) void k_gemm_ksplit(KArgs g) {
         for (int y = 0; y < 2; ++y)
           acc[x][y] = __builtin_amdgcn_mfma_f64_16x16x4f64(f.b[y][kk], f.a[x][kk], acc[x][y], 0, 0, 0);
   };
-  // this wave's whole chunks: wave, wave + 8, ...
+  // this wave's whole chunks: wave, wave + KW, ...
   const int64_t full = (kend - kbeg) / 16;
   const int left = (int)((kend - kbeg) % 16);
   Frags f0, f1;
@@ -553,6 +554,11 @@ struct Plan {
 // the most of its MFMA, LDS and L2 time, plus writing and reading the K
 // splits' partials at about 4 TB/s and the launch that adds them.
 // far: the 64-bit form, built for TT = 2 only.
+// K of at most kShortK: the rounds' stores run beside the products of other
+// blocks and bound most of these, at 1785 B a cycle; blocks whose waves hold 128
+// rows of a column (WM = 1, TT = 1) write the longest runs.  14919 x 3410 x 6
+// takes 115 us with those, 121 with WM = 8, 158 with TT = 2 and 203 with both.
+constexpr int64_t kShortK = 128;
 void try_wide(Plan& best, int64_t M, int64_t N, int64_t K, bool may_split, bool far) {
   for (int wm : {8, 1}) {
     const int64_t T = wm == 8 ? M : N, ns = cdiv(wm == 8 ? N : M, 16);
@@ -563,6 +569,14 @@ void try_wide(Plan& best, int64_t M, int64_t N, int64_t K, bool may_split, bool 
       const int ts = (int)cdiv(ns, tiles_s);
       const double rows = 128.0 * tt + 16.0 * ts;
       const double slice = 600.0 + std::max({512.0 * tt * ts, 128.0 * (tt + ts) + rows, rows * 128.0 / 12.0});
+      if (K <= kShortK) {
+        const double out = (double)M * (double)N * 8.0 / 1785.0;
+        const double runs = tt == 1 ? (wm == 1 ? 1.0 : 1.05) : (wm == 1 ? 1.1 : 1.4);
+        const double cost = (double)cdiv(tiles_t * tiles_s, kCUs) * (double)cdiv(K, kBK) * slice + 5000.0 +
+                            std::max(40.0 * tt * ts, out * runs);
+        if (cost < best.cost) best = Plan{true, far, wm, tt, ts, 1, tiles_t, tiles_s, cost};
+        continue;
+      }
       const int64_t most = may_split ? std::max<int64_t>(1, std::min<int64_t>(128, K / 64)) : 1;
       for (int64_t sp = 1; sp <= most; ++sp) {
         const int64_t per = cdiv(cdiv(K, sp), kBK) * kBK;
@@ -580,9 +594,24 @@ void try_wide(Plan& best, int64_t M, int64_t N, int64_t K, bool may_split, bool 
 // block per CU and 8 otherwise.  A block's chunks (16 of K for each of its
 // waves) are bound by the latency of their loads, by its MFMAs (1024 cycles per
 // 4 waves) or, with more than one block per CU, by the loads' L1 traffic.
-void try_ksplit(Plan& best, int64_t M, int64_t N, int64_t K, bool may_split) {
+// K of at most kShortK gives a wave one chunk or none, and several blocks run on
+// a CU at once: 2 waves a block there, or 8 while their blocks are few.  Measured,
+// before (wide or 8 waves) and after: 694 x 454 x 32 12.7 -> 6.9 us, 439 x 1788 x 76
+// 18 -> 9.9, 1457 x 5553 x 14 36 -> 28 (with the wide kernel's rule above).
+// From 8192 of K on, both operands contiguous along K (TN) ask for them in
+// half lines, at 2700 B a cycle once 32 tiles do so: 403 x 403 x 20000 is 278 us
+// of that, and 164 on the wide kernel.
+void try_ksplit(Plan& best, bool tn_form, int64_t M, int64_t N, int64_t K, bool may_split) {
   const int64_t tm = cdiv(M, 32), tn = cdiv(N, 32);
   if (tm * tn >= (int64_t)1 << 31) return;
+  if (K <= kShortK) {
+    const double t = (double)(tm * tn) / kCUs, k16 = (double)cdiv(K, kBK);
+    const double eight = std::max(7000.0, t * (2570.0 + 330.0 * k16));
+    const double two = std::max(6000.0 + 1000.0 * std::ceil(k16 / 2), t * (1170.0 + 540.0 * k16));
+    if (eight < best.cost) best = Plan{false, false, 8, 1, 1, 1, tm, tn, eight};
+    if (two < best.cost) best = Plan{false, false, 2, 1, 1, 1, tm, tn, two};
+    return;
+  }
   const int64_t most = may_split ? std::max<int64_t>(1, std::min<int64_t>(64, K / 512)) : 1;
   for (int64_t sp = 1; sp <= most; ++sp) {
     const int64_t per = cdiv(cdiv(K, sp), kBK) * kBK;
@@ -591,6 +620,7 @@ void try_ksplit(Plan& best, int64_t M, int64_t N, int64_t K, bool may_split) {
     const int kw = blocks <= kCUs && per > 16 * 8 ? 16 : 8;
     const double rounds = (double)cdiv(blocks, kCUs), chunk = kw == 16 ? 4600.0 : blocks <= kCUs ? 3000.0 : 4500.0;
     double cost = rounds * ((double)cdiv(per, 16 * kw) * chunk + 4000.0);
+    if (tn_form && kw == 16 && K >= 8192 && tm * tn >= 32) cost = std::max(cost, (double)(tm * tn) * (double)K * 512.0 / 2700.0);
     if (sp > 1) cost += 8000.0 + 16.0 * (double)sp * (double)M * (double)N / 1700.0;
     if (cost < best.cost) best = Plan{false, false, kw, 1, 1, (int)sp, tm, tn, cost};
   }
@@ -605,7 +635,7 @@ bool near_enough(bool k_contiguous, int64_t ld) { return ld <= (int64_t)1 << (k_
 
 Plan choose(bool ta, bool tb, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, bool may_split) {
   Plan p;
-  try_ksplit(p, M, N, K, may_split);
+  try_ksplit(p, ta && !tb, M, N, K, may_split);
   try_wide(p, M, N, K, may_split, !near_enough(ta, lda) || !near_enough(!tb, ldb));
   return p;
 }
@@ -625,7 +655,7 @@ void gemm_f64_series(hipStream_t stream, char transB, int64_t M, int64_t N, int6
                 "gemm_f64_series: not products of one pass");
   SKEMA_REQUIRE(lda >= M && ldb >= (tb ? N : K), kErrShape, "gemm_f64_series: leading dimension too small");
   Plan p;
-  try_ksplit(p, M, N, K, true);
+  try_ksplit(p, false, M, N, K, true);
   KArgs a;
   a.M = M; a.N = N; a.K = K; a.A = A; a.lda = lda; a.B = B; a.ldb = ldb; a.out = out;
   a.tiles_t = (int)p.tiles_t; a.tiles_s = (int)p.tiles_s;
@@ -635,6 +665,7 @@ void gemm_f64_series(hipStream_t stream, char transB, int64_t M, int64_t N, int6
   a.chain = sr.chain ? (int)sr.count : 1;
   const dim3 grid((unsigned)(p.tiles_t * p.tiles_s), sr.chain ? 1u : (unsigned)sr.count, 1);
   if (p.wm == 16) launch_series<16>(stream, tb, a, grid);
+  else if (p.wm == 2) launch_series<2>(stream, tb, a, grid);
   else launch_series<8>(stream, tb, a, grid);
   check_launch("k_gemm_ksplit (series)");
 }
@@ -676,6 +707,7 @@ void gemm_f64(hipStream_t stream, char transA, char transB, int64_t M, int64_t N
     check_launch("k_gemm_wide");
   } else {
     if (p.wm == 16) launch_ksplit<16>(stream, ta, tb, a, grid);
+    else if (p.wm == 2) launch_ksplit<2>(stream, ta, tb, a, grid);
     else launch_ksplit<8>(stream, ta, tb, a, grid);
     check_launch("k_gemm_ksplit");
   }

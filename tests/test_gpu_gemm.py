@@ -118,3 +118,19 @@ def test_leading_dimensions_around_32_bit_slices(S, side, trans, M, N, K, ld):
         S.GaussDimRedux(M, K, data=A).lmap(1.0, X, 0.0, "N", trans, C_out=out)
     want = A @ B
     assert np.linalg.norm(host(out) - want) <= TOL * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("K", [1, 15, 16, 17, 32, 33, 65, 127, 128])
+@pytest.mark.parametrize("trans", ["NN", "TN", "NT", "TT"])
+def test_short_k(S, trans, K):
+    """Enough 32 x 32 tiles for the blocks of two waves, whose K loop ends within
+    either wave's first chunks, and the wide kernel's large outputs."""
+    for M, N in ((1999, 1001), (4111, 3300)):
+        print(f"case gemm short K {M}x{N}x{K} {trans}", flush=True)
+        rng = np.random.default_rng(M + K)
+        A, B = rng.standard_normal((M, K)), rng.standard_normal((K, N))
+        mp = S.GaussDimRedux(*(A if trans[0] == "N" else A.T).shape, data=A if trans[0] == "N" else A.T)
+        out = dev(np.full((M, N), np.nan))
+        mp.lmap(1.0, dev(B if trans[1] == "N" else B.T), 0.0, trans[0], trans[1], C_out=out)
+        want = A @ B
+        assert np.linalg.norm(host(out) - want) <= TOL * np.linalg.norm(want)

@@ -131,3 +131,21 @@ wide = [n for n in names() if "k_gemm_wide" in n]
 far = ld > 1 << (25 if tb == "T" else 21)
 assert len(wide) == 1 and ("ELb1EEEv" in wide[0]) == far, wide
 """)
+
+
+@pytest.mark.parametrize("M,N,K,kernel", [
+    (694, 454, 32, "k_gemm_ksplitILi8E"),      # few tiles: their K loop's latency
+    (1950, 449, 45, "k_gemm_ksplitILi2E"),     # many small ones: their rate
+    (1601, 14345, 46, "k_gemm_wideILi1ELi1E"), # bound by its stores
+    (100, 3000, 129, "k_gemm_ksplitILi8E"),    # past the short ones
+])
+def test_products_with_short_k_take_the_kernel_that_measured_fastest(runtime, M, N, K, kernel):
+    run(runtime, rf"""
+ctx = context()
+M, N, K = {M}, {N}, {K}
+mp, B, out = dense_map(ctx, M, K), device(K * N), device(M * N)
+rt.rt_forget()
+L.call("skema_map_lmap", mp, 1.0, B, K, N, K, 0.0, b"N", b"N", 0, 0, out, M)
+got = names()
+assert len(got) == 1 and {kernel!r} in got[0], got
+""")
