@@ -394,25 +394,28 @@ __global__ void k_csc_left_sparse(const int64_t* ptr, const int32_t* row, const 
   }
 }
 
-// out(i, p) = sum over row i's entries (j, a) of a M(p, j): 16 rows and 64 PR
-// map rows p a block, each wave four rows one after another (entries in order,
-// four and their map columns in flight), then through LDS so that a column of
-// the output is written 16 rows (128 bytes) at a time.  One thread per output
-// with p fastest wrote every 8 bytes to a line of its own: 4096 x 304 outputs
-// with 15 entries a row took 48 us, 24 here.
-constexpr int kRightTile = 16;
-template <int PR>
+// out(i, p) = sum over row i's entries (j, a) of a M(p, j): RT rows and LP PR
+// map rows p a block.  A row is taken by LP lanes of a wave (16 or 32 where there
+// are no more map rows, so that a wave has four or two rows at once), a wave's
+// rows one after another (entries in order, four and their map columns in flight),
+// then through LDS so that a column of the output is written RT rows at a time
+// (16: 128 bytes).  One thread per output with p fastest wrote every 8 bytes to a
+// line of its own: 4096 x 304 outputs with 15 entries a row took 48 us, 24 here.
+template <int PR, int RT, int LP>
 __global__ __launch_bounds__(256) void k_csr_right_dense(const int64_t* __restrict__ rowptr, const int32_t* __restrict__ col,
                                                          const double* __restrict__ val, int64_t rows,
                                                          const double* __restrict__ M, int64_t ldm, int64_t kk, GemmOut o) {
-  __shared__ double tile[64 * PR][kRightTile + 1];
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int64_t r0 = (int64_t)blockIdx.x * kRightTile, p0 = (int64_t)blockIdx.y * (64 * PR);
+  constexpr int AT = 256 / LP;  // rows at a time
+  static_assert(RT % AT == 0, "whole passes");
+  __shared__ double tile[LP * PR][RT + 1];
+  const int tid = threadIdx.x, lane = tid % LP;
+  const int own = LP == 64 ? __builtin_amdgcn_readfirstlane(tid / 64) : tid / LP;
+  const int64_t r0 = (int64_t)blockIdx.x * RT, p0 = (int64_t)blockIdx.y * (LP * PR);
   int64_t at[PR];
 #pragma unroll
-  for (int r = 0; r < PR; ++r) at[r] = p0 + lane + 64 * r < kk ? p0 + lane + 64 * r : kk - 1;
-  for (int q = 0; q < kRightTile / 4; ++q) {
-    const int64_t i = r0 + 4 * q + wave;
+  for (int r = 0; r < PR; ++r) at[r] = p0 + lane + LP * r < kk ? p0 + lane + LP * r : kk - 1;
+  for (int q = 0; q < RT / AT; ++q) {
+    const int64_t i = r0 + AT * q + own;
     if (i >= rows) break;
     const int64_t lo = rowptr[i], hi = rowptr[i + 1];
     double acc[PR];
@@ -443,11 +446,11 @@ __global__ __launch_bounds__(256) void k_csr_right_dense(const int64_t* __restri
       for (int r = 0; r < PR; ++r) acc[r] += a * m[at[r]];
     }
 #pragma unroll
-    for (int r = 0; r < PR; ++r) tile[lane + 64 * r][4 * q + wave] = acc[r];
+    for (int r = 0; r < PR; ++r) tile[lane + LP * r][AT * q + own] = acc[r];
   }
   __syncthreads();
-  for (int x = tid; x < 64 * PR * kRightTile; x += 256) {
-    const int ii = x % kRightTile, pp = x / kRightTile;
+  for (int x = tid; x < LP * PR * RT; x += 256) {
+    const int ii = x % RT, pp = x / RT;
     if (r0 + ii < rows && p0 + pp < kk) put(o, r0 + ii, p0 + pp, tile[pp][ii]);
   }
 }
@@ -639,15 +642,30 @@ void csc_left_sparse(hipStream_t st, const CscWindow& H, const Csr& Mt, int64_t 
 void csr_right_dense(hipStream_t st, const int64_t* rowptr, const int32_t* col, const double* val, int64_t rows,
                      const double* M, int64_t ldm, int64_t kk, const GemmOut& out) {
   if (rows == 0 || kk == 0) return;
-  const int pr = (int)std::min<int64_t>(5, cdiv(kk, (int64_t)64));  // 5: the 304 rows of a rank-25 [Omega; Psi]
-  const dim3 grid(blocks_for(rows, kRightTile), (unsigned)cdiv(kk, (int64_t)64 * pr));
-#define SKEMA_RIGHT(PR) \
-  hipLaunchKernelGGL(k_csr_right_dense<PR>, grid, dim3(256), 0, st, rowptr, col, val, rows, M, ldm, kk, out)
-  if (pr == 1) SKEMA_RIGHT(1);
-  else if (pr == 2) SKEMA_RIGHT(2);
-  else if (pr == 3) SKEMA_RIGHT(3);
-  else if (pr == 4) SKEMA_RIGHT(4);
-  else SKEMA_RIGHT(5);
+  // Map rows in equal parts of at most 320 (five a lane: 44 KB of LDS, three blocks a
+  // CU; 328 rows as 3 + 3 lots of 64, not 5 + 1), unless that leaves CUs without a
+  // block: then 64 a block, and 4 rows a block instead of 16 where it still does.
+  // Whole calls on windows with 300 entries a row, always 16 rows and all parts a
+  // block -> so (one thread per output): 64 rows, 197 map rows 226 -> 73 us (143);
+  // 1000 rows, 304 map rows 264 -> 200 (226).  Up to 32 map rows, a wave a row ->
+  // several rows a wave: 60000 rows of 50, 9 map rows 148 -> 102 us (139).
+  const int64_t parts = cdiv(kk, (int64_t)320), tall = cdiv(rows, (int64_t)16);
+  int pr = (int)cdiv(cdiv(kk, (int64_t)64), parts);
+  if (tall * parts < 256) pr = 1;
+  const int64_t ny = cdiv(kk, (int64_t)64 * pr);
+  const bool few = tall * ny < 256;
+#define SKEMA_RIGHT(PR, RT, LP)                                                                                   \
+  hipLaunchKernelGGL((k_csr_right_dense<PR, RT, LP>), dim3(blocks_for(rows, RT), (unsigned)ny), dim3(256), 0, st, \
+                     rowptr, col, val, rows, M, ldm, kk, out)
+  if (kk <= 16) SKEMA_RIGHT(1, 16, 16);
+  else if (kk <= 32 && few) SKEMA_RIGHT(1, 8, 32);
+  else if (kk <= 32) SKEMA_RIGHT(1, 16, 32);
+  else if (few) SKEMA_RIGHT(1, 4, 64);
+  else if (pr == 1) SKEMA_RIGHT(1, 16, 64);
+  else if (pr == 2) SKEMA_RIGHT(2, 16, 64);
+  else if (pr == 3) SKEMA_RIGHT(3, 16, 64);
+  else if (pr == 4) SKEMA_RIGHT(4, 16, 64);
+  else SKEMA_RIGHT(5, 16, 64);
 #undef SKEMA_RIGHT
   check_launch("k_csr_right_dense");
 }

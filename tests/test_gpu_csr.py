@@ -1,5 +1,7 @@
 """GPU checks of the CSR kernels with dense maps at their tile edges, and of
 the window inspection, against the oracle."""
+import functools
+
 import numpy as np
 import pytest
 import scipy.sparse as sp
@@ -99,3 +101,25 @@ def test_csr_sign_maps(S, m, n, k, s, density, window, conv):
     g.linear_update(S.CrsMatrix.from_scipy(A))
     for a, b in zip(g.state(), (osk.X, osk.Y, osk.Z)):
         assert O.rel_err(a, b) <= TOL
+
+
+@functools.lru_cache(maxsize=None)
+def _shared_matrix(m, density):
+    return _matrix(m, m, density, m)
+
+
+# Map rows up to 16 and 32 (several rows a wave), 64 a block, one part of two to
+# five times 64 and two equal parts; windows of a few rows, of a last ragged tile of
+# 4, 8 and 16, and long enough for the wider blocks; entries in groups of four.
+@pytest.mark.parametrize("k", [1, 16, 17, 32, 33, 64, 129, 320, 321, 390])
+@pytest.mark.parametrize("m,rows,density", [(400, 3, 0.05), (1300, 1299, 0.01), (9000, 8501, 0.001)])
+def test_csr_rows_times_dense_map(S, m, rows, density, k):
+    print(f"case csr rows {rows} of {m} k={k}", flush=True)
+    A = _shared_matrix(m, density)
+    om = S.GaussDimRedux(m, k, seed=3, dist="normal")
+    g = S.SketchySPD(S.AlgParams(matrix_m=m, matrix_n=m, rank=1, sketch_range=k, window=rows, issparse=True), omega=om)
+    Ad = S.CrsMatrix.from_scipy(A)
+    g.update(Ad, (m - rows, m))
+    want = A[m - rows:] @ om.download()
+    got = g.state()
+    assert O.rel_err(got[m - rows:], want) <= TOL and not got[:m - rows].any()

@@ -149,3 +149,27 @@ L.call("skema_map_lmap", mp, 1.0, B, K, N, K, 0.0, b"N", b"N", 0, 0, out, M)
 got = names()
 assert len(got) == 1 and {kernel!r} in got[0], got
 """)
+
+
+@pytest.mark.parametrize("rows,k,kernel,grid", [
+    (64, 197, "ILi1ELi4ELi64E", (16, 4, 1)),      # too few blocks of 16 rows: 4 rows and 64 map rows a block
+    (1000, 304, "ILi1ELi16ELi64E", (63, 5, 1)),   # 64 map rows a block are enough
+    (20000, 304, "ILi5ELi16ELi64E", (1250, 1, 1)),
+    (20000, 328, "ILi3ELi16ELi64E", (1250, 2, 1)),  # equal parts
+    (20000, 9, "ILi1ELi16ELi16E", (1250, 1, 1)),    # four rows a wave
+])
+def test_csr_row_product_splits(runtime, rows, k, kernel, grid):
+    run(runtime, rf"""
+ctx = context()
+m, rows, k = 30000, {rows}, {k}
+p = L.skema_params()
+L.load().skema_params_default(C.byref(p))
+p.m, p.n, p.rank, p.range, p.window, p.issparse = m, m, 1, k, rows, 1
+sp = C.c_void_p()
+L.call("skema_spd_create", ctx, C.byref(p), dense_map(ctx, m, k), C.byref(sp))
+rowptr, col, val = device(m + 1), device(1000, 4), device(1000)
+rt.rt_forget()
+L.call("skema_spd_update_csr", sp, rowptr, col, val, 0, rows)
+got = [(n, g) for n, g in launched() if "k_csr_right_dense" in n]
+assert len(got) == 1 and {kernel!r} in got[0][0] and got[0][1] == {grid!r}, got
+""")
