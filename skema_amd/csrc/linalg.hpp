@@ -38,14 +38,24 @@ bool thin_qr_products(hipStream_t st, int64_t m, int64_t n, double* A, int64_t l
 // R (n x n, upper, zero below) from the factored A.
 void extract_r(hipStream_t st, int64_t n, const double* A, int64_t lda, double* R, int64_t ldr);
 
+// Whether the panel products take less time than the column by column form: not
+// for a few columns, where their five launches and the wait for their flag cost
+// more than a launch a column, or, up to 1024 rows, one launch for all columns,
+// whose time grows with the rows.  The factors of a 5000 x 300 sketch by products
+// -> column by column: range 1 791 -> 423 us, range 5 964 -> 728, range 8
+// 1158 -> 976; range 9 983 by products.
+inline bool panel_products_pay(int64_t m, int64_t n) { return n > 8 || (m > 512 && m <= 1024) || m > 32768; }
+
 // The same for any A: `load` writes the matrix into A (again, to be factored
 // with householder_qr, where the products gave up).  tau: n entries of scratch.
 template <class Load>
 void thin_qr(hipStream_t st, int64_t m, int64_t n, double* A, int64_t lda, double* Q, int64_t ldq, double* R, int64_t ldr,
              double* tau, DevBuf* work, GemmWorkspace* gws, Load&& load) {
   load();
-  if (thin_qr_products(st, m, n, A, lda, Q, ldq, R, ldr, work, gws)) return;
-  load();
+  if (panel_products_pay(m, n)) {
+    if (thin_qr_products(st, m, n, A, lda, Q, ldq, R, ldr, work, gws)) return;
+    load();
+  }
   householder_qr(st, m, n, A, lda, tau, work, gws);
   if (R) extract_r(st, n, A, lda, R, ldr);
   householder_q(st, m, n, A, lda, Q, ldq, work, gws);

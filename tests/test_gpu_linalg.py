@@ -89,3 +89,24 @@ def test_thin_qr_panels(S, m, n, k, decay, true_rank):
     if true_rank:
         Ua, Va = O.align_signs(U, V, Ur, Vr)
         assert O.rel_err(Ua * Sv, Ur * Sr) <= TOL and O.rel_err(Va * Sv, Vr * Sr) <= TOL
+
+
+# Few columns: column by column up to 512 rows, above 1024 and up to 32768, by
+# products between and beyond; the core's own factors have 2 k + 1 rows.
+@pytest.mark.parametrize("k", [2, 5, 8])
+@pytest.mark.parametrize("m,n", [(60, 50), (900, 520), (1500, 300), (33000, 40)])
+def test_low_rank_approx_of_a_few_columns(S, m, n, k):
+    print(f"case low_rank_approx {m}x{n} k={k}", flush=True)
+    rng = np.random.default_rng(m + k)
+    A = (rng.standard_normal((m, 30)) * 0.5 ** np.arange(30)) @ rng.standard_normal((30, n)) / np.sqrt(m)
+    p = O.AlgParams(matrix_m=m, matrix_n=n, rank=2, sketch_range=k, sketch_core=2 * k + 1, window=m)
+    osk = O.SketchySVD(p)
+    osk.linear_update(A)
+    Ur, Sr, Vr = osk.low_rank_approx()
+    g = S.SketchySVD(to_gpu_params(p), maps=gpu_maps({"Upsilon": osk.Upsilon, "Omega": osk.Omega, "Phi": osk.Phi,
+                                                      "Psi": osk.Psi}))
+    g.linear_update(dev(A))
+    U, Sv, V = g.low_rank_approx()
+    for name in ("Q", "P", "T1", "T2"):
+        assert O.rel_err(g.checkpoint(name), osk.checkpoints[name]) <= TOL, name
+    assert np.abs(Sv - Sr).max() <= TOL * Sr[0]

@@ -173,3 +173,18 @@ L.call("skema_spd_update_csr", sp, rowptr, col, val, 0, rows)
 got = [(n, g) for n, g in launched() if "k_csr_right_dense" in n]
 assert len(got) == 1 and {kernel!r} in got[0][0] and got[0][1] == {grid!r}, got
 """)
+
+
+@pytest.mark.parametrize("m,k,products", [(5000, 5, False), (5000, 9, True), (300, 8, False), (1000, 5, True),
+                                          (100000, 5, True)])
+def test_a_few_columns_are_factored_one_by_one(runtime, m, k, products):
+    run(runtime, rf"""
+ctx = context()
+m, k = {m}, {k}
+sk = sketch(ctx, m, 200, k, 2 * k + 1)
+U, S, V = device(2 * m), device(2), device(2 * 200)
+rt.rt_forget()
+L.call("skema_low_rank_approx_device", sk, U, m, S, V, 200)
+used = [n for n in names() if "k_panel_mul" in n]
+assert bool(used) == {products}, used
+""")
