@@ -30,8 +30,8 @@ void householder_q(hipStream_t st, int64_t m, int64_t n, const double* A, int64_
 // Thin Q (m x n) and, where R is not null, R (n x n) of A (m x n, m >= n,
 // overwritten) with the signs of householder_qr, its panels factored by
 // products (qr_panel.hip).  False when a panel's columns are too dependent for
-// that (or not finite): A, Q and R then hold nothing of use.  Waits for the
-// stream.
+// that (or not finite), or one has nothing below its diagonal (its sign is not the
+// products' to pick): A, Q and R then hold nothing of use.  Waits for the stream.
 bool thin_qr_products(hipStream_t st, int64_t m, int64_t n, double* A, int64_t lda, double* Q, int64_t ldq, double* R,
                       int64_t ldr, DevBuf* work, GemmWorkspace* gws);
 

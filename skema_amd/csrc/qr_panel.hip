@@ -18,7 +18,9 @@
 // Q1 departs from orthonormal by eps cond(P)^2; the second pass brings it to eps
 // while that is well below 1.  A panel whose G1 has no Cholesky factor or whose
 // |G2 - I| exceeds 1e-4 (columns dependent to about 1e-6) sets `bad`, and the
-// caller factors the matrix anew column by column.
+// caller factors the matrix anew column by column.  So does a column with (next to)
+// nothing below its diagonal, |pivot| = 1 to rounding: dlarfg keeps its sign when
+// the rest is exactly zero (tau = 0), which the products cannot tell.
 //
 // Measured, one panel of 65536 rows: 5 launches, 85 us in all (34 and 930 us);
 // Q and R of the five factors of a 65536 x 16384 sketch with range 401 (X^T, Y,
@@ -307,10 +309,12 @@ __global__ __launch_bounds__(kOne) void k_panel_reflect(const double* part, int 
 #pragma unroll
     for (int c = 0; c < kNb; ++c) m[c] = inv ? 0.0 : A[li][c];
     double dj[kNb];
+    bool alone = false;  // a column with nothing below its diagonal
 #pragma unroll
     for (int c = 0; c < kNb; ++c) {
       const double piv = read_lane(m[c], c);
       const bool none = square && c == jb - 1;
+      alone = alone || (c < jb && !none && fabs(piv) > 1.0 - 1e-13);
       const double d = none ? copysign(1.0, piv) : -copysign(1.0, piv);
       const double p = none ? 0.0 : d * piv - 1.0;
       const double rp = none ? 0.0 : 1.0 / p;
@@ -326,6 +330,7 @@ __global__ __launch_bounds__(kOne) void k_panel_reflect(const double* part, int 
 #pragma unroll
       for (int t = c + 1; t < kNb; ++t) m[t] -= f * read_lane(m[t], c);
     }
+    if (alone && lane == 0) *bad = 1;
     if (lane < kNb) {
       double dl = 0.0;
 #pragma unroll

@@ -110,3 +110,37 @@ def test_low_rank_approx_of_a_few_columns(S, m, n, k):
     for name in ("Q", "P", "T1", "T2"):
         assert O.rel_err(g.checkpoint(name), osk.checkpoints[name]) <= TOL, name
     assert np.abs(Sv - Sr).max() <= TOL * Sr[0]
+
+
+@pytest.mark.parametrize("m,n", [(300, 200), (1500, 64)])
+@pytest.mark.parametrize("form", ["triangular", "block", "diagonal"])
+def test_thin_qr_of_columns_without_anything_below_the_diagonal(S, m, n, form):
+    """dlarfg leaves such a column and its sign alone (tau = 0): Q and P as
+    LAPACK's, from a state that holds one (block: the sixteenth column, once the
+    fifteen before it are reduced)."""
+    print(f"case thin qr {form} {m}x{n}", flush=True)
+    k = 40
+    rng = np.random.default_rng(m)
+
+    def tall(rows):
+        B = 0.1 * rng.standard_normal((rows, k))
+        sign = np.where(rng.random(k) < 0.5, -1.0, 1.0)
+        B[np.arange(k), np.arange(k)] += sign * (1.0 + rng.random(k))
+        if form == "triangular":
+            return np.triu(B)
+        if form == "diagonal":
+            return B * np.eye(rows, k)
+        B[16:, :16] = 0.0
+        return B
+
+    p = O.AlgParams(matrix_m=m, matrix_n=n, rank=4, sketch_range=k, sketch_core=2 * k + 1, window=m)
+    osk = O.SketchySVD(p)
+    osk.linear_update(np.zeros((m, n)))
+    osk.X, osk.Y, osk.Z = tall(n).T.copy(), tall(m), rng.standard_normal((2 * k + 1, 2 * k + 1))
+    osk.low_rank_approx()
+    g = S.SketchySVD(to_gpu_params(p), maps=gpu_maps({"Upsilon": osk.Upsilon, "Omega": osk.Omega, "Phi": osk.Phi,
+                                                      "Psi": osk.Psi}))
+    g.set_state(osk.X, osk.Y, osk.Z)
+    g.low_rank_approx()
+    for name in ("Q", "P", "T1", "T2"):
+        assert O.rel_err(g.checkpoint(name), osk.checkpoints[name]) <= TOL, name
