@@ -552,14 +552,16 @@ struct Plan {
 
 // Estimated cycles of the wide kernel: rounds of 256 blocks, a slice costing
 // the most of its MFMA, LDS and L2 time, plus writing and reading the K
-// splits' partials at about 4 TB/s and the launch that adds them.
+// splits' partials at about 4 TB/s and the launch that adds them.  The partials
+// stay within most_bytes.
 // far: the 64-bit form, built for TT = 2 only.
 // K of at most kShortK: the rounds' stores run beside the products of other
 // blocks and bound most of these, at 1785 B a cycle; blocks whose waves hold 128
 // rows of a column (WM = 1, TT = 1) write the longest runs.  14919 x 3410 x 6
 // takes 115 us with those, 121 with WM = 8, 158 with TT = 2 and 203 with both.
 constexpr int64_t kShortK = 128;
-void try_wide(Plan& best, int64_t M, int64_t N, int64_t K, bool may_split, bool far) {
+void try_wide(Plan& best, int64_t M, int64_t N, int64_t K, size_t most_bytes, bool far) {
+  const int64_t room = (int64_t)(most_bytes / sizeof(double)) / (M * N);  // splits whose partials fit
   for (int wm : {8, 1}) {
     const int64_t T = wm == 8 ? M : N, ns = cdiv(wm == 8 ? N : M, 16);
     for (int tt : {2, 1}) {
@@ -577,7 +579,7 @@ void try_wide(Plan& best, int64_t M, int64_t N, int64_t K, bool may_split, bool 
         if (cost < best.cost) best = Plan{true, far, wm, tt, ts, 1, tiles_t, tiles_s, cost};
         continue;
       }
-      const int64_t most = may_split ? std::max<int64_t>(1, std::min<int64_t>(128, K / 64)) : 1;
+      const int64_t most = std::max<int64_t>(1, std::min<int64_t>({128, K / 64, room}));
       for (int64_t sp = 1; sp <= most; ++sp) {
         const int64_t per = cdiv(cdiv(K, sp), kBK) * kBK;
         const int64_t real = per ? cdiv(K, per) : 1;
@@ -601,7 +603,7 @@ void try_wide(Plan& best, int64_t M, int64_t N, int64_t K, bool may_split, bool 
 // From 8192 of K on, both operands contiguous along K (TN) ask for them in
 // half lines, at 2700 B a cycle once 32 tiles do so: 403 x 403 x 20000 is 278 us
 // of that, and 164 on the wide kernel.
-void try_ksplit(Plan& best, bool tn_form, int64_t M, int64_t N, int64_t K, bool may_split) {
+void try_ksplit(Plan& best, bool tn_form, int64_t M, int64_t N, int64_t K, size_t most_bytes) {
   const int64_t tm = cdiv(M, 32), tn = cdiv(N, 32);
   if (tm * tn >= (int64_t)1 << 31) return;
   if (K <= kShortK) {
@@ -612,7 +614,8 @@ void try_ksplit(Plan& best, bool tn_form, int64_t M, int64_t N, int64_t K, bool 
     if (two < best.cost) best = Plan{false, false, 2, 1, 1, 1, tm, tn, two};
     return;
   }
-  const int64_t most = may_split ? std::max<int64_t>(1, std::min<int64_t>(64, K / 512)) : 1;
+  const int64_t room = (int64_t)(most_bytes / sizeof(double)) / (M * N);
+  const int64_t most = std::max<int64_t>(1, std::min<int64_t>({64, K / 512, room}));
   for (int64_t sp = 1; sp <= most; ++sp) {
     const int64_t per = cdiv(cdiv(K, sp), kBK) * kBK;
     if ((per ? cdiv(K, per) : 1) != sp) continue;
@@ -633,10 +636,15 @@ void try_ksplit(Plan& best, bool tn_form, int64_t M, int64_t N, int64_t K, bool 
 // (5.38 on the small kernel).
 bool near_enough(bool k_contiguous, int64_t ld) { return ld <= (int64_t)1 << (k_contiguous ? 21 : 25); }
 
-Plan choose(bool ta, bool tb, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, bool may_split) {
+// What the K splits' partials of one product may take, for the context's life:
+// 8 splits of 4096 x 1204 are 316 MB; more (4 of 66000 x 604, 1.28 GB) would even
+// out the last round of a product that has many.
+constexpr size_t kMostPartials = (size_t)512 << 20;
+
+Plan choose(bool ta, bool tb, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, size_t most_bytes) {
   Plan p;
-  try_ksplit(p, ta && !tb, M, N, K, may_split);
-  try_wide(p, M, N, K, may_split, !near_enough(ta, lda) || !near_enough(!tb, ldb));
+  try_ksplit(p, ta && !tb, M, N, K, most_bytes);
+  try_wide(p, M, N, K, most_bytes, !near_enough(ta, lda) || !near_enough(!tb, ldb));
   return p;
 }
 
@@ -644,7 +652,7 @@ Plan choose(bool ta, bool tb, int64_t M, int64_t N, int64_t K, int64_t lda, int6
 
 bool gemm_f64_one_pass(char transB, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb) {
   if (M <= 0 || N <= 0 || K <= 0) return false;
-  const Plan p = choose(false, transB == 'T' || transB == 't', M, N, K, lda, ldb, true);
+  const Plan p = choose(false, transB == 'T' || transB == 't', M, N, K, lda, ldb, kMostPartials);
   return p.cost < 1e300 && !p.wide && p.splits == 1;
 }
 
@@ -655,7 +663,7 @@ void gemm_f64_series(hipStream_t stream, char transB, int64_t M, int64_t N, int6
                 "gemm_f64_series: not products of one pass");
   SKEMA_REQUIRE(lda >= M && ldb >= (tb ? N : K), kErrShape, "gemm_f64_series: leading dimension too small");
   Plan p;
-  try_ksplit(p, false, M, N, K, true);
+  try_ksplit(p, false, M, N, K, kMostPartials);
   KArgs a;
   a.M = M; a.N = N; a.K = K; a.A = A; a.lda = lda; a.B = B; a.ldb = ldb; a.out = out;
   a.tiles_t = (int)p.tiles_t; a.tiles_s = (int)p.tiles_s;
@@ -684,7 +692,22 @@ void gemm_f64(hipStream_t stream, char transA, char transB, int64_t M, int64_t N
   SKEMA_REQUIRE(out.nsplit == N || out.ldc2 >= M, kErrShape, "gemm_f64: ldc too small");
   SKEMA_REQUIRE(M * N < (int64_t)1 << 40, kErrShape, "gemm_f64: output too large");
 
-  const Plan p = choose(ta, tb, M, N, K, lda, ldb, ws != nullptr);
+  // Fewer splits where the device has no room for the partials.
+  size_t most = ws ? kMostPartials : 0;
+  Plan p;
+  for (;;) {
+    p = choose(ta, tb, M, N, K, lda, ldb, most);
+    if (p.splits == 1) break;
+    const size_t need = (size_t)p.splits * M * N * sizeof(double);
+    try {
+      ws->buf.reserve(need);
+      break;
+    } catch (const Error& e) {
+      if (e.code != kErrOom) throw;
+      (void)hipGetLastError();
+      most = need / 2;
+    }
+  }
   SKEMA_REQUIRE(p.cost < 1e300, kErrShape, "gemm_f64: too many tiles");
 
   KArgs a;
@@ -692,10 +715,7 @@ void gemm_f64(hipStream_t stream, char transA, char transB, int64_t M, int64_t N
   a.tiles_t = (int)p.tiles_t; a.tiles_s = (int)p.tiles_s;
   a.partial = nullptr;
   a.k_per_split = K > 0 ? cdiv(cdiv(K, (int64_t)p.splits), kBK) * kBK : 0;
-  if (p.splits > 1) {
-    ws->buf.reserve((size_t)p.splits * M * N * sizeof(double));
-    a.partial = ws->buf.as<double>();
-  }
+  if (p.splits > 1) a.partial = ws->buf.as<double>();
   dim3 grid((unsigned)(p.tiles_t * p.tiles_s), 1, (unsigned)p.splits);
   if (p.wide) {
     if (p.far && p.wm == 8) launch_wide_s<8, 2, true>(stream, ta, tb, a, grid, p.ts);

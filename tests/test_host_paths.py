@@ -188,3 +188,29 @@ L.call("skema_low_rank_approx_device", sk, U, m, S, V, 200)
 used = [n for n in names() if "k_panel_mul" in n]
 assert bool(used) == {products}, used
 """)
+
+
+def test_split_products_stay_within_their_scratch(runtime):
+    """Partials of at most 512 MiB, fewer splits where that is not to be had, and
+    none at all."""
+    run(runtime, r"""
+def product(M, N, K, room):
+    ctx = context()
+    mp, B, out = dense_map(ctx, M, K), device(K * N), device(M * N)
+    rt.rt_forget()
+    before = rt.rt_used()
+    rt.rt_set_limit(before + room)
+    L.call("skema_map_lmap", mp, 1.0, B, K, N, K, 0.0, b"N", b"N", 0, 0, out, M)
+    rt.rt_set_limit(1 << 60)
+    splits = [g[2] for n, g in launched() if "k_gemm_" in n]
+    assert len(splits) == 1
+    return splits[0], rt.rt_used() - before
+
+splits, kept = product(4096, 1204, 16384, 1 << 60)
+assert splits == 8 and kept <= 512 * MiB, (splits, kept)
+splits, kept = product(4096, 1204, 16384, 200 * MiB)
+assert 1 < splits < 8 and kept <= 200 * MiB, (splits, kept)
+assert product(4096, 1204, 16384, 1 * MiB) == (1, 0)
+splits, kept = product(66000, 604, 8192, 1 << 60)
+assert kept <= 512 * MiB, (splits, kept)
+""")
