@@ -637,8 +637,9 @@ int skema_linear_update_dense(skema_sketch* h, const double* A, int64_t lda) {
     } else {
       zero_state(sk);
       int64_t next = 0;  // first row of the windows not taken in groups
-      for (const int64_t w = sk.p.window; w < sk.p.m;) {
-        const int64_t took = update_dense_windows(sk, A + next, lda, next, w, (sk.p.m - next) / w);
+      const int64_t w = sk.p.window;
+      for (int64_t took = sk.p.m / w; w < sk.p.m;) {  // no group larger than the one before it
+        took = update_dense_windows(sk, A + next, lda, next, w, std::min(took, (sk.p.m - next) / w));
         if (took == 0) break;
         next += took * w;
       }

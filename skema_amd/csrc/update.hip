@@ -200,11 +200,19 @@ int64_t update_dense_windows(Sketch& sk, const double* H, int64_t ldh, int64_t r
       !gemm_f64_one_pass('N', s, s, w, sk.ldphi, w))
     return 0;
   count = std::min<int64_t>({count, ((int64_t)128 << 20) / (w * (n + s) * 8), (int64_t)65535});
+  for (; count >= 2; count /= 2) {  // smaller groups, or none, where the device has no room for G
+    try {
+      sk.G.reserve((size_t)count * w * s * sizeof(double));
+      break;
+    } catch (const Error& e) {
+      if (e.code != kErrOom) throw;
+      (void)hipGetLastError();
+    }
+  }
   if (count < 2) return 0;
   Ctx* c = sk.ctx;
   hipStream_t st = c->stream;
   const double eta = sk.p.eta, nu = sk.p.nu;
-  sk.G.reserve((size_t)count * w * s * sizeof(double));
   double* G = sk.G.as<double>();
   GemmSeries sr;
   sr.count = count;

@@ -214,3 +214,20 @@ assert product(4096, 1204, 16384, 1 * MiB) == (1, 0)
 splits, kept = product(66000, 604, 8192, 1 << 60)
 assert kept <= 512 * MiB, (splits, kept)
 """)
+
+
+@pytest.mark.parametrize("room_windows,groups", [(1 << 20, [60]), (20, [15, 15, 15, 15]), (1, [])])
+def test_grouped_windows_fit_the_memory_there_is(runtime, room_windows, groups):
+    """60 windows whose G takes 30 KB each: one group, smaller ones, or the
+    windows one by one."""
+    run(runtime, rf"""
+ctx = context()
+m, n, w, k, s = 6000, 300, 100, 21, 43
+sk, A = sketch(ctx, m, n, k, s, window=w), device(m * n)
+rt.rt_forget()
+rt.rt_set_limit(rt.rt_used() + {room_windows} * w * s * 8)
+L.call("skema_linear_update_dense", sk, A, m)
+got = launched()
+series = [g[1] for name, g in got if "k_gemm_ksplit" in name and "Lb1EEEv" in name and g[1] > 1]
+assert series == {groups!r}, got
+""")
