@@ -543,6 +543,7 @@ int skema_sketch_create(skema_ctx* ctx, const skema_params* p, skema_map* upsilo
     sk.Y.alloc((size_t)p->m * sk.k * sizeof(double));
     sk.Z.alloc((size_t)sk.s * sk.s * sizeof(double));
     zero_state(sk);
+    if (sk.sparse_maps) prepare_csr_maps(sk);  // last: it does without where memory is short
     auto& ti = sk.timings["init"];
     const char* names[4] = {"upsilon", "omega", "phi", "psi"};
     for (int i = 0; i < 4; ++i) ti[names[i]] = sk.maps[i]->init_seconds;

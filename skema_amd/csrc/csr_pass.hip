@@ -880,13 +880,19 @@ __global__ void k_pair_ell(const uint16_t* a, int za, const uint16_t* b, int zb,
 // (32 bytes a column each in 32-bit entries) that an L2 does not hold: one
 // 32-byte record of both in place of two requests, half the table.  4e6
 // nonzeros, 200000 rows, zeta = 8: 114 -> 59 us, 56 with the registers held to
-// five waves a SIMD.
+// five waves a SIMD.  Without room for it the pass reads the maps' own tables.
 void prepare_csr_maps(Sketch& sk) {
   const Map &u = *sk.maps[0], &f = *sk.maps[2];
   if (!u.ell16.p || !f.ell16.p || u.ell_zeta > 8 || f.ell_zeta > 8) return;
   const int64_t m = sk.p.m;
   hipStream_t st = sk.ctx->stream;
-  sk.ell_pair.alloc((size_t)m * 32);
+  try {
+    sk.ell_pair.alloc((size_t)m * 32);
+  } catch (const Error& e) {
+    if (e.code != kErrOom) throw;
+    (void)hipGetLastError();
+    return;
+  }
   hipLaunchKernelGGL(k_pair_ell, dim3((unsigned)std::min<int64_t>(cdiv(16 * m, 256), 8192)), dim3(256), 0, st,
                      u.ell16.as<uint16_t>(), u.ell_zeta, f.ell16.as<uint16_t>(), f.ell_zeta, m,
                      sk.ell_pair.as<uint16_t>());

@@ -13,7 +13,6 @@
 #include <algorithm>
 #include <cmath>
 
-#include "csr_pass.hpp"
 #include "linalg.hpp"
 #include "lowp.hpp"
 #include "rbf.hpp"
@@ -102,7 +101,6 @@ void prepare_sketch_maps(Sketch& sk) {
       rp[j + 1] = (int64_t)ci.size();
     }
     upload_csr(sk.sp_ompsT, n, k + s, (int64_t)ci.size(), rp.data(), ci.data(), v.data(), st);
-    prepare_csr_maps(sk);
     return;
   }
   auto logical = [&](Map* m, DevBuf& own, const double*& ptr, int64_t& ld) {

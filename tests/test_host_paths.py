@@ -231,3 +231,33 @@ got = launched()
 series = [g[1] for name, g in got if "k_gemm_ksplit" in name and "Lb1EEEv" in name and g[1] > 1]
 assert series == {groups!r}, got
 """)
+
+
+def test_sketch_without_room_for_its_joint_map_records(runtime):
+    """The records (32 bytes a row) are an extra: a sketch that fits without them
+    is made, and takes the pass that reads the maps' own tables."""
+    run(runtime, r"""
+ctx = context()
+m, n, k, s, nnz = 20000, 400, 9, 19, 5000
+rowptr, col, val = device(m + 1), device(nnz, 4), device(nnz)
+rt.rt_inspection(0, nnz, 0)
+
+def left_product(sk):
+    rt.rt_forget()
+    L.call("skema_linear_update_csr", sk, rowptr, col, val)
+    return [n for n in names() if "k_left_" in n]
+
+p = L.skema_params()
+L.load().skema_params_default(C.byref(p))
+p.m, p.n, p.rank, p.range, p.core, p.window, p.dim_redux, p.issparse = m, n, 2, k, s, m, L.MAP_SPARSE_SIGN, 1
+maps = [sign_map(ctx, *shape) for shape in ((k, m), (k, n), (s, m), (s, n))]
+roomy, tight = C.c_void_p(), C.c_void_p()
+before = rt.rt_used()
+L.call("skema_sketch_create", ctx, C.byref(p), *maps, C.byref(roomy))
+takes = rt.rt_used() - before
+rt.rt_set_limit(rt.rt_used() + takes - 32 * m)
+L.call("skema_sketch_create", ctx, C.byref(p), *maps, C.byref(tight))
+rt.rt_set_limit(1 << 60)
+assert len(left_product(roomy)) == 1 and "k_left_tile" in left_product(roomy)[0]
+assert len(left_product(tight)) == 1 and "k_left_fx" in left_product(tight)[0]
+""")
