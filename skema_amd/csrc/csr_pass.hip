@@ -847,22 +847,6 @@ bool csc_by_buckets(hipStream_t st, const int64_t* rowptr, const int32_t* col, c
   return true;
 }
 
-// Columns a tile for k_left_tile, 0 when it does not apply: the tile's
-// accumulators fit its LDS, at most kMaxTiles tiles, and of those the fewest
-// rounds x columns over the 256 CUs (one block each).  Whole passes, CSC ->
-// tiles: 500 x 300 with 3000 nonzeros 98 -> 93 us, 100000 x 200 with 2e5
-// 131 -> 96, 20000 x 50000 with 1e5 166 -> 140, 200000 x 20000 with 4e6
-// 309 -> 278: the faster one wherever it fits.
-int64_t left_tile_cols(int64_t n, int64_t na) {
-  const int64_t lo = cdiv(n, kMaxTiles), hi = std::min<int64_t>(kTileSlots / na, kTileCols);
-  int64_t best = 0, best_cost = INT64_MAX;
-  for (int64_t tc = lo; tc <= hi; ++tc) {
-    const int64_t cost = cdiv(cdiv(n, tc), 256) * tc;
-    if (cost <= best_cost) { best_cost = cost; best = tc; }
-  }
-  return best;
-}
-
 // Joint records of two maps' packed ELL columns: entry f of column c of the
 // first at pair[16 c + f], of the second at pair[16 c + 8 + f]; 0 past z.
 __global__ void k_pair_ell(const uint16_t* a, int za, const uint16_t* b, int zb, int64_t cols, uint16_t* pair) {
@@ -875,6 +859,25 @@ __global__ void k_pair_ell(const uint16_t* a, int za, const uint16_t* b, int zb,
 }
 
 }  // namespace
+
+// Columns a tile for k_left_tile, 0 when it does not apply: the tile's
+// accumulators fit its LDS, at most kMaxTiles tiles and 2^31 counts (one for a tile
+// and kL1Rows rows), and of those the fewest rounds x columns over the 256 CUs (one
+// block each).  Whole passes with evenly spread columns, CSC -> tiles: 500 x 300
+// with 3000 nonzeros 98 -> 93 us, 100000 x 200 with 2e5 131 -> 96, 20000 x 50000 with
+// 1e5 166 -> 140, 200000 x 20000 with 4e6 309 -> 278.  With heavy columns side by side
+// the level-1 scatter bounds both: 200000 x 20000 with 4e6, half of them in the first 40
+// columns 4.26 -> 4.19 ms, in the first 400 1.17 -> 1.09, sorted Zipf 6.33 -> 6.23.
+int64_t left_tile_cols(int64_t m, int64_t n, int64_t na) {
+  const int64_t lo = cdiv(n, kMaxTiles), hi = std::min<int64_t>(kTileSlots / na, kTileCols);
+  int64_t best = 0, best_cost = INT64_MAX;
+  for (int64_t tc = lo; tc <= hi; ++tc) {
+    if (cdiv(n, tc) * cdiv(m, (int64_t)kL1Rows) >= (int64_t)1 << 31) continue;
+    const int64_t cost = cdiv(cdiv(n, tc), 256) * tc;
+    if (cost <= best_cost) { best_cost = cost; best = tc; }
+  }
+  return best;
+}
 
 // The left product gathers both maps' columns for every nonzero, from tables
 // (32 bytes a column each in 32-bit entries) that an L2 does not hold: one
@@ -930,7 +933,7 @@ void update_csr_all(Sketch& sk, const int64_t* rowptr, const int32_t* col, const
     Wm = reinterpret_cast<double*>(scr.as<char>() + align_up((size_t)W * sizeof(double), 256));
     SKEMA_HIP(hipMemcpyAsync(cw, hw.data(), (size_t)W * sizeof(double), hipMemcpyHostToDevice, st));
     // the fixed-point products take the column entries in any order
-    const int64_t tc = sk.ell_pair.p && buckets_fit(nnz) ? left_tile_cols(n, k + s) : 0;
+    const int64_t tc = sk.ell_pair.p && buckets_fit(nnz) ? left_tile_cols(m, n, k + s) : 0;
     if (tc > 0)
       tiles = bucket_columns(st, rowptr, col, val, m, n, nnz, tc, 0, sk.win);
     else if (!sk.sparse_maps || !csc_by_buckets(st, rowptr, col, val, m, n, nnz, sk.win, H))

@@ -5,6 +5,10 @@
 
 namespace skema {
 
+// Columns a tile of the left product over m x n entries with na map rows in all;
+// 0: the column by column form.
+int64_t left_tile_cols(int64_t m, int64_t n, int64_t na);
+
 // What the pass keeps of a sketch's sparse maps (Sketch::ell_pair).
 void prepare_csr_maps(Sketch& sk);
 

@@ -261,3 +261,19 @@ rt.rt_set_limit(1 << 60)
 assert len(left_product(roomy)) == 1 and "k_left_tile" in left_product(roomy)[0]
 assert len(left_product(tight)) == 1 and "k_left_fx" in left_product(tight)[0]
 """)
+
+
+@pytest.mark.parametrize("m,n,na,taken", [(200000, 20000, 304, True), (1_050_000_000, 512, 15, True),
+                                          (1_200_000_000, 512, 15, True), (2_000_000_000, 512, 15, True),
+                                          (1_200_000_000, 20000, 304, False), (1000, 100000, 304, False)])
+def test_column_tiles_leave_countable_blocks(runtime, m, n, na, taken):
+    """A count per tile and 256 rows, 2^31 of them at most: above a billion rows
+    fewer and wider tiles, or the other form, which such a matrix always fitted."""
+    run(runtime, rf"""
+f = L.load()._ZN5skema14left_tile_colsElll
+f.restype, f.argtypes = C.c_int64, [C.c_int64] * 3
+tc = f({m}, {n}, {na})
+assert (tc > 0) == {taken}, tc
+if tc > 0:
+    assert -(-{n} // tc) * -(-{m} // 256) < 1 << 31, tc
+""")
