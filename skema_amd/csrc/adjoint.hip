@@ -423,16 +423,16 @@ void rbf_sketch_loss_grad(Ctx* c, const double* X, int64_t n, int64_t d, int64_t
   }
   hipStream_t st = c->stream;
   const int64_t h = k + s;
-  DevBuf nrm(n * sizeof(double)), OP((size_t)h * n * sizeof(double)), F((size_t)n * 3 * h * sizeof(double)),
-      PhiL((size_t)s * n * sizeof(double)), W((size_t)s * s * sizeof(double)), sc(2 * sizeof(double)), red;
+  DevBuf nrm(n * sizeof(double)), F((size_t)n * 3 * h * sizeof(double)), PhiL((size_t)s * n * sizeof(double)), W((size_t)s * s * sizeof(double)), sc(2 * sizeof(double)), red;
   Timed tf(c, "rbf_forward");
   row_norms2(st, X, n, d, ldp, nrm.as<double>());
-  logical_copy(st, omega, OP.as<double>(), h);
-  logical_copy(st, psi, OP.as<double>() + k, h);
+  double* Fp = F.as<double>();
+  double* OP = Fp + 2 * h * n;  // [Omega; Psi] (h x n), where F[:, 2h:3h] comes later
+  logical_copy(st, omega, OP, h);
+  logical_copy(st, psi, OP + k, h);
   logical_copy(st, phi, PhiL.as<double>(), s);
   RbfRows all;
   all.X = X; all.n = n; all.ldp = ldp; all.d = d; all.nrm = nrm.as<double>(); all.gamma = gamma; all.rows = n;
-  double* Fp = F.as<double>();
   double* Y = Fp;           // F[:, 0:k]   = Y = K Omega^T
   double* G = Fp + k * n;   // F[:, k:h]   = G = K Psi^T, then Phi^T W
   // forward: [Y | G] window by window
@@ -443,7 +443,7 @@ void rbf_sketch_loss_grad(Ctx* c, const double* X, int64_t n, int64_t d, int64_t
     GemmOut o;
     o.C1 = Y + r0; o.ldc1 = n; o.alpha1 = 1.0; o.beta1 = 0.0; o.nsplit = k;
     o.C2 = G + r0; o.ldc2 = n; o.alpha2 = 1.0; o.beta2 = 0.0;
-    rbf_products_f64(c, w, nullptr, 0, 0, GemmOut{}, OP.as<double>(), h, h, o, false);
+    rbf_products_f64(c, w, nullptr, 0, 0, GemmOut{}, OP, h, h, o, false);
   }
   // W = Phi G (s x s); loss = ||Y||^2 + ||W||^2
   gemm_f64(st, 'N', 'N', s, s, n, 1.0, PhiL.as<double>(), s, G, n, 0.0, W.as<double>(), s, &c->gws);
@@ -452,10 +452,10 @@ void rbf_sketch_loss_grad(Ctx* c, const double* X, int64_t n, int64_t d, int64_t
   tf.stop();
   double hs[2];
   SKEMA_HIP(hipMemcpyAsync(hs, sc.p, 2 * sizeof(double), hipMemcpyDeviceToHost, st));
-  // B = [Y | Phi^T W] in place of G; F[:, h:2h] = OP^T; F[:, 2h:3h] = B again,
+  // B = [Y | Phi^T W] in place of G; F[:, h:2h] = OP^T; F[:, 2h:3h] = B over OP,
   // so R = [OP^T | B] is F from column h on
   gemm_f64(st, 'T', 'N', n, s, s, 1.0, PhiL.as<double>(), s, W.as<double>(), s, 0.0, G, n, &c->gws);
-  transpose(st, h, n, OP.as<double>(), h, Fp + h * n, n);
+  transpose(st, h, n, OP, h, Fp + h * n, n);
   copy_matrix(st, n, h, Fp, n, Fp + 2 * h * n, n);
   SKEMA_HIP(hipStreamSynchronize(st));
   *loss = hs[0] + hs[1];
@@ -464,6 +464,7 @@ void rbf_sketch_loss_grad(Ctx* c, const double* X, int64_t n, int64_t d, int64_t
     return;
   }
   // panels of up to 2048 rows
+  PhiL.release();  // its place for X1 and T
   const int64_t d1 = d + 1;
   DevBuf X1((size_t)n * d1 * sizeof(double)), T((size_t)n * d1 * sizeof(double));
   hipLaunchKernelGGL(k_points_one, dim3((unsigned)std::min<int64_t>(cdiv(n, 256), 1024), (unsigned)d1), dim3(256), 0, st,

@@ -277,3 +277,18 @@ assert (tc > 0) == {taken}, tc
 if tc > 0:
     assert -(-{n} // tc) * -(-{m} // 256) < 1 << 31, tc
 """)
+
+
+def test_loss_and_gradient_hold_the_maps_once(runtime):
+    """[B | OP^T | B] and the maps' copies in three times h n doubles, not four,
+    beside Phi, the points and the least K rows."""
+    run(runtime, r"""
+ctx = context()
+n, d, k, s = 20000, 16, 101, 203
+h = k + s
+maps = [dense_map(ctx, rows, n) for rows in (k, s, s)]
+X, dX = device(n * d), device(n * d)
+loss, dg = C.c_double(), C.c_double()
+rt.rt_set_limit(rt.rt_used() + (3 * h * n + s * n + s * s + 2 * n) * 8 + 40 * MiB)
+L.call("skema_rbf_sketch_loss_grad", ctx, X, n, d, n, 0.1, *maps, 4096, L.PREC_FP64, C.byref(loss), dX, n, C.byref(dg))
+""")
