@@ -6,12 +6,14 @@
 // through the matrix cores five times:
 //   G1 = P^T P,  G1 = R1^T R1             (Cholesky)
 //   Q1 = P R1^{-1},  G2 = Q1^T Q1 = R2^T R2
-//   Q  = Q1 R2^{-1}, R' = R2 R1           (Cholesky QR twice: Q orthonormal to eps)
+//   Q  = Q1 R2^{-1}, R' = R2 R1           (Cholesky QR twice: Q orthonormal to eps;
+//                                          Yamamoto, Nakatsukasa, Yanagisawa, Fukaya 2015)
 // and the reflectors follow from Q: with D the signs LAPACK's dlarfg would pick
 // (R = D R', R_jj = -sign(a_jj) |.|), Q D - [I; 0] = V U with V unit lower
 // trapezoidal and U upper triangular, an LU factorisation without pivoting whose
-// pivots lie in [-2, -1] because D_j is picked against the sign of the pivot, and
-// H(0) ... H(31) = I - V T V^T with T = -U V_1^{-T} (V_1: V's top 32 rows).  So
+// pivots lie in [-2, -1] because D_j is picked against the sign of the pivot
+// (Householder vectors from an orthonormal panel: Ballard, Demmel, Grigori,
+// Jacquelin, Knight, Nguyen, Solomonik 2015), and H(0) ... H(31) = I - V T V^T with T = -U V_1^{-T} (V_1: V's top 32 rows).  So
 // V, T, R are Householder's, to rounding, and the trailing columns and Q are
 // formed with blocked products as before.
 //

@@ -495,7 +495,7 @@ __global__ __launch_bounds__(64 * (kTallRows / (16 * kTallXT)), 1) void k_rbf_ri
       if (y + 2 < TNC) o2 = op_at(y + 2);
 #pragma unroll
       for (int x = 0; x < XT; ++x) acc[x][y] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kv[x], o, acc[x][y], 0, 0, 0);
-      // K values e in [32 y / TNC, 32 (y + 1) / TNC) of this lane's 32 (x, h, v)
+      // K values e in [8 XT y / TNC, 8 XT (y + 1) / TNC) of this lane's 8 XT (x, h, v)
 #pragma unroll
       for (int e = (8 * XT * y) / TNC; e < (8 * XT * (y + 1)) / TNC; ++e) {
         const int x = e / 8, h = (e / 4) % 2, v = e % 4;

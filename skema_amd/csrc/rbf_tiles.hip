@@ -4,8 +4,9 @@
 //   left : X       <- nu X + eta * Upsilon[:, idx] K_w     (k x n)
 //   right: [y | G]  =  K_w [Omega; Psi]^T                   (w x (k+s))
 // K costs 2 d + about 40 (exp) operations an element to form and 16 bytes of
-// traffic a use, the products 2 (2k + s): at k = 201, s = 403 writing K once and
-// reading it twice is 1/15 of the products' time.  Generating K inside each
+// traffic a use, the products 2 (2k + s): at k = 201, s = 403 the bytes of writing
+// K once and reading it twice take 1/15 of the products' time at the copy rate,
+// forming K and all 12%.  Generating K inside each
 // product's own tile loop instead (no K in memory) kept the product at 21 to 43
 // TF, because the Gram, the exponentials and their barriers stood between its
 // MFMAs, and formed K twice; here both products run at the GEMM's 58 to 64 TF.
